@@ -5,7 +5,9 @@
 #include <stdint.h>
 
 #include <string>
+#include <vector>
 
+#include "pt_internal.h"
 #include "pt_types.h"
 
 namespace pt {
@@ -46,6 +48,29 @@ struct DevBuf {
     template <class T> T *as() const { return (T *)p; }
 };
 
+// One device allocation cut into several arrays (a hipMalloc and a hipFree cost as much as a
+// kernel each).  want() notes the pointers, alloc() sets them.
+struct WorkArrays {
+    struct Want {
+        void **p;
+        size_t bytes;
+    };
+    std::vector<Want> wants;
+    DevBuf buf;
+    template <class T> void want(T *&p, size_t n) { wants.push_back({(void **)&p, (n * sizeof(T) + 255) / 256 * 256}); }
+    void alloc() {
+        size_t total = 256;
+        for (const Want &w : wants) total += w.bytes;
+        buf.alloc(total);
+        size_t at = 0;
+        for (const Want &w : wants) {
+            *w.p = buf.as<char>() + at;
+            at += w.bytes;
+        }
+        wants.clear();
+    }
+};
+
 struct BvhInfo {
     int numNodes = 0;      // 4-wide nodes
     int depth = 0;         // levels of 4-wide nodes
@@ -72,5 +97,29 @@ void buildEnvTables(const float4 *rgba, int w, int h, int sinWeight, float2 *row
 void packEnvPdf(float4 *rgba, const float *texelPdf, int n, hipStream_t stream);
 
 int deviceCUs();
+
+// Exclusive prefix sums of m counters in place, the total to data[m] (m + 1 entries); tmp holds
+// scanEntries(m).
+size_t scanEntries(int m);
+void scanCounts(uint32_t *data, int m, uint32_t *tmp, hipStream_t stream);
+
+// The scene's arrays on the device as the host describes them, in input order, and the device
+// records made from them.  Kept for edits: a material changes in place, and an emission edit
+// makes the emitter list again.
+struct SceneArrays {
+    int nTri = 0, nSph = 0, nMat = 0;
+    WorkArrays arrays;
+    float *pos = nullptr, *sph = nullptr;   // 9 per triangle, 4 per sphere
+    int *triMat = nullptr, *sphMat = nullptr;
+    HostMaterial *mats = nullptr;
+    // Uploads s and writes its primitive records (triangles, then spheres), the per-vertex
+    // normals that differ from the flat ones, and the bounds (+-infinity without primitives).
+    void load(const pt_scene &s, DevBuf &records, DevBuf &normals, float lo[3], float hi[3], hipStream_t stream);
+    HostMaterial material(int id, hipStream_t stream) const;
+    void setMaterial(int id, const HostMaterial &m, DevBuf &records, hipStream_t stream);
+    void buildMaterials(DevBuf &records, hipStream_t stream) const;
+    // Emitter records (3 float4 each) in the reference's light order; returns their number.
+    int buildEmitters(DevBuf &records, hipStream_t stream) const;
+};
 
 }  // namespace pt

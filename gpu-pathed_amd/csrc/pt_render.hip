@@ -1694,10 +1694,7 @@ struct pt_renderer {
     bool packetCamera = true;  // camera runs of one pixel's samples traced as one packet
     bool traceStats = false;   // PT_OPT_TRACE_STATS: instrumented trace kernels
     bool hasScene = false;
-    // host copies needed for edits
-    std::vector<HostMaterial> mats;
-    std::vector<int> triMat, sphMat;
-    std::vector<float> triPos, sph;
+    SceneArrays scene;   // the scene as described, kept for edits
     HostCamera camHost;
     PtCamera cam{};
     int maxDepth = 3;  // scene.h:18 defaultMaxDepth
@@ -1792,44 +1789,10 @@ void computeCamera(pt_renderer *r) {
     c.H = r->H;
 }
 
-void uploadMaterials(pt_renderer *r) {
-    std::vector<PtMaterial> m(r->mats.size());
-    for (size_t i = 0; i < m.size(); i++) {
-        const HostMaterial &h = r->mats[i];
-        const bool lamb = h.type == PT_LAMBERTIAN;
-        m[i].a = make_float4(h.albedo[0], h.albedo[1], h.albedo[2], (float)h.type);
-        const float param = h.type == PT_GLASS ? h.ior : (h.type == PT_MICROFACET ? h.alpha : 0.f);
-        m[i].b = make_float4(lamb ? h.emit[0] : 0.f, lamb ? h.emit[1] : 0.f, lamb ? h.emit[2] : 0.f, param);
-    }
-    r->materials.alloc(std::max<size_t>(1, m.size()) * sizeof(PtMaterial));
-    if (!m.empty()) PT_HIP_TRY(hipMemcpyAsync(r->materials.p, m.data(), m.size() * sizeof(PtMaterial), hipMemcpyHostToDevice, r->stream));
-    r->view.materials = r->materials.as<PtMaterial>();
-    r->view.numMaterials = (int)m.size();
-}
-
-// Emitter records in the reference light order (scene_data.cu:92-115); rebuilt after edits
-// so that emission changes also change the light list.
-void uploadEmitters(pt_renderer *r) {
-    std::vector<float4> e;
-    const int64_t nt = (int64_t)r->triMat.size();
-    for (int64_t i = 0; i < nt; i++) {
-        if (!isEmissive(r->mats[r->triMat[i]])) continue;
-        const float *p = &r->triPos[i * 9];
-        e.push_back(make_float4(p[0], p[1], p[2], asFloat(r->triMat[i])));
-        e.push_back(make_float4(p[3], p[4], p[5], asFloat(PT_TAG_FLAT)));
-        e.push_back(make_float4(p[6], p[7], p[8], asFloat((int)i)));
-    }
-    for (size_t i = 0; i < r->sphMat.size(); i++) {
-        if (!isEmissive(r->mats[r->sphMat[i]])) continue;
-        const float *s = &r->sph[i * 4];
-        e.push_back(make_float4(s[0], s[1], s[2], asFloat(r->sphMat[i])));
-        e.push_back(make_float4(s[3], 0.f, 0.f, asFloat(PT_TAG_SPHERE)));
-        e.push_back(make_float4(0.f, 0.f, 0.f, asFloat(~(int)i)));
-    }
-    r->emitters.alloc(std::max<size_t>(1, e.size()) * sizeof(float4));
-    if (!e.empty()) PT_HIP_TRY(hipMemcpyAsync(r->emitters.p, e.data(), e.size() * sizeof(float4), hipMemcpyHostToDevice, r->stream));
+// The emitter list, rebuilt after edits so that emission changes also change it.
+void buildEmitters(pt_renderer *r) {
+    r->view.numEmitters = r->scene.buildEmitters(r->emitters, r->stream);
     r->view.emitters = r->emitters.as<float4>();
-    r->view.numEmitters = (int)(e.size() / 3);
 }
 
 // Path pool sized to the work at hand: `need` paths rounded up to a power of two, at least
@@ -2252,58 +2215,13 @@ int pt_renderer_set_scene(pt_renderer *r, const pt_scene *s) {
     if (s->mats.empty()) return fail(PT_ERR_INVALID, "pt_renderer_set_scene: scene has no materials");
     PT_API_BEGIN
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
-    r->mats = s->mats;
-    r->triMat = s->triMat;
-    r->sphMat = s->sphMat;
-    r->triPos = s->pos;
-    r->sph = s->sph;
     r->camHost = s->cam;
     computeCamera(r);
     // primitive records in input order (triangles, then spheres)
     const int64_t n = nt + ns;
-    std::vector<float4> recs((size_t)std::max<int64_t>(n, 1) * 3);
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    auto grow = [&](float x, float y, float z) {
-        lo[0] = std::min(lo[0], x); lo[1] = std::min(lo[1], y); lo[2] = std::min(lo[2], z);
-        hi[0] = std::max(hi[0], x); hi[1] = std::max(hi[1], y); hi[2] = std::max(hi[2], z);
-    };
-    std::vector<float4> nrm;
-    for (int64_t i = 0; i < nt; i++) {
-        const float *p = &s->pos[i * 9];
-        int tag = PT_TAG_FLAT;
-        if (s->hasNormals) {
-            // keep per-vertex normals only where they differ from the flat normal
-            const float e1[3] = {p[3] - p[0], p[4] - p[1], p[5] - p[2]}, e2[3] = {p[6] - p[0], p[7] - p[1], p[8] - p[2]};
-            float g[3] = {e1[1] * e2[2] - e1[2] * e2[1], -(e1[0] * e2[2] - e1[2] * e2[0]), e1[0] * e2[1] - e1[1] * e2[0]};
-            const float gl = sqrtf(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]);
-            bool flat = gl > 0.f;
-            const float *nv = &s->nrm[i * 9];
-            for (int v = 0; v < 3 && flat; v++)
-                for (int k = 0; k < 3; k++)
-                    if (fabsf(nv[v * 3 + k] - g[k] / gl) > 1e-6f) flat = false;
-            if (!flat) {
-                tag = (int)(nrm.size() / 3);
-                for (int v = 0; v < 3; v++) nrm.push_back(make_float4(nv[v * 3], nv[v * 3 + 1], nv[v * 3 + 2], 0.f));
-            }
-        }
-        recs[i * 3] = make_float4(p[0], p[1], p[2], asFloat(s->triMat[i]));
-        recs[i * 3 + 1] = make_float4(p[3], p[4], p[5], asFloat(tag));
-        recs[i * 3 + 2] = make_float4(p[6], p[7], p[8], asFloat((int)i));
-        for (int v = 0; v < 3; v++) grow(p[v * 3], p[v * 3 + 1], p[v * 3 + 2]);
-    }
-    for (int64_t i = 0; i < ns; i++) {
-        const float *q = &s->sph[i * 4];
-        const int64_t k = nt + i;
-        recs[k * 3] = make_float4(q[0], q[1], q[2], asFloat(s->sphMat[i]));
-        recs[k * 3 + 1] = make_float4(q[3], 0.f, 0.f, asFloat(PT_TAG_SPHERE));
-        recs[k * 3 + 2] = make_float4(0.f, 0.f, 0.f, asFloat(~(int)i));
-        grow(q[0], q[1], q[2]);
-    }
-    r->primsIn.alloc(recs.size() * sizeof(float4));
-    PT_HIP_TRY(hipMemcpyAsync(r->primsIn.p, recs.data(), recs.size() * sizeof(float4), hipMemcpyHostToDevice, r->stream));
-    r->prims.alloc(recs.size() * sizeof(float4));
-    r->normals.alloc(std::max<size_t>(nrm.size(), 1) * sizeof(float4));
-    if (!nrm.empty()) PT_HIP_TRY(hipMemcpyAsync(r->normals.p, nrm.data(), nrm.size() * sizeof(float4), hipMemcpyHostToDevice, r->stream));
+    float lo[3], hi[3];
+    r->scene.load(*s, r->primsIn, r->normals, lo, hi, r->stream);
+    r->prims.alloc(sizeof(float4) * 3 * (size_t)std::max<int64_t>(n, 1));
     for (int k = 0; k < 3; k++) {
         r->sceneLo[k] = std::isfinite(lo[k]) ? lo[k] : 0.f;
         r->sceneHi[k] = std::isfinite(hi[k]) ? hi[k] : 1.f;
@@ -2319,8 +2237,10 @@ int pt_renderer_set_scene(pt_renderer *r, const pt_scene *s) {
     r->view.normals = r->normals.as<float4>();
     r->view.numPrims = (int)n;
     r->view.numNodes = r->bvh.numNodes;
-    uploadMaterials(r);
-    uploadEmitters(r);
+    r->scene.buildMaterials(r->materials, r->stream);
+    r->view.materials = r->materials.as<PtMaterial>();
+    r->view.numMaterials = r->scene.nMat;
+    buildEmitters(r);
     // environment
     r->view.env = PtEnv{};
     if (s->envW > 0 && s->envH > 0) {
@@ -2372,21 +2292,20 @@ int pt_renderer_set_camera(pt_renderer *r, const float origin[3], const float ta
 int pt_renderer_set_material(pt_renderer *r, int id, int type, const float albedo[3], const float emit[3], float ior, float alpha) {
     if (guard("pt_renderer_set_material", r)) return PT_ERR_INVALID;
     if (!r->hasScene) return fail(PT_ERR_STATE, "pt_renderer_set_material: no scene");
-    if (id < 0 || id >= (int)r->mats.size()) return fail(PT_ERR_INVALID, "pt_renderer_set_material: material id out of range");
+    if (id < 0 || id >= r->scene.nMat) return fail(PT_ERR_INVALID, "pt_renderer_set_material: material id out of range");
     if (type < PT_LAMBERTIAN || type > PT_MICROFACET) return fail(PT_ERR_INVALID, "pt_renderer_set_material: bad material type");
     if (r->inFlight) return fail(PT_ERR_STATE, "pt_renderer_set_material: a pass is still running");
     PT_API_BEGIN
-    HostMaterial &m = r->mats[id];
+    PT_HIP_TRY(hipStreamSynchronize(r->stream));
+    HostMaterial m = r->scene.material(id, r->stream);
     const bool wasEmissive = isEmissive(m);
     m.type = type;
     if (albedo) memcpy(m.albedo, albedo, 12);
     if (emit) memcpy(m.emit, emit, 12);
     m.ior = ior;
     m.alpha = alpha;
-    PT_HIP_TRY(hipStreamSynchronize(r->stream));
-    uploadMaterials(r);
-    if (wasEmissive || isEmissive(m)) uploadEmitters(r);
-    PT_HIP_TRY(hipStreamSynchronize(r->stream));
+    r->scene.setMaterial(id, m, r->materials, r->stream);
+    if (wasEmissive || isEmissive(m)) buildEmitters(r);
     r->resetPending = true;
     return PT_OK;
     PT_API_END("pt_renderer_set_material")
@@ -3057,7 +2976,7 @@ void prepareBatch(pt_batch *b, int scale) {
     for (size_t j = 0; j < b->jobs.size(); j++) b->order[j] = (int)j;
     auto cost = [&](int j) {
         const pt_renderer *r = b->jobs[j];
-        return (double)r->W * r->H * b->spp[j] * std::log2(2.0 + (double)r->triMat.size() + (double)r->sphMat.size());
+        return (double)r->W * r->H * b->spp[j] * std::log2(2.0 + (double)r->scene.nTri + (double)r->scene.nSph);
     };
     std::stable_sort(b->order.begin(), b->order.end(), [&](int x, int y) { return cost(x) < cost(y); });
     if (b->wavefront) {
@@ -3084,7 +3003,7 @@ void buildWave(pt_batch *b) {
         nN += r->bvh.numNodes;
         nP += r->view.numPrims;
         nNrm += (int64_t)(r->normals.bytes / sizeof(float4));
-        nM += (int64_t)r->mats.size();
+        nM += r->scene.nMat;
         nE += r->view.numEmitters;
         w->stackNeed = std::max(w->stackNeed, r->stackNeed);
     }
@@ -3100,7 +3019,7 @@ void buildWave(pt_batch *b) {
     for (size_t j = 0; j < b->jobs.size(); j++) {
         pt_renderer *r = b->jobs[j];
         const int nn = r->bvh.numNodes, np = r->view.numPrims, ne = r->view.numEmitters;
-        const int64_t nrm = (int64_t)(r->normals.bytes / sizeof(float4)), nm = (int64_t)r->mats.size();
+        const int64_t nrm = (int64_t)(r->normals.bytes / sizeof(float4)), nm = r->scene.nMat;
         float4 *dn = w->nodes.as<float4>() + (size_t)PT_NODE_F4 * oN, *dp = w->prims.as<float4>() + 3 * (size_t)oP;
         float4 *de = w->emitters.as<float4>() + 3 * (size_t)oE;
         PT_HIP_TRY(hipMemcpyAsync(dn, r->nodes.p, sizeof(float4) * PT_NODE_F4 * (size_t)nn, hipMemcpyDeviceToDevice, b->stream));
@@ -3624,7 +3543,7 @@ int pt_batch_get_render_stats(pt_batch *b, int index, pt_batch_render_stats *out
     out->width = r->W;
     out->height = r->H;
     out->spp = (int)r->spp;
-    out->triangles = (int64_t)r->triMat.size();
+    out->triangles = (int64_t)r->scene.nTri;
     out->rays = renderRays(b, index);
     out->latency_ms = index < (int)b->latencyMs.size() ? b->latencyMs[index] : 0.0;
     return PT_OK;

@@ -1,0 +1,271 @@
+// pt_upload.hip -- the scene's device records made on the device from the host arrays as they are.
+//
+// A scene upload copies positions, material ids, spheres and materials to the device unchanged
+// and builds the 48-byte primitive records, the 32-byte material records, the scene bounds, the
+// per-vertex normals worth keeping and the emitter list there.  What bounds it is the copy over
+// the host link (80 B per triangle of a scene with per-face materials).  Making the records on
+// the host wrote and faulted in another 170 B per triangle of fresh host memory for one pass of
+// trivial work: 1.31M triangles with per-face materials took 43 ms on the host before, beside
+// 21 ms of kernels.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+
+#include "pt_gpu.h"
+#include "pt_internal.h"
+
+namespace pt {
+
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kBoundsBlocks = 512;
+inline unsigned blocksOf(int64_t n) { return (unsigned)std::max<int64_t>(1, (n + kThreads - 1) / kThreads); }
+
+__global__ __launch_bounds__(kThreads) void k_upload_prims(const float *pos, const int *triMat, const uint32_t *normalAt, const uint32_t *smooth, int nt,
+                                                           const float *sph, const int *sphMat, int ns, float4 *recs) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nt) {
+        const float *p = pos + 9 * (size_t)i;
+        // smooth triangles point at their three normals, in order
+        const int tag = smooth && smooth[i] ? (int)normalAt[i] : PT_TAG_FLAT;
+        recs[3 * (size_t)i] = make_float4(p[0], p[1], p[2], asFloat(triMat[i]));
+        recs[3 * (size_t)i + 1] = make_float4(p[3], p[4], p[5], asFloat(tag));
+        recs[3 * (size_t)i + 2] = make_float4(p[6], p[7], p[8], asFloat(i));
+    } else if (i < nt + ns) {
+        const int k = i - nt;
+        const float *q = sph + 4 * (size_t)k;
+        recs[3 * (size_t)i] = make_float4(q[0], q[1], q[2], asFloat(sphMat[k]));
+        recs[3 * (size_t)i + 1] = make_float4(q[3], 0.f, 0.f, asFloat(PT_TAG_SPHERE));
+        recs[3 * (size_t)i + 2] = make_float4(0.f, 0.f, 0.f, asFloat(~k));
+    }
+}
+
+// Bounds of the records' vertices and sphere centres: a box per block, then one block's fold.
+__device__ __forceinline__ void blockBounds(float lo[3], float hi[3], float *out) {
+    __shared__ float part[kThreads / 64][6];
+    for (int k = 0; k < 3; k++)
+        for (int off = 32; off >= 1; off >>= 1) {
+            lo[k] = fminf(lo[k], __shfl_xor(lo[k], off));
+            hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], off));
+        }
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < 3; k++) {
+            part[threadIdx.x >> 6][k] = lo[k];
+            part[threadIdx.x >> 6][3 + k] = hi[k];
+        }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int k = 0; k < 6; k++) {
+            float v = part[0][k];
+            for (int w = 1; w < kThreads / 64; w++) v = k < 3 ? fminf(v, part[w][k]) : fmaxf(v, part[w][k]);
+            out[k] = v;
+        }
+}
+
+__global__ __launch_bounds__(kThreads) void k_bounds(const float4 *recs, int n, float *boxes) {
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    auto grow = [&](float4 v) {
+        const float c[3] = {v.x, v.y, v.z};
+        for (int k = 0; k < 3; k++) {
+            lo[k] = fminf(lo[k], c[k]);
+            hi[k] = fmaxf(hi[k], c[k]);
+        }
+    };
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const float4 a = recs[3 * (size_t)i], b = recs[3 * (size_t)i + 1], c = recs[3 * (size_t)i + 2];
+        grow(a);
+        if (asInt(b.w) != PT_TAG_SPHERE) {
+            grow(b);
+            grow(c);
+        }
+    }
+    blockBounds(lo, hi, boxes + 6 * blockIdx.x);
+}
+
+__global__ __launch_bounds__(kThreads) void k_bounds_fold(const float *boxes, int n, float *out) {
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int i = threadIdx.x; i < n; i += blockDim.x)
+        for (int k = 0; k < 3; k++) {
+            lo[k] = fminf(lo[k], boxes[6 * i + k]);
+            hi[k] = fmaxf(hi[k], boxes[6 * i + 3 + k]);
+        }
+    blockBounds(lo, hi, out);
+}
+
+// 1 where a triangle's per-vertex normals differ from its flat one (only those are kept).
+__global__ __launch_bounds__(kThreads) void k_smooth_flags(const float *pos, const float *nrm, int nt, uint32_t *smooth, uint32_t *rank) {
+#pragma clang fp contract(off)
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nt) return;
+    const float *p = pos + 9 * (size_t)i, *nv = nrm + 9 * (size_t)i;
+    const float e1[3] = {p[3] - p[0], p[4] - p[1], p[5] - p[2]}, e2[3] = {p[6] - p[0], p[7] - p[1], p[8] - p[2]};
+    const float g[3] = {e1[1] * e2[2] - e1[2] * e2[1], -(e1[0] * e2[2] - e1[2] * e2[0]), e1[0] * e2[1] - e1[1] * e2[0]};
+    const float gl = sqrtf(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]);
+    bool flat = gl > 0.f;
+    for (int v = 0; v < 3; v++)
+        for (int k = 0; k < 3; k++)
+            if (fabsf(nv[v * 3 + k] - g[k] / gl) > 1e-6f) flat = false;
+    smooth[i] = flat ? 0u : 1u;
+    rank[i] = flat ? 0u : 1u;
+}
+
+__global__ __launch_bounds__(kThreads) void k_keep_normals(const float *nrm, const uint32_t *smooth, const uint32_t *rank, int nt, float4 *out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nt || !smooth[i]) return;
+    const float *nv = nrm + 9 * (size_t)i;
+    for (int v = 0; v < 3; v++) out[3 * (size_t)rank[i] + v] = make_float4(nv[3 * v], nv[3 * v + 1], nv[3 * v + 2], 0.f);
+}
+
+// Emission is a Lambertian's alone (params.h:37-70).
+__device__ __forceinline__ bool emits(const HostMaterial &m) {
+    return m.type == PT_LAMBERTIAN && (m.emit[0] != 0.f || m.emit[1] != 0.f || m.emit[2] != 0.f);
+}
+
+__global__ __launch_bounds__(kThreads) void k_materials(const HostMaterial *mats, int first, int n, PtMaterial *out) {
+    const int i = first + blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= first + n) return;
+    const HostMaterial h = mats[i];
+    const bool lamb = h.type == PT_LAMBERTIAN;
+    const float param = h.type == PT_GLASS ? h.ior : (h.type == PT_MICROFACET ? h.alpha : 0.f);
+    out[i].a = make_float4(h.albedo[0], h.albedo[1], h.albedo[2], (float)h.type);
+    out[i].b = make_float4(lamb ? h.emit[0] : 0.f, lamb ? h.emit[1] : 0.f, lamb ? h.emit[2] : 0.f, param);
+}
+
+__global__ __launch_bounds__(kThreads) void k_emitter_flags(const HostMaterial *mats, const int *triMat, int nt, const int *sphMat, int ns,
+                                                            uint32_t *rank) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nt + ns) return;
+    rank[i] = emits(mats[i < nt ? triMat[i] : sphMat[i - nt]]) ? 1u : 0u;
+}
+
+// Emitter records in the reference light order (scene_data.cu:92-115): emissive triangles by
+// index, then emissive spheres.  Their normals are the flat ones.
+__global__ __launch_bounds__(kThreads) void k_emitters(const HostMaterial *mats, const float *pos, const int *triMat, int nt, const float *sph,
+                                                       const int *sphMat, int ns, const uint32_t *rank, float4 *out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nt + ns) return;
+    float4 *o = out + 3 * (size_t)rank[i];
+    if (i < nt) {
+        const int mat = triMat[i];
+        if (!emits(mats[mat])) return;
+        const float *p = pos + 9 * (size_t)i;
+        o[0] = make_float4(p[0], p[1], p[2], asFloat(mat));
+        o[1] = make_float4(p[3], p[4], p[5], asFloat(PT_TAG_FLAT));
+        o[2] = make_float4(p[6], p[7], p[8], asFloat(i));
+    } else {
+        const int k = i - nt, mat = sphMat[k];
+        if (!emits(mats[mat])) return;
+        const float *s = sph + 4 * (size_t)k;
+        o[0] = make_float4(s[0], s[1], s[2], asFloat(mat));
+        o[1] = make_float4(s[3], 0.f, 0.f, asFloat(PT_TAG_SPHERE));
+        o[2] = make_float4(0.f, 0.f, 0.f, asFloat(~k));
+    }
+}
+
+template <class T> void upload(T *d, const std::vector<T> &v, hipStream_t stream) {
+    if (!v.empty()) PT_HIP_TRY(hipMemcpyAsync(d, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, stream));
+}
+
+}  // namespace
+
+void SceneArrays::load(const pt_scene &s, DevBuf &records, DevBuf &normals, float lo[3], float hi[3], hipStream_t stream) {
+    nTri = (int)s.triMat.size();
+    nSph = (int)s.sphMat.size();
+    nMat = (int)s.mats.size();
+    const int n = nTri + nSph;
+    const bool smoothed = s.hasNormals && nTri > 0;
+    arrays.want(pos, s.pos.size());
+    arrays.want(triMat, s.triMat.size());
+    arrays.want(sph, s.sph.size());
+    arrays.want(sphMat, s.sphMat.size());
+    arrays.want(mats, s.mats.size());
+    arrays.alloc();
+    WorkArrays work;
+    float *nrm = nullptr, *boxes;
+    uint32_t *smooth = nullptr, *rank = nullptr, *scanTmp = nullptr;
+    work.want(boxes, 6 * (kBoundsBlocks + 1));
+    if (smoothed) {
+        work.want(nrm, s.nrm.size());
+        work.want(smooth, nTri);
+        work.want(rank, (size_t)nTri + 1);
+        work.want(scanTmp, scanEntries(nTri));
+    }
+    work.alloc();
+    upload(pos, s.pos, stream);
+    upload(triMat, s.triMat, stream);
+    upload(sph, s.sph, stream);
+    upload(sphMat, s.sphMat, stream);
+    upload(mats, s.mats, stream);
+    if (smoothed) {
+        upload(nrm, s.nrm, stream);
+        k_smooth_flags<<<blocksOf(nTri), kThreads, 0, stream>>>(pos, nrm, nTri, smooth, rank);
+        scanCounts(rank, nTri, scanTmp, stream);
+        uint32_t kept = 0;
+        PT_HIP_TRY(hipMemcpyAsync(&kept, rank + nTri, sizeof kept, hipMemcpyDeviceToHost, stream));
+        PT_HIP_TRY(hipStreamSynchronize(stream));
+        normals.alloc(std::max<size_t>(3 * (size_t)kept, 1) * sizeof(float4));
+        k_keep_normals<<<blocksOf(nTri), kThreads, 0, stream>>>(nrm, smooth, rank, nTri, normals.as<float4>());
+    } else {
+        normals.alloc(sizeof(float4));
+    }
+    records.alloc(sizeof(float4) * 3 * (size_t)std::max(n, 1));
+    k_upload_prims<<<blocksOf(n), kThreads, 0, stream>>>(pos, triMat, rank, smooth, nTri, sph, sphMat, nSph, records.as<float4>());
+    const int bb = (int)std::min<unsigned>(kBoundsBlocks, blocksOf(n));
+    k_bounds<<<bb, kThreads, 0, stream>>>(records.as<float4>(), n, boxes);
+    k_bounds_fold<<<1, kThreads, 0, stream>>>(boxes, bb, boxes + 6 * kBoundsBlocks);
+    PT_HIP_TRY(hipGetLastError());
+    float b[6];
+    PT_HIP_TRY(hipMemcpyAsync(b, boxes + 6 * kBoundsBlocks, sizeof b, hipMemcpyDeviceToHost, stream));
+    PT_HIP_TRY(hipStreamSynchronize(stream));
+    for (int k = 0; k < 3; k++) {
+        lo[k] = b[k];
+        hi[k] = b[3 + k];
+    }
+}
+
+HostMaterial SceneArrays::material(int id, hipStream_t stream) const {
+    HostMaterial m;
+    PT_HIP_TRY(hipMemcpyAsync(&m, mats + id, sizeof m, hipMemcpyDeviceToHost, stream));
+    PT_HIP_TRY(hipStreamSynchronize(stream));
+    return m;
+}
+
+void SceneArrays::setMaterial(int id, const HostMaterial &m, DevBuf &records, hipStream_t stream) {
+    PT_HIP_TRY(hipMemcpyAsync(mats + id, &m, sizeof m, hipMemcpyHostToDevice, stream));
+    k_materials<<<1, kThreads, 0, stream>>>(mats, id, 1, records.as<PtMaterial>());
+    PT_HIP_TRY(hipGetLastError());
+    PT_HIP_TRY(hipStreamSynchronize(stream));
+}
+
+void SceneArrays::buildMaterials(DevBuf &records, hipStream_t stream) const {
+    records.alloc(sizeof(PtMaterial) * (size_t)std::max(nMat, 1));
+    if (nMat > 0) k_materials<<<blocksOf(nMat), kThreads, 0, stream>>>(mats, 0, nMat, records.as<PtMaterial>());
+    PT_HIP_TRY(hipGetLastError());
+}
+
+int SceneArrays::buildEmitters(DevBuf &records, hipStream_t stream) const {
+    const int n = nTri + nSph;
+    uint32_t count = 0, *rank, *scanTmp;
+    WorkArrays work;
+    if (n > 0) {
+        work.want(rank, (size_t)n + 1);
+        work.want(scanTmp, scanEntries(n));
+        work.alloc();
+        k_emitter_flags<<<blocksOf(n), kThreads, 0, stream>>>(mats, triMat, nTri, sphMat, nSph, rank);
+        scanCounts(rank, n, scanTmp, stream);
+        PT_HIP_TRY(hipMemcpyAsync(&count, rank + n, sizeof count, hipMemcpyDeviceToHost, stream));
+        PT_HIP_TRY(hipStreamSynchronize(stream));
+    }
+    records.alloc(sizeof(float4) * std::max<size_t>(3 * (size_t)count, 1));
+    if (count > 0) {
+        k_emitters<<<blocksOf(n), kThreads, 0, stream>>>(mats, pos, triMat, nTri, sph, sphMat, nSph, rank, records.as<float4>());
+        PT_HIP_TRY(hipGetLastError());
+        // the ranks are freed on return
+        PT_HIP_TRY(hipStreamSynchronize(stream));
+    }
+    return (int)count;
+}
+
+}  // namespace pt
