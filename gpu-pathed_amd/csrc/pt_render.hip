@@ -364,10 +364,28 @@ __device__ __forceinline__ Rng cameraRng(const ChunkParams &cp, int path) {
 // the nearest is visited next and the others are pushed far-first on a per-lane stack (any-hit
 // queries too: nearer occluders are found sooner).
 //
-// The stack has two levels: the top LDS entries of each lane (stack[level * blockDim + lane],
-// LDS entries per lane) and, below them, a spill area in global memory interleaved by lane
-// (spill[(level - LDS) * lanes + lane]), sized for the deepest stack the tree can need.  The
-// small LDS part keeps the trace kernels' occupancy high; deep stacks are rare.
+// The stack of a lane is a column of LDS rows (kTraceThreads ints apart): a sentinel at the
+// bottom, the newest STACK or so entries above it, and below those, for trees that need them,
+// older entries in a spill area in global memory interleaved by lane
+// (spill[entry * lanes + lane]).  When the LDS part fills up its older half moves to the spill
+// area, and when the sentinel comes up with entries spilled the newest of them move back: both
+// are rare, and the node step itself knows only LDS.
+//
+// What bounds the kernels is the L1's lookup rate, one access per cycle and CU: every lane's 16
+// bytes of a node are an access of their own (neighbouring lanes rarely hold the same node), seven
+// per node visit, and they fill 99% of the cycles of the icosphere's incoherent bounces (TD busy
+// 100%, VALU 69%).  The node step leaves those loads as they are and needs few instructions beside
+// them (about 85; the first version's, with a compare-and-select sorting network, separate push,
+// pop and leaf branches and the stack's row stride in a register, took about 150 and VALU issue was
+// the larger share: room extend 7087 -> 6594 us and shadow 4004 -> 3802 us a pass, icosphere extend
+// 7425 -> 7028 us and shadow 4944 -> 4600 us):
+//  - the children are sorted as 64-bit keys, entry distance above child reference, with
+//    v_min_f64 / v_max_f64: two instructions per exchange instead of five.  A key's upper word is
+//    a finite float's bits, or +-infinity's, so the key is an ordinary double and orders as one;
+//    children at equal distances are ordered by reference;
+//  - all four children are written to the stack, farthest first, missed ones last, and the top
+//    is read back: one path for the nearest child, for a pop after a node without hits, and for
+//    the entry below, which is next when the top one is a leaf to park.
 //
 // Scheduling: a wave runs traversal rounds (descent to a leaf, the leaf's primitives, one pop)
 // on every lane that holds a ray, and lanes whose ray has finished take new rays from the
@@ -383,12 +401,56 @@ struct TraceHit {
 
 typedef __attribute__((address_space(3))) int LdsInt;
 
+// Rows of a lane's stack column: a spare one (read, never used, below the sentinel), the
+// sentinel, the entries, those that kDescentSteps node steps can add past the last, and the
+// number of spilled entries.
+static constexpr int kStackSentinel = 1;
+static constexpr int kStackFirst = 2;
+constexpr int stackCountRow(int entries) { return kStackFirst + entries + 6; }
+constexpr int stackRows(int entries) { return stackCountRow(entries) + 1; }
+
 struct TraceStack {
-    LdsInt *lds;    // this lane's first LDS entry; entries blockDim.x apart
-    int *spill;     // this lane's first spill entry; entries spillStride apart
-    int spillCap;   // spill entries per lane
+    LdsInt *column;   // this lane's row 0; rows kTraceThreads apart
+    int *spill;       // this lane's first spill entry; entries spillStride apart
+    int spillCap;     // spill entries per lane (0: the tree never needs them)
     int spillStride;
 };
+
+// Largest and smallest of floats that are never signalling NaNs (the compiler quiets its operands
+// first, an instruction each time round a loop).
+__device__ __forceinline__ float max2(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float min2(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float min3(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// A sort key: a float (not NaN) above a child reference.
+__device__ __forceinline__ double sortKey(float t, int ref) {
+    return __builtin_bit_cast(double, (uint64_t)(uint32_t)asInt(t) << 32 | (uint32_t)ref);
+}
+__device__ __forceinline__ int keyRef(double k) { return (int)(uint32_t)__builtin_bit_cast(uint64_t, k); }
+// a becomes the larger of the two, b the smaller
+__device__ __forceinline__ void keyOrder(double &a, double &b) {
+    double hi, lo;
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    a = hi;
+    b = lo;
+}
 
 __device__ __forceinline__ void cswap(float &ta, int &ra, float &tb, int &rb) {
     const bool s = tb < ta;
@@ -402,8 +464,9 @@ __device__ __forceinline__ void cswap(float &ta, int &ra, float &tb, int &rb) {
 
 // One ray in flight on a lane: the slab-test and watertight-test set-ups, the search interval
 // (tmax is the closest hit's distance once prim >= 0), the closest hit's primitive and
-// barycentrics, and the traversal position (node >= 0: a 4-wide node; < 0: the rest of a
-// leaf, ~((remaining - 1) << PT_LEAF_COUNT_SHIFT | next primitive); sp: stack depth).
+// barycentrics, and the traversal position (node >= 0: a 4-wide node; < 0: a leaf,
+// ~((primitives - 1) << PT_LEAF_COUNT_SHIFT | first), or kTraceDone; sp: the stack's first free
+// entry).
 struct LaneRay {
     WtRay wr;
     f3 d;
@@ -412,7 +475,8 @@ struct LaneRay {
     float tmin, tmax;
     float u, v;
     int prim;
-    int node, sp;
+    int node;
+    LdsInt *sp;
 };
 
 __device__ __forceinline__ void laneRayStart(LaneRay &r, f3 o, f3 d, float tmin, float tmax, int root = 0) {
@@ -436,7 +500,6 @@ __device__ __forceinline__ void laneRayStart(LaneRay &r, f3 o, f3 d, float tmin,
     r.v = 0.f;
     r.prim = INT32_MIN;
     r.node = root;
-    r.sp = 0;
 }
 
 __device__ __forceinline__ TraceHit laneRayHit(const LaneRay &r) {
@@ -448,25 +511,11 @@ __device__ __forceinline__ TraceHit laneRayHit(const LaneRay &r) {
     return th;
 }
 
-// One traversal round of a lane's ray.  The wave descends through 4-wide nodes, nearest hit
-// child first, popping the stack after a node whose children all miss, until (nearly) every
-// lane has found a leaf or exhausted its stack; a lane that finds a leaf while others are
-// still searching parks it and keeps descending (speculatively, with the interval it has), up
-// to a second leaf.  Then the parked leaves' primitives are tested together.  Leaves are tested in
-// the order a depth-first traversal reaches them, and a node visited only because its leaf
-// was parked holds no primitive at or below the final tmax, so the hit does not depend on the
-// schedule.  Returns true when the ray is finished: the stack is exhausted, or an any-hit query
-// found an occluder.
 static constexpr int kTraceDone = INT32_MIN;   // LaneRay::node once the stack is exhausted
 // Searching lanes a wave leaves behind to test its parked leaves: waiting for the last few
-// lanes of a round costs more than another round (C1: 4 -> 3398, 12 -> 3413, 20 -> 3347,
-// 32 -> 3250 Mrays/s; 0, wait for every lane: 3207; on the current tree 8 -> 4395,
-// 12 -> 4420, 16 -> 4408)
+// lanes of a round costs more than another round.
 static constexpr int kDescentTail = 12;
-// Node steps per check of the descent's exit conditions: two steps save the ballots of every
-// other step (C1 4452 -> 4498 Mrays/s with the trace kernels' register cap raised from 72 to
-// 80, six waves per SIMD, which the default 11 blocks per CU do not exceed; at 72 registers the
-// second step spills).
+// Node steps per check of the descent's exit conditions and of the stack's room.
 static constexpr int kDescentSteps = 2;
 
 // Per-lane traversal counts of the instrumented trace kernels (STATS).
@@ -474,104 +523,114 @@ struct TraceCount {
     int rays = 0, nodes = 0, prims = 0;
 };
 
+template <int STACK> __device__ __forceinline__ void stackStart(LaneRay &r, const TraceStack &ts) {
+    r.sp = ts.column + kStackFirst * kTraceThreads;
+    if (ts.spillCap > 0) ts.column[stackCountRow(STACK) * kTraceThreads] = 0;
+}
+
+// Makes room: the older half of the LDS entries moves to the spill area.
+template <int STACK> __device__ __forceinline__ LdsInt *stackEvict(LdsInt *sp, const TraceStack ts, int *overflow) {
+    constexpr int kMove = STACK / 2;
+    LdsInt *first = ts.column + kStackFirst * kTraceThreads;
+    LdsInt *count = ts.column + stackCountRow(STACK) * kTraceThreads;
+    const int n = *count;
+    if (n + kMove > ts.spillCap) {
+        atomicAdd(overflow, 1);
+        return first;   // the traversal ends early; the caller of the pass is told
+    }
+    for (int k = 0; k < kMove; k++) ts.spill[(size_t)(n + k) * ts.spillStride] = first[k * kTraceThreads];
+    *count = n + kMove;
+    LdsInt *to = first;
+    for (LdsInt *from = first + kMove * kTraceThreads; from < sp; from += kTraceThreads, to += kTraceThreads) *to = *from;
+    return to;
+}
+
+// Moves the newest spilled entries back into an empty LDS part; returns its first free entry (the
+// one above the sentinel when nothing was spilled).
+template <int STACK> __device__ __forceinline__ LdsInt *stackRefill(const TraceStack ts) {
+    constexpr int kMove = STACK / 2;
+    LdsInt *first = ts.column + kStackFirst * kTraceThreads;
+    LdsInt *count = ts.column + stackCountRow(STACK) * kTraceThreads;
+    const int n = *count;
+    if (n == 0) return first;
+    for (int k = 0; k < kMove; k++) first[k * kTraceThreads] = ts.spill[(size_t)(n - kMove + k) * ts.spillStride];
+    *count = n - kMove;
+    return first + kMove * kTraceThreads;
+}
+
+// One traversal round of a lane's ray.  The wave descends through 4-wide nodes, nearest hit
+// child first, until (nearly) every lane has found a leaf or exhausted its stack; a lane that
+// finds a leaf while others are still searching parks it and keeps descending (speculatively,
+// with the interval it has), up to a second leaf.  Then the parked leaves' primitives are tested
+// together.  Leaves are tested in the order a depth-first traversal reaches them, and a node
+// visited only because its leaf was parked holds no primitive at or below the final tmax, so the
+// hit does not depend on the schedule.  Returns true when the ray is finished: the stack is
+// exhausted, or an any-hit query found an occluder.
 template <bool ANY, int STACK, bool STATS = false>
 __device__ __forceinline__ bool traceRound(const PtSceneView &sc, LaneRay &r, const TraceStack &ts, int *overflow, TraceCount *tc = nullptr) {
-    const int stride = blockDim.x;
-    // general push (LDS, then the spill area); the common closest-hit case writes LDS directly
-    auto push = [&](int ref) {
-        if (r.sp < STACK) {
-            ts.lds[r.sp * stride] = ref;
-            r.sp++;
-        } else if (r.sp - STACK < ts.spillCap) {
-            ts.spill[(size_t)(r.sp - STACK) * ts.spillStride] = ref;
-            r.sp++;
-        } else {
-            atomicAdd(overflow, 1);
-        }
-    };
-    auto pop = [&]() {
-        if (r.sp == 0) {
-            r.node = kTraceDone;
-        } else {
-            r.sp--;
-            // an LDS read at a clamped level and, only below the LDS part, the spill read (the
-            // LDS pointer's address space keeps the two from becoming one flat load)
-            int v = ts.lds[min(r.sp, STACK - 1) * stride];
-            if (r.sp >= STACK) v = ts.spill[(size_t)(r.sp - STACK) * ts.spillStride];
-            r.node = v;
-        }
-    };
     const char *nodes = (const char *)sc.nodes;
     int leaf = 0;   // parked leaf reference (< 0), or 0
+    if (r.node < 0) {
+        // the second leaf of the last round (a finished ray is not traced further)
+        leaf = r.node;
+        r.sp -= kTraceThreads;
+        r.node = *r.sp;
+    }
     while (true) {
         // the descent ends when no lane is still looking for a leaf, or when at most
         // kDescentTail lanes are and at least one lane holds a parked leaf (the searching
         // lanes carry on next round); every pass through this loop moves a searching lane on
-        const uint64_t searching = __ballot(leaf == 0 && r.node != kTraceDone);
+        const uint64_t searching = __ballot(leaf == 0 && r.node >= 0);
         if (searching == 0) break;
         if (__popcll(searching) <= kDescentTail && __ballot(leaf != 0) != 0) break;
-        // kDescentSteps node steps per check of the exit conditions: a lane that parks a leaf
-        // in the first step keeps descending internal nodes in the next (as it would while
-        // other lanes search) and idles at its second leaf, so only the checks' cost changes
+        if (ts.spillCap > 0 && r.sp > ts.column + (kStackFirst + STACK - 1) * kTraceThreads) r.sp = stackEvict<STACK>(r.sp, ts, overflow);
+        // a lane that parks a leaf in the first step keeps descending internal nodes in the next
+        // (as it would while other lanes search) and idles at its second leaf
 #pragma unroll
         for (int step = 0; step < kDescentSteps; step++) {
-        if (r.node >= 0) {
-            if constexpr (STATS) tc->nodes++;
-            // 32-bit offsets from the array base (a node array stays below 4 GiB); a node is
-            // 128 bytes, so the near bound's offset is an OR and the far bound of the same axis
-            // (the other float4 of the pair) is that offset XOR 16
-            const uint32_t base = (uint32_t)r.node * (uint32_t)(PT_NODE_F4 * 16);
-            const uint32_t ax = base | r.nX, ay = base | r.nY, az = base | r.nZ;
-            const float4 nx = *(const float4 *)(nodes + ax), fx = *(const float4 *)(nodes + (ax ^ 16u));
-            const float4 ny = *(const float4 *)(nodes + ay), fy = *(const float4 *)(nodes + (ay ^ 16u));
-            const float4 nz = *(const float4 *)(nodes + az), fz = *(const float4 *)(nodes + (az ^ 16u));
-            const int4 rf = *(const int4 *)(nodes + (base + 96u));
-            float tn[4];
-            int ref[4] = {rf.x, rf.y, rf.z, rf.w};
-            const float bnx[4] = {nx.x, nx.y, nx.z, nx.w}, bfx[4] = {fx.x, fx.y, fx.z, fx.w};
-            const float bny[4] = {ny.x, ny.y, ny.z, ny.w}, bfy[4] = {fy.x, fy.y, fy.z, fy.w};
-            const float bnz[4] = {nz.x, nz.y, nz.z, nz.w}, bfz[4] = {fz.x, fz.y, fz.z, fz.w};
+            if (r.node >= 0) {
+                if constexpr (STATS) tc->nodes++;
+                // 32-bit offsets from the array base (a node array stays below 4 GiB); a node is
+                // 128 bytes, so the near bound's offset is an OR and the far bound of the same axis
+                // (the other float4 of the pair) is that offset XOR 16
+                const uint32_t base = (uint32_t)r.node * (uint32_t)(PT_NODE_F4 * 16);
+                const uint32_t ax = base | r.nX, ay = base | r.nY, az = base | r.nZ;
+                const float4 nx = *(const float4 *)(nodes + ax), fx = *(const float4 *)(nodes + (ax ^ 16u));
+                const float4 ny = *(const float4 *)(nodes + ay), fy = *(const float4 *)(nodes + (ay ^ 16u));
+                const float4 nz = *(const float4 *)(nodes + az), fz = *(const float4 *)(nodes + (az ^ 16u));
+                const int4 rf = *(const int4 *)(nodes + (base + 96u));
+                const float bnx[4] = {nx.x, nx.y, nx.z, nx.w}, bfx[4] = {fx.x, fx.y, fx.z, fx.w};
+                const float bny[4] = {ny.x, ny.y, ny.z, ny.w}, bfy[4] = {fy.x, fy.y, fy.z, fy.w};
+                const float bnz[4] = {nz.x, nz.y, nz.z, nz.w}, bfz[4] = {fz.x, fz.y, fz.z, fz.w};
+                const int ref[4] = {rf.x, rf.y, rf.z, rf.w};
+                double key[4];
+                int hits = 0;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                // an unused slot holds an inverted box (lower bounds +1e30, upper -1e30): it misses
-                const float lo = fmaxf(fmaxf(bnx[k] * r.ix - r.ox, bny[k] * r.iy - r.oy), fmaxf(bnz[k] * r.iz - r.oz, r.tmin));
-                const float hi = fminf(fminf(bfx[k] * r.ix - r.ox, bfy[k] * r.iy - r.oy), fminf(bfz[k] * r.iz - r.oz, r.tmax));
-                tn[k] = lo <= hi ? lo : INFINITY;
-            }
-            // the references are used only when a child is hit; this empty statement keeps
-            // their load beside the box loads instead of after the box test, a second round
-            // trip on the common path
-            asm volatile("" : "+v"(ref[0]), "+v"(ref[1]), "+v"(ref[2]), "+v"(ref[3]));
-            // hit children nearest first (any-hit queries too: occluders nearer the origin are
-            // found sooner)
-            cswap(tn[0], ref[0], tn[1], ref[1]);
-            cswap(tn[2], ref[2], tn[3], ref[3]);
-            cswap(tn[0], ref[0], tn[2], ref[2]);
-            cswap(tn[1], ref[1], tn[3], ref[3]);
-            cswap(tn[1], ref[1], tn[2], ref[2]);
-            if (tn[0] == INFINITY) {
-                pop();
-            } else {
-                // hit children are a prefix of the sorted slots: push all but the nearest,
-                // the second nearest on top
-                const int more = (tn[1] != INFINITY) + (tn[2] != INFINITY) + (tn[3] != INFINITY);
-                if (r.sp + 3 <= STACK) {
-                    if (more >= 3) ts.lds[r.sp * stride] = ref[3];
-                    if (more >= 2) ts.lds[(r.sp + more - 2) * stride] = ref[2];
-                    if (more >= 1) ts.lds[(r.sp + more - 1) * stride] = ref[1];
-                    r.sp += more;
-                } else {
-                    if (more >= 3) push(ref[3]);
-                    if (more >= 2) push(ref[2]);
-                    if (more >= 1) push(ref[1]);
+                for (int k = 0; k < 4; k++) {
+                    // an unused slot holds an inverted box (lower bounds +1e30, upper -1e30): it misses
+                    const float lo = max3(bnx[k] * r.ix - r.ox, bny[k] * r.iy - r.oy, max2(bnz[k] * r.iz - r.oz, r.tmin));
+                    const float hi = min3(bfx[k] * r.ix - r.ox, bfy[k] * r.iy - r.oy, min2(bfz[k] * r.iz - r.oz, r.tmax));
+                    const bool in = lo <= hi;
+                    key[k] = sortKey(in ? lo : -INFINITY, ref[k]);
+                    hits += in ? 1 : 0;
                 }
-                r.node = ref[0];
+                // farthest first, missed children last
+                keyOrder(key[0], key[1]);
+                keyOrder(key[2], key[3]);
+                keyOrder(key[0], key[2]);
+                keyOrder(key[1], key[3]);
+                keyOrder(key[1], key[2]);
+#pragma unroll
+                for (int k = 0; k < 4; k++) r.sp[k * kTraceThreads] = keyRef(key[k]);
+                // the top: the nearest hit child, or without one the entry that was there before
+                LdsInt *top = r.sp + (hits - 1) * kTraceThreads;
+                const int first = top[0], second = top[-kTraceThreads];
+                const bool park = (uint32_t)first > (uint32_t)kTraceDone && leaf == 0;
+                leaf = park ? first : leaf;
+                r.node = park ? second : first;
+                r.sp = park ? top - kTraceThreads : top;
             }
-        } else if (leaf == 0 && r.node != kTraceDone) {
-            leaf = r.node;
-            pop();
-        }
-        // lanes holding a parked leaf and a second one, or done, wait for the others
+            // lanes holding a parked leaf and a second one, or done, wait for the others
         }
     }
     if (leaf != 0) {
@@ -607,12 +666,17 @@ __device__ __forceinline__ bool traceRound(const PtSceneView &sc, LaneRay &r, co
             }
         }
     }
+    if (r.node == kTraceDone && ts.spillCap > 0) {
+        r.sp = stackRefill<STACK>(ts) - kTraceThreads;
+        r.node = *r.sp;
+    }
     return r.node == kTraceDone;
 }
 
-__device__ __forceinline__ TraceStack traceStack(int *sstack, int *spill, int spillCap) {
+template <int STACK> __device__ __forceinline__ TraceStack traceStack(int *sstack, int *spill, int spillCap) {
     TraceStack ts;
-    ts.lds = (LdsInt *)(sstack + threadIdx.x);
+    ts.column = (LdsInt *)(sstack + threadIdx.x);
+    ts.column[kStackSentinel * kTraceThreads] = kTraceDone;
     ts.spillStride = gridDim.x * blockDim.x;
     ts.spill = spill + blockIdx.x * blockDim.x + threadIdx.x;
     ts.spillCap = spillCap;
@@ -698,6 +762,7 @@ __device__ __forceinline__ void traceQueue(const PtSceneView &sc, int *counters,
                     int root = 0;
                     load(ray, o, d, tmin, tmax, root);
                     laneRayStart(r, o, d, tmin, tmax, root);
+                    stackStart<STACK>(r, ts);
                     if constexpr (STATS) tc.rays++;
                 }
             }
@@ -726,12 +791,12 @@ __device__ __forceinline__ void traceQueue(const PtSceneView &sc, int *counters,
 // STATS: the instrumented build that adds its rays, node visits and primitive tests to
 // tstat[0..2].
 template <int STACK, bool BATCH = false, bool STATS = false>
-__global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 5) void k_extend(PtSceneView sc, int *counters, int bounce, int segLen,
+__global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_extend(PtSceneView sc, int *counters, int bounce, int segLen,
                                                                               const float4 *rayO, const float4 *rayD, float4 camO, float4 *hits,
                                                                               int refill, int *spill, int spillCap, int *overflow,
                                                                               ChunkParams cp = ChunkParams{}, unsigned long long *tstat = nullptr) {
-    __shared__ int sstack[STACK * kTraceThreads];
-    const TraceStack ts = traceStack(sstack, spill, spillCap);
+    __shared__ int sstack[stackRows(STACK) * kTraceThreads];
+    const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
     traceQueue<false, STACK, STATS>(
         sc, counters, bounce, PT_Q_RAYS, PT_Q_FETCH_EXT, segLen, refill, ts, overflow,
         [&](int i, f3 &o, f3 &d, float &tmin, float &tmax, int &root) {
@@ -886,15 +951,15 @@ __global__ __launch_bounds__(kTraceThreads, 6) void k_extend_packet(PtSceneView 
 // unoccluded ray adds its light contribution to its path.
 // BATCH: sL.w holds the ray's render, whose root node starts the traversal.
 template <int STACK, bool BATCH = false, bool STATS = false>
-__global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 5) void k_shadow(PtSceneView sc, int *counters, int bounce, int segLen,
+__global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_shadow(PtSceneView sc, int *counters, int bounce, int segLen,
                                                                               const float4 *sO, const float4 *sD, const float4 *sL, float4 *Lpath,
                                                                               int refill, int *spill, int spillCap, int *overflow,
                                                                               const BatchRender *renders = nullptr, unsigned long long *tstat = nullptr) {
-    __shared__ int sstack[STACK * kTraceThreads];
+    __shared__ int sstack[stackRows(STACK) * kTraceThreads];
     // each lane's path index, kept from the ray's load (a re-read after the traversal would be a
     // dependent round trip ahead of the radiance update)
     __shared__ int sPath[kTraceThreads];
-    const TraceStack ts = traceStack(sstack, spill, spillCap);
+    const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
     int adds = 0;
     traceQueue<true, STACK, STATS>(
         sc, counters, bounce, PT_Q_SHADOW, PT_Q_FETCH_SHADOW, segLen, refill, ts, overflow,
@@ -1828,7 +1893,7 @@ void zeroAccum(pt_renderer *r) {
 
 // Spill area of the traversal stacks: entries beyond the LDS part for every lane of the grid.
 int *ensureSpill(pt_renderer *r, int grid, int *cap) {
-    *cap = std::max(0, r->stackNeed - r->ldsStack);
+    *cap = r->stackNeed > r->ldsStack ? r->stackNeed : 0;
     const size_t bytes = (size_t)grid * kTraceThreads * std::max(*cap, 1) * sizeof(int);
     if (r->pp->spill.bytes < bytes) r->pp->spill.alloc(bytes);
     return r->pp->spill.as<int>();
