@@ -60,6 +60,11 @@ enum {
     S_COUNT = S_TRACE + 6
 };
 
+// Counters of chunks whose paths are traced whole (k_paths): per segment four fields (rays, shadow
+// rays, radiance additions of vertices and of shadow rays) of kMaxBounces ints.
+static constexpr int kPathSegs = 16;
+static constexpr int kPathCounters = 4 * kMaxBounces;
+
 static constexpr int kTraceThreads = 128;
 // Default path-pool capacity: 2^26 paths (about 13 GB of SoA path state), a whole 1024^2 x
 // 64 spp pass in one chunk, so that every bounce's queues stay long.
@@ -1133,6 +1138,59 @@ __device__ __forceinline__ float mixturePdf(const GuideRec &g, f3 w) {
     return q;
 }
 
+// Radiance a ray brings from the environment.  A camera miss and one whose vertex sampled no
+// light take it as is (environment_light.h:68-83); others weight it against the light sample
+// (sampler.h:127-140: the environment's share of the light selection).
+__device__ __forceinline__ f3 missRadiance(const PtSceneView &lv, int nee, int depth, float prevPdf, f3 thr, f3 d) {
+    if (depth == 0 || !nee || prevPdf < 0.f || !lv.env.present) return thr * envEmit(lv.env, d);
+    float pe;
+    const f3 e = envEmitPdf(lv.env, d, &pe);
+    return thr * e * balance(prevPdf, pe * frcp((float)(lv.numEmitters + 1)));
+}
+
+// Radiance a surface point sends back along the ray that found it (lambertian.cu:5-11: emission
+// seen from the front only).
+__device__ __forceinline__ f3 surfaceRadiance(const PtSceneView &lv, int nee, int depth, float prevPdf, f3 thr, f3 o, const SurfacePoint &sp, f3 wo,
+                                              const PtMaterial &m, int type) {
+    if (!(type == PT_MAT_LAMBERTIAN && wo.z >= 0.f && (m.b.x != 0.f || m.b.y != 0.f || m.b.z != 0.f))) return mk(0.f);
+    const f3 e = mk(m.b.x, m.b.y, m.b.z);
+    if (depth == 0 || !nee || prevPdf < 0.f) return thr * e;
+    return thr * e * balance(prevPdf, pdfSceneLight(lv, o, sp));
+}
+
+// The light sample of a vertex (directSampleLights, path_tracer.cu:83-126): true when a shadow ray
+// is to be traced, with its contribution.  pdfOf(wi): the density of the direction sampling
+// technique at a local direction and its world one.  A scene without lights draws the three
+// uniforms and adds nothing.
+template <class PdfOf>
+__device__ __forceinline__ bool lightSample(const PtSceneView &lv, Rng &rng, const SurfacePoint &sp, const Frame &fr, f3 wo, const PtMaterial &m, f3 thr,
+                                            PdfOf pdfOf, LightSample *ls, f3 *contrib) {
+    const float l1 = rng.uniform(), l2 = rng.uniform(), l3 = rng.uniform();
+    const bool anyLight = lv.numEmitters > 0 || lv.env.present;
+    if (anyLight) *ls = sampleLights(lv, sp.p, l1, l2, l3);
+    if (!(anyLight && dot(ls->n, ls->wi) < 0.f && ls->pdf > 0.f)) return false;
+    const f3 wiL = toLocal(fr, ls->wi);
+    const float w = balance(ls->pdf, pdfOf(wiL, ls->wi));
+    *contrib = thr * (ls->emitted * w * bsdfF(m, wo, wiL) * (fabsf(dot(sp.n, ls->wi)) * frcp(ls->pdf)));
+    return !isZero(*contrib) && !(contrib->x != contrib->x);
+}
+
+// The direction a vertex samples from its BSDF.
+__device__ __forceinline__ BsdfSample sampleDirection(const PtMaterial &m, int type, f3 wo, Rng &rng) {
+    const int dims = bsdfDims(type);
+    const float x1 = dims >= 1 ? rng.uniform() : 0.f;
+    const float x2 = dims >= 2 ? rng.uniform() : 0.f;
+    return bsdfSample(m, wo, x1, x2);
+}
+
+// Throughput along a sampled direction; false when the path ends there.
+__device__ __forceinline__ bool continuePath(const BsdfSample &bs, f3 thr, f3 *nb) {
+    *nb = mk(0.f);
+    if (isZero(bs.f) || !(bs.pdf > 0.f)) return false;
+    *nb = thr * (bs.f * (fabsf(bs.wi.z) * frcp(bs.pdf)));
+    return !isZero(*nb) && nb->x == nb->x;
+}
+
 // One path vertex per lane.  Plain (GUIDED = false): the reference's NEE + MIS estimator
 // (path_tracer.cu:142-184) with the BSDF-sampled emitter term folded into the next vertex's
 // emission, or the naive estimator (:186-233).  Guided: at Lambert and Beckmann vertices the
@@ -1270,27 +1328,14 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
             }
             const int slot = asInt(h.w);
             if (slot == INT32_MIN) {
-                // miss: environment (camera miss: environment_light.h:68-83 as is)
-                if (depth == 0 || !cp.nee || prevPdf < 0.f || !lv.env.present) {
-                    L = thr * envEmit(lv.env, d);
-                } else {
-                    // sampler.h:127-140: light-selection share of the environment density
-                    float pe;
-                    const f3 e = envEmitPdf(lv.env, d, &pe);
-                    L = thr * e * balance(prevPdf, pe * frcp((float)(lv.numEmitters + 1)));
-                }
+                L = missRadiance(lv, cp.nee, depth, prevPdf, thr, d);
             } else {
                 const SurfacePoint sp = surfaceAt(lv, slot, o, d, h.x, h.y, h.z);
                 const Frame fr = makeFrame(sp.n);
                 const f3 wo = normalize(toLocal(fr, -d));
                 const PtMaterial m = lv.materials[sp.mat];
                 const int type = matType(m);
-                // lambertian.cu:5-11: emission seen from the front only
-                if (type == PT_MAT_LAMBERTIAN && wo.z >= 0.f && (m.b.x != 0.f || m.b.y != 0.f || m.b.z != 0.f)) {
-                    const f3 e = mk(m.b.x, m.b.y, m.b.z);
-                    if (depth == 0 || !cp.nee || prevPdf < 0.f) L = thr * e;
-                    else L = thr * e * balance(prevPdf, pdfSceneLight(lv, o, sp));
-                }
+                L = surfaceRadiance(lv, cp.nee, depth, prevPdf, thr, o, sp, wo, m, type);
                 if (depth + 1 < maxDepth) {
                     Rng rng;
                     if constexpr (BATCH) {
@@ -1342,48 +1387,31 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
                             bs.f = bsdfF(m, wo, bs.wi);
                             bs.delta = false;
                         } else {
-                            const int dims = bsdfDims(type);
-                            const float x1 = dims >= 1 ? rng.uniform() : 0.f;
-                            const float x2 = dims >= 2 ? rng.uniform() : 0.f;
-                            bs = bsdfSample(m, wo, x1, x2);
+                            bs = sampleDirection(m, type, wo, rng);
                         }
                         pbRec = bsdfSamplePdf(m, wo, bs.wi);
                         pdfDir = frac * mixturePdf(G, toWorld(fr, bs.wi)) + (1.f - frac) * pbRec;
                         bs.pdf = pdfDir;
                     } else {
-                        const int dims = bsdfDims(type);
-                        const float x1 = dims >= 1 ? rng.uniform() : 0.f;
-                        const float x2 = dims >= 2 ? rng.uniform() : 0.f;
-                        bs = bsdfSample(m, wo, x1, x2);
+                        bs = sampleDirection(m, type, wo, rng);
                         pdfDir = bs.pdf;
                     }
                     // the continuation's queue slot is claimed here and used after the light
                     // sample, whose work hides the atomic's round trip
-                    bool pushRay = false;
-                    f3 nb = mk(0.f);
-                    if (!isZero(bs.f) && bs.pdf > 0.f) {
-                        nb = thr * (bs.f * (fabsf(bs.wi.z) * frcp(bs.pdf)));
-                        pushRay = !isZero(nb) && nb.x == nb.x;
-                    }
+                    f3 nb;
+                    const bool pushRay = continuePath(bs, thr, &nb);
                     const PendingAppend rayAppend = segAppendIssue(pushRay, counters, seg, bounce + 1, PT_Q_RAYS);
                     bool pushShadow = false;
                     f3 contrib = mk(0.f);
                     LightSample ls;
                     if (cp.nee && !bs.delta) {
-                        // directSampleLights (path_tracer.cu:83-126); a scene without lights
-                        // draws the three uniforms and adds nothing
-                        const float l1 = rng.uniform(), l2 = rng.uniform(), l3 = rng.uniform();
-                        const bool anyLight = lv.numEmitters > 0 || lv.env.present;
-                        if (anyLight) ls = sampleLights(lv, sp.p, l1, l2, l3);
-                        if (anyLight && dot(ls.n, ls.wi) < 0.f && ls.pdf > 0.f) {
-                            const f3 wiL = toLocal(fr, ls.wi);
-                            float pB;
-                            if (GUIDED && guidedV) pB = frac * mixturePdf(G, ls.wi) + (1.f - frac) * bsdfSamplePdf(m, wo, wiL);
-                            else pB = cp.misSample ? bsdfSamplePdf(m, wo, wiL) : bsdfPdf(m, wo, wiL);
-                            const float w = balance(ls.pdf, pB);
-                            contrib = thr * (ls.emitted * w * bsdfF(m, wo, wiL) * (fabsf(dot(sp.n, ls.wi)) * frcp(ls.pdf)));
-                            pushShadow = !isZero(contrib) && !(contrib.x != contrib.x);
-                        }
+                        pushShadow = lightSample(
+                            lv, rng, sp, fr, wo, m, thr,
+                            [&](f3 wiL, f3 wi) {
+                                if (GUIDED && guidedV) return frac * mixturePdf(G, wi) + (1.f - frac) * bsdfSamplePdf(m, wo, wiL);
+                                return cp.misSample ? bsdfSamplePdf(m, wo, wiL) : bsdfPdf(m, wo, wiL);
+                            },
+                            &ls, &contrib);
                     }
                     const PendingAppend shadowAppend = segAppendIssue(pushShadow, counters, seg, bounce, PT_Q_SHADOW);
                     spawned += (pushShadow ? 1 : 0) + (pushRay ? 1 : 0);
@@ -1441,6 +1469,113 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
     waveSum(adds, &counters[ptQueueField(homeSegment(), bounce, PT_Q_LADD_SHADE)]);
 }
 
+// Traces every active lane's ray to its end (lanes of a wave that wait for the longest ray idle:
+// nothing refills them here).
+template <bool ANY, int STACK>
+__device__ __forceinline__ void traceLanes(const PtSceneView &sc, LaneRay &r, bool active, f3 o, f3 d, float tmin, float tmax, const TraceStack &ts,
+                                           int *overflow) {
+    r.prim = INT32_MIN;
+    bool busy = active && sc.numNodes > 0;
+    if (busy) {
+        laneRayStart(r, o, d, tmin, tmax);
+        stackStart<STACK>(r, ts);
+    }
+    while (__ballot(busy) != 0)
+        if (busy) busy = !traceRound<ANY, STACK>(sc, r, ts, overflow);
+}
+
+// A small chunk's paths from the camera to their end in one launch: a wave takes 64 paths and
+// alternates between tracing its lanes' rays, shading their hits and tracing their shadow rays,
+// with the path state in registers.  The arithmetic is the queue kernels' own, step by step, so a
+// path's radiance is theirs bit for bit.
+//
+// The queue kernels need their queues long: each launch lasts at least as long as its longest ray
+// takes alone (40-70 us in a mesh) plus its start, three of them per bounce, however few rays are
+// left.  Here the longest paths overlap all other work.  Against that, lanes whose path has ended
+// stay idle and a wave waits for its longest ray at every bounce, which costs more than the
+// launches once the chip is full several times over: see wholePaths.  Taking new paths into idle
+// lanes between bounces did not help (2048x1024 of 327k triangles 1603 -> 1693 us: the lanes'
+// different depths spilled more state than they filled idle time).
+static constexpr int kPathBlocksPerCU = 8;   // of two waves: four waves per SIMD
+template <int STACK>
+__global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, float4 *Lpath, int *pathCounters, int *spill,
+                                                           int spillCap, int *overflow) {
+    __shared__ int sstack[stackRows(STACK) * kTraceThreads];
+    const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
+    const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), waves = (int)((gridDim.x * blockDim.x) >> 6);
+    int *count = pathCounters + (wave % kPathSegs) * kPathCounters;
+    auto tally = [&](int field, int bounce, bool mine) {
+        const int n = __popcll(__ballot(mine));
+        if (n > 0 && laneId() == 0) atomicAdd(&count[field * kMaxBounces + bounce], n);
+    };
+    for (int run = wave; run < (cp.nPaths + 63) / 64; run += waves) {
+        const int path = run * 64 + laneId();
+        bool alive = path < cp.nPaths;
+        int s, col;
+        const int pixel = cp.pixBegin + chunkPixelOf(cp, alive ? path : 0, &s);
+        const int row = divmodEst(pixel, cp.W, &col);
+        Rng rng = seedRng(cp.seed, (uint32_t)pixel, (uint32_t)(cp.sampleBase + s));
+        const float jx = rng.uniform(), jy = rng.uniform();
+        f3 o, d;
+        cameraRay(cam, row, col, jx, jy, &o, &d);
+        f3 thr = mk(1.f), acc = mk(0.f);
+        float prevPdf = -1.f;
+        for (int depth = 0; depth < cp.maxDepth && __ballot(alive) != 0; depth++) {
+            tally(0, depth, alive);
+            LaneRay r;
+            traceLanes<false, STACK>(sc, r, alive, o, d, depth == 0 ? 0.f : kBounceEps, FLT_MAX, ts, overflow);
+            bool addL = false, pushRay = false, pushShadow = false;
+            f3 p = mk(0.f), contrib = mk(0.f), lightDir = mk(0.f), next = mk(0.f), nb = mk(0.f);
+            float lightDist = 0.f, nextPdf = -1.f;
+            if (alive) {
+                f3 L;
+                if (r.prim == INT32_MIN) {
+                    L = missRadiance(sc, cp.nee, depth, prevPdf, thr, d);
+                } else {
+                    const TraceHit h = laneRayHit(r);
+                    const SurfacePoint sp = surfaceAt(sc, h.prim, o, d, h.t, h.u, h.v);
+                    const Frame fr = makeFrame(sp.n);
+                    const f3 wo = normalize(toLocal(fr, -d));
+                    const PtMaterial m = sc.materials[sp.mat];
+                    const int type = matType(m);
+                    L = surfaceRadiance(sc, cp.nee, depth, prevPdf, thr, o, sp, wo, m, type);
+                    if (depth + 1 < cp.maxDepth) {
+                        const BsdfSample bs = sampleDirection(m, type, wo, rng);
+                        pushRay = continuePath(bs, thr, &nb);
+                        nextPdf = bs.delta ? -1.f : bs.pdf;
+                        if (cp.nee && !bs.delta) {
+                            LightSample ls;
+                            pushShadow = lightSample(
+                                sc, rng, sp, fr, wo, m, thr, [&](f3 wiL, f3) { return cp.misSample ? bsdfSamplePdf(m, wo, wiL) : bsdfPdf(m, wo, wiL); }, &ls,
+                                &contrib);
+                            lightDir = ls.wi;
+                            lightDist = ls.dist;
+                        }
+                        p = sp.p;
+                        next = toWorld(fr, bs.wi);
+                    }
+                }
+                addL = !isZero(L);
+                if (depth == 0 || addL) acc = acc + L;
+            }
+            tally(2, depth, addL);
+            if (cp.nee) {
+                tally(1, depth, pushShadow);
+                traceLanes<true, STACK>(sc, r, pushShadow, p, lightDir, kShadowEps, lightDist - 2e-4f, ts, overflow);
+                const bool lit = pushShadow && r.prim == INT32_MIN;
+                if (lit) acc = acc + contrib;
+                tally(3, depth, lit);
+            }
+            alive = pushRay;
+            o = p;
+            d = next;
+            thr = nb;
+            prevPdf = nextPdf;
+        }
+        if (path < cp.nPaths) Lpath[path] = f4(acc, 0.f);
+    }
+}
+
 // Training targets: weight = (radiance after the vertex's sampled direction) / luminance of the
 // throughput at the vertex, i.e. the MC estimate of f cos L_i / p for the sampled direction.
 // Records live in per-segment parts of recSeg entries; block 0 also writes the exclusive prefix
@@ -1482,28 +1617,58 @@ __global__ __launch_bounds__(256) void k_guide_finalize(float4 *records, int rec
     }
 }
 
+// What a chunk's accumulation does beside adding to the FP64 sums.
+struct PassEnd {
+    int fresh = 0;                // 1: the accumulator starts from zero here (it holds an older image)
+    float *radiance = nullptr;    // the pass's last chunk: the framebuffers (nullptr: not yet)
+    uchar4 *rgba = nullptr;
+    double invSpp = 0.0;
+};
+
+// mean radiance + the uchar4 framebuffer of framebuffer.cu:35-40 (color.h:7-28 sRGB)
+__device__ __forceinline__ void writePixel(const double a[3], double invSpp, int p, float *radiance, uchar4 *rgba) {
+    unsigned char o[3];
+    for (int k = 0; k < 3; k++) {
+        const float v = (float)(a[k] * invSpp);
+        radiance[3 * (size_t)p + k] = v;
+        o[k] = srgbByte(v);
+    }
+    rgba[p] = make_uchar4(o[0], o[1], o[2], 255);
+}
+
 // Per pixel of the chunk: FP64 sum over the chunk's sample rows (framebuffer.cu:7-41 keeps a
-// running FP32 mean instead).  Block 0 also folds the chunk's queue counters into the stats.
-__global__ __launch_bounds__(256) void k_accumulate(ChunkParams cp, const float4 *Lpath, double *accum, const int *counters, unsigned long long *stats) {
+// running FP32 mean instead), and at the end of a pass the framebuffers from the sums just made.
+// Block 0 also folds the chunk's counters into the stats: the queues', or those of a chunk traced
+// whole (pathCounters), which it clears for the next.
+__global__ __launch_bounds__(256) void k_accumulate(ChunkParams cp, const float4 *Lpath, double *accum, const int *counters, int *pathCounters,
+                                                    unsigned long long *stats, PassEnd end) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x == 0) {
-        for (int b = threadIdx.x; b < kMaxBounces; b += blockDim.x) {
-            unsigned long long v[4] = {0, 0, 0, 0};
-            for (int seg = 0; seg < PT_QUEUE_SEGS; seg++) {
-                v[0] += (unsigned long long)counters[ptQueueField(seg, b, PT_Q_RAYS)];
-                v[1] += (unsigned long long)counters[ptQueueField(seg, b, PT_Q_SHADOW)];
-                v[2] += (unsigned long long)counters[ptQueueField(seg, b, PT_Q_LADD_SHADE)];
-                v[3] += (unsigned long long)counters[ptQueueField(seg, b, PT_Q_LADD_SHADOW)];
+        constexpr int kStat[4] = {S_RAYS, S_SHADOW, S_LADD_SHADE, S_LADD_SHADOW};
+        if (pathCounters) {
+            // a thread per counter: field, then bounce
+            for (int k = threadIdx.x; k < kPathCounters; k += blockDim.x) {
+                unsigned long long v = 0;
+                for (int seg = 0; seg < kPathSegs; seg++) {
+                    v += (unsigned long long)pathCounters[seg * kPathCounters + k];
+                    pathCounters[seg * kPathCounters + k] = 0;
+                }
+                if (v) atomicAdd(&stats[kStat[k / kMaxBounces] + k % kMaxBounces], v);
             }
-            atomicAdd(&stats[S_RAYS + b], v[0]);
-            atomicAdd(&stats[S_SHADOW + b], v[1]);
-            atomicAdd(&stats[S_LADD_SHADE + b], v[2]);
-            atomicAdd(&stats[S_LADD_SHADOW + b], v[3]);
+        } else {
+            for (int b = threadIdx.x; b < kMaxBounces; b += blockDim.x) {
+                constexpr int kField[4] = {PT_Q_RAYS, PT_Q_SHADOW, PT_Q_LADD_SHADE, PT_Q_LADD_SHADOW};
+                for (int f = 0; f < 4; f++) {
+                    unsigned long long v = 0;
+                    for (int seg = 0; seg < PT_QUEUE_SEGS; seg++) v += (unsigned long long)counters[ptQueueField(seg, b, kField[f])];
+                    if (v) atomicAdd(&stats[kStat[f] + b], v);
+                }
+            }
         }
         if (threadIdx.x == 0) atomicAdd(&stats[S_PATHS], (unsigned long long)cp.nPaths);
     }
     double sx = 0.0, sy = 0.0, sz = 0.0;
-    if (cp.pixelMajor) {
+    if (cp.pixelMajor && cp.samples > 1) {
         // A pixel's samples are contiguous: the block's 256 pixels are read in tiles of
         // kAccTile samples per pixel (each pixel's run of records loaded by neighbouring
         // lanes) into LDS, and each thread sums its pixel's samples in sample order, the same
@@ -1533,9 +1698,7 @@ __global__ __launch_bounds__(256) void k_accumulate(ChunkParams cp, const float4
             }
             __syncthreads();
         }
-        if (p >= cp.npix) return;
-    } else {
-        if (p >= cp.npix) return;
+    } else if (p < cp.npix) {
         for (int s = 0; s < cp.samples; s++) {
             const float4 l = Lpath[(size_t)s * cp.npix + p];
             sx += (double)l.x;
@@ -1543,10 +1706,16 @@ __global__ __launch_bounds__(256) void k_accumulate(ChunkParams cp, const float4
             sz += (double)l.z;
         }
     }
+    if (p >= cp.npix) return;
     double *a = accum + 3 * (size_t)(cp.pixBegin + p);
-    a[0] += sx;
-    a[1] += sy;
-    a[2] += sz;
+    double v[3] = {0.0, 0.0, 0.0};
+    if (!end.fresh)
+        for (int k = 0; k < 3; k++) v[k] = a[k];
+    v[0] += sx;
+    v[1] += sy;
+    v[2] += sz;
+    for (int k = 0; k < 3; k++) a[k] = v[k];
+    if (end.radiance) writePixel(v, end.invSpp, cp.pixBegin + p, end.radiance, end.rgba);
 }
 
 // Batch wavefront: per (group, pixel) of the chunk, the FP64 sum over the group's sample rows
@@ -1648,17 +1817,9 @@ __global__ void k_rebase_prims(float4 *recs, int count, int matOff, int normOff)
     if (tag >= 0) p1.w = asFloat(tag + normOff);
 }
 
-// mean radiance + the uchar4 framebuffer of framebuffer.cu:35-40 (color.h:7-28 sRGB)
 __global__ __launch_bounds__(256) void k_tonemap(const double *accum, int npix, double invSpp, float *radiance, uchar4 *rgba) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npix) return;
-    unsigned char o[3];
-    for (int k = 0; k < 3; k++) {
-        const float v = (float)(accum[3 * (size_t)p + k] * invSpp);
-        radiance[3 * (size_t)p + k] = v;
-        o[k] = srgbByte(v);
-    }
-    rgba[p] = make_uchar4(o[0], o[1], o[2], 255);
+    if (p < npix) writePixel(accum + 3 * (size_t)p, invSpp, p, radiance, rgba);
 }
 
 // Normals view (g_buffer.cu:27-57): colour (n + 1) / 2 of the primary hit at the pixel centre
@@ -1740,7 +1901,7 @@ const char *kKernelNames[K_NUM] = {"raygen", "extend", "shade", "shadow", "accum
 // SoA path state, traversal stack spill area and queue counters of up to `pool` paths.
 struct PathPool {
     int64_t pool = 0;
-    DevBuf rayO[2], rayD[2], st[2], beta[2], hits, sO, sD, sL, Lpath, counters, overflow, spill;
+    DevBuf rayO[2], rayD[2], st[2], beta[2], hits, sO, sD, sL, Lpath, counters, pathCounters, overflow, spill;
 };
 
 struct pt_renderer {
@@ -2034,9 +2195,41 @@ GuideSceneNorm guideNorm(pt_renderer *r) {
     return nm;
 }
 
-void runChunk(pt_renderer *r, const ChunkParams &cp) {
+// Whether a chunk's paths are traced whole (k_paths) or through the queues.  us a pass, queues /
+// whole: 256^2 pixels of 327k triangles 847 / 323, of the Cornell box 361 / 97, 1 sample each;
+// 2^20 paths: Cornell box 728 / 415, 5k triangles 775 / 464, 1.31M triangles 1816 / 1154, room of
+// 1M at depth 16 6534 / 5473; 2^21 paths: 5k triangles 936 / 821, 1.31M at depth 4 1931 / 1990,
+// room of 1M at depth 16 9526 / 10978; 2^23 paths: Cornell box 3727 / 2761, 17 nodes 1606 / 1401,
+// 304 nodes 2122 / 2106, 1229 nodes 2483 / 2710.  The timed and the counting kernels are the
+// queues', and so are a batch's: its chunks are filled with paths of several renders.
+bool wholePaths(const pt_renderer *r, const ChunkParams &cp) {
+    if (r->type == PT_RENDERER_GUIDED || r->profile || r->traceStats || !r->ownsStream) return false;
+    const int nodes = r->view.numNodes;
+    return cp.nPaths <= (nodes <= 16 ? 1 << 23 : nodes <= 4096 ? 1 << 21 : 1 << 20);
+}
+
+void accumulateChunk(pt_renderer *r, const ChunkParams &cp, bool whole, const PassEnd &end) {
+    KTimer t(r, K_ACCUM);
+    k_accumulate<<<(cp.npix + 255) / 256, 256, 0, r->stream>>>(cp, r->pp->Lpath.as<float4>(), r->accum.as<double>(), r->pp->counters.as<int>(),
+                                                              whole ? r->pp->pathCounters.as<int>() : nullptr, r->stats.as<unsigned long long>(), end);
+    PT_HIP_TRY(hipGetLastError());
+}
+
+void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEnd{}) {
     int *ctr = r->pp->counters.as<int>();
     const bool guided = r->type == PT_RENDERER_GUIDED;
+    if (wholePaths(r, cp)) {
+        const int grid = std::min((cp.nPaths + kTraceThreads - 1) / kTraceThreads, r->cus * kPathBlocksPerCU);
+        int cap = 0;
+        int *sp = ensureSpill(r, grid, &cap);
+        float4 *L = r->pp->Lpath.as<float4>();
+        int *pc = r->pp->pathCounters.as<int>(), *ov = r->pp->overflow.as<int>();
+        if (r->ldsStack == 32) k_paths<32><<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, L, pc, sp, cap, ov);
+        else k_paths<16><<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, L, pc, sp, cap, ov);
+        PT_HIP_TRY(hipGetLastError());
+        accumulateChunk(r, cp, true, end);
+        return;
+    }
     {
         KTimer t(r, K_RAYGEN);
         k_queue_reset<<<PT_QUEUE_SEGS + 1, 256, 0, r->stream>>>(ctr, PT_Q_RAYS, cp.nPaths, cp.segLen, 1);
@@ -2105,12 +2298,7 @@ void runChunk(pt_renderer *r, const ChunkParams &cp) {
         }
         cur = 1 - cur;
     }
-    {
-        KTimer t(r, K_ACCUM);
-        k_accumulate<<<(cp.npix + 255) / 256, 256, 0, r->stream>>>(cp, r->pp->Lpath.as<float4>(), r->accum.as<double>(), ctr,
-                                                                  r->stats.as<unsigned long long>());
-        PT_HIP_TRY(hipGetLastError());
-    }
+    accumulateChunk(r, cp, false, end);
     if (guided && r->gTrainSteps > 0) {
         KTimer t(r, K_GUIDE_TRAIN);
         const int nrec = (int)r->gRecCap;
@@ -2244,6 +2432,8 @@ int pt_renderer_create(int width, int height, pt_renderer **out) {
     r->pp->counters.alloc(kNumCounters * sizeof(int));
     r->pp->overflow.alloc(sizeof(int));
     PT_HIP_TRY(hipMemsetAsync(r->pp->overflow.p, 0, sizeof(int), r->stream));
+    r->pp->pathCounters.alloc(kPathSegs * kPathCounters * sizeof(int));
+    PT_HIP_TRY(hipMemsetAsync(r->pp->pathCounters.p, 0, kPathSegs * kPathCounters * sizeof(int), r->stream));
     k_zero_u64<<<1, 512, 0, r->stream>>>(r->stats.as<unsigned long long>(), S_COUNT);
     zeroAccum(r);
     computeCamera(r);
@@ -2492,9 +2682,20 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
     if (r->inFlight) return fail(PT_ERR_STATE, "pt_renderer_render_async: previous pass not polled");
     if (spp <= 0) return fail(PT_ERR_INVALID, "pt_renderer_render_async: spp must be positive");
     PT_API_BEGIN
-    if (r->resetPending) zeroAccum(r);
-    PT_HIP_TRY(hipEventRecord(r->evBegin, r->stream));
     const int npix = r->W * r->H;
+    // a new image: its first chunk writes the accumulator instead of adding to it where that
+    // chunk covers every pixel
+    bool fresh = r->resetPending;
+    if (fresh && r->type == PT_RENDERER_NORMALS) {
+        zeroAccum(r);
+        fresh = false;
+    }
+    if (fresh) {
+        r->spp = 0;
+        r->resetPending = false;
+    }
+    PT_HIP_TRY(hipEventRecord(r->evBegin, r->stream));
+    bool toned = false;
     r->lastChunks.clear();
     if (r->type == PT_RENDERER_NORMALS) {
         // one centre ray per pixel, added once per pass (the reference's framebuffer sees
@@ -2513,9 +2714,23 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
         ensurePool(r, (int64_t)npix * spp);
         if (r->type == PT_RENDERER_GUIDED) ensureGuide(r);
         planChunks(r, spp, r->lastChunks);
+        if (fresh && (r->maxDepth <= 0 || r->lastChunks[0].npix != npix)) {
+            zeroAccum(r);
+            fresh = false;
+        }
         if (r->maxDepth > 0) {
             for (const ChunkParams &cp : r->lastChunks) {
-                runChunk(r, cp);
+                PassEnd end;
+                end.fresh = fresh ? 1 : 0;
+                fresh = false;
+                // the pass's framebuffers with its last sums, unless the kernels are timed apart
+                if (&cp == &r->lastChunks.back() && cp.npix == npix && !r->profile) {
+                    end.radiance = r->radiance.as<float>();
+                    end.rgba = r->rgba.as<uchar4>();
+                    end.invSpp = 1.0 / (double)(r->spp + spp);
+                    toned = true;
+                }
+                runChunk(r, cp, end);
                 r->pixelsAccumulated += cp.npix;
                 r->samplesAccumulated += (double)cp.npix * cp.samples;
             }
@@ -2527,7 +2742,7 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
     r->lastPassSingleChunk = r->lastChunks.size() == 1;
     r->lastPassSamples = r->lastChunks.empty() ? 0 : r->lastChunks[0].samples;
     r->lastPassPixelMajor = !r->lastChunks.empty() && r->lastChunks[0].pixelMajor;
-    tonemap(r);
+    if (!toned) tonemap(r);
     PT_HIP_TRY(hipEventRecord(r->evEnd, r->stream));
     r->inFlight = true;
     return PT_OK;
@@ -3035,7 +3250,7 @@ void prepareBatch(pt_batch *b, int scale) {
     }
     ensurePool(b->jobs[0], need);
     int cap = 0;
-    ensureSpill(b->jobs[deepest], b->jobs[0]->cus * b->cfg.trace, &cap);
+    ensureSpill(b->jobs[deepest], traceGrid(b->jobs[deepest]), &cap);
     b->stamps.alloc((b->jobs.size() + 1) * sizeof(unsigned long long));
     b->order.resize(b->jobs.size());
     for (size_t j = 0; j < b->jobs.size(); j++) b->order[j] = (int)j;
@@ -3453,6 +3668,8 @@ int pt_batch_create(pt_batch **out) {
     b->pp->counters.alloc(kNumCounters * sizeof(int));
     b->pp->overflow.alloc(sizeof(int));
     PT_HIP_TRY(hipMemsetAsync(b->pp->overflow.p, 0, sizeof(int), b->stream));
+    b->pp->pathCounters.alloc(kPathSegs * kPathCounters * sizeof(int));
+    PT_HIP_TRY(hipMemsetAsync(b->pp->pathCounters.p, 0, kPathSegs * kPathCounters * sizeof(int), b->stream));
     int dev = 0, khz = 0;
     PT_HIP_TRY(hipGetDevice(&dev));
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0) b->clockKHz = khz;
