@@ -71,6 +71,21 @@ struct WorkArrays {
     }
 };
 
+// Copies device memory to pageable host memory behind the stream's work and waits for it: through
+// pinned staging memory, a piece copied out by the CPU while the next ones are on the link.
+void readToHost(void *dst, const void *src, size_t bytes, hipStream_t stream);
+
+// An int of pinned host memory that kernels can write, from a page shared by the process's
+// objects (pinning memory for each costs 100 us); null when the page is used up.
+class HostWord {
+public:
+    HostWord();
+    ~HostWord();
+    HostWord(const HostWord &) = delete;
+    HostWord &operator=(const HostWord &) = delete;
+    int *p = nullptr;
+};
+
 struct BvhInfo {
     int numNodes = 0;      // 4-wide nodes
     int depth = 0;         // levels of 4-wide nodes

@@ -1623,6 +1623,8 @@ struct PassEnd {
     float *radiance = nullptr;    // the pass's last chunk: the framebuffers (nullptr: not yet)
     uchar4 *rgba = nullptr;
     double invSpp = 0.0;
+    const int *overflow = nullptr;   // the pass's last kernel: traversal overflows so far,
+    int *overflowSeen = nullptr;     // and where the host reads them
 };
 
 // mean radiance + the uchar4 framebuffer of framebuffer.cu:35-40 (color.h:7-28 sRGB)
@@ -1716,6 +1718,7 @@ __global__ __launch_bounds__(256) void k_accumulate(ChunkParams cp, const float4
     v[2] += sz;
     for (int k = 0; k < 3; k++) a[k] = v[k];
     if (end.radiance) writePixel(v, end.invSpp, cp.pixBegin + p, end.radiance, end.rgba);
+    if (end.overflow && p == 0) *end.overflowSeen = *end.overflow;
 }
 
 // Batch wavefront: per (group, pixel) of the chunk, the FP64 sum over the group's sample rows
@@ -1817,9 +1820,10 @@ __global__ void k_rebase_prims(float4 *recs, int count, int matOff, int normOff)
     if (tag >= 0) p1.w = asFloat(tag + normOff);
 }
 
-__global__ __launch_bounds__(256) void k_tonemap(const double *accum, int npix, double invSpp, float *radiance, uchar4 *rgba) {
+__global__ __launch_bounds__(256) void k_tonemap(const double *accum, int npix, PassEnd end) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < npix) writePixel(accum + 3 * (size_t)p, invSpp, p, radiance, rgba);
+    if (p < npix) writePixel(accum + 3 * (size_t)p, end.invSpp, p, end.radiance, end.rgba);
+    if (end.overflow && p == 0) *end.overflowSeen = *end.overflow;
 }
 
 // Normals view (g_buffer.cu:27-57): colour (n + 1) / 2 of the primary hit at the pixel centre
@@ -1933,6 +1937,10 @@ struct pt_renderer {
     int traceBlocksPerCU = kDefaultTraceBlocks, shadeBlocksPerCU = 8;
     // accumulation
     DevBuf accum, radiance, rgba, stats;
+    // the traversal's overflow count as of the last pass, written by its last kernel; stale after
+    // traversals outside a pass
+    std::unique_ptr<HostWord> overflowSeen;
+    bool overflowStale = true;
     int64_t spp = 0;
     bool resetPending = false;
     // pass tracking
@@ -2356,11 +2364,24 @@ void planChunks(const pt_renderer *r, int spp, std::vector<ChunkParams> &out) {
     }
 }
 
+// The framebuffers and the overflow count, written by a pass's last kernel.
+PassEnd passEnd(pt_renderer *r, double invSpp) {
+    PassEnd end;
+    end.radiance = r->radiance.as<float>();
+    end.rgba = r->rgba.as<uchar4>();
+    end.invSpp = invSpp;
+    if (r->overflowSeen && r->overflowSeen->p) {
+        end.overflow = r->pp->overflow.as<int>();
+        end.overflowSeen = r->overflowSeen->p;
+    }
+    return end;
+}
+
 void tonemap(pt_renderer *r) {
     KTimer t(r, K_TONEMAP);
     const int npix = r->W * r->H;
     const double inv = r->spp > 0 ? 1.0 / (double)r->spp : 0.0;
-    k_tonemap<<<(npix + 255) / 256, 256, 0, r->stream>>>(r->accum.as<double>(), npix, inv, r->radiance.as<float>(), r->rgba.as<uchar4>());
+    k_tonemap<<<(npix + 255) / 256, 256, 0, r->stream>>>(r->accum.as<double>(), npix, passEnd(r, inv));
     PT_HIP_TRY(hipGetLastError());
 }
 
@@ -2429,6 +2450,7 @@ int pt_renderer_create(int width, int height, pt_renderer **out) {
     r->radiance.alloc(npix * 3 * sizeof(float));
     r->rgba.alloc(npix * 4);
     r->stats.alloc(S_COUNT * sizeof(unsigned long long));
+    r->overflowSeen = std::make_unique<HostWord>();
     r->pp->counters.alloc(kNumCounters * sizeof(int));
     r->pp->overflow.alloc(sizeof(int));
     PT_HIP_TRY(hipMemsetAsync(r->pp->overflow.p, 0, sizeof(int), r->stream));
@@ -2720,16 +2742,12 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
         }
         if (r->maxDepth > 0) {
             for (const ChunkParams &cp : r->lastChunks) {
+                // the pass's framebuffers with its last sums, unless the kernels are timed apart
                 PassEnd end;
+                toned = &cp == &r->lastChunks.back() && cp.npix == npix && !r->profile;
+                if (toned) end = passEnd(r, 1.0 / (double)(r->spp + spp));
                 end.fresh = fresh ? 1 : 0;
                 fresh = false;
-                // the pass's framebuffers with its last sums, unless the kernels are timed apart
-                if (&cp == &r->lastChunks.back() && cp.npix == npix && !r->profile) {
-                    end.radiance = r->radiance.as<float>();
-                    end.rgba = r->rgba.as<uchar4>();
-                    end.invSpp = 1.0 / (double)(r->spp + spp);
-                    toned = true;
-                }
                 runChunk(r, cp, end);
                 r->pixelsAccumulated += cp.npix;
                 r->samplesAccumulated += (double)cp.npix * cp.samples;
@@ -2744,6 +2762,7 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
     r->lastPassPixelMajor = !r->lastChunks.empty() && r->lastChunks[0].pixelMajor;
     if (!toned) tonemap(r);
     PT_HIP_TRY(hipEventRecord(r->evEnd, r->stream));
+    r->overflowStale = !r->overflowSeen || !r->overflowSeen->p;
     r->inFlight = true;
     return PT_OK;
     PT_API_END("pt_renderer_render_async")
@@ -2778,7 +2797,8 @@ int pt_renderer_synchronize(pt_renderer *r) {
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
     if (r->inFlight) finishPass(r);
     int ov = 0;
-    PT_HIP_TRY(hipMemcpy(&ov, r->pp->overflow.p, sizeof(int), hipMemcpyDeviceToHost));
+    if (r->overflowStale) PT_HIP_TRY(hipMemcpy(&ov, r->pp->overflow.p, sizeof(int), hipMemcpyDeviceToHost));
+    else ov = *(volatile int *)r->overflowSeen->p;
     if (ov != 0) return fail(PT_ERR_NUMERIC, "pt_renderer_synchronize: traversal stack overflowed");
     return PT_OK;
     PT_API_END("pt_renderer_synchronize")
@@ -2807,7 +2827,7 @@ int pt_renderer_get_radiance(pt_renderer *r, float *out) {
     PT_API_BEGIN
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
     if (r->inFlight) finishPass(r);
-    PT_HIP_TRY(hipMemcpy(out, r->radiance.p, (size_t)r->W * r->H * 3 * sizeof(float), hipMemcpyDeviceToHost));
+    readToHost(out, r->radiance.p, (size_t)r->W * r->H * 3 * sizeof(float), r->stream);
     return PT_OK;
     PT_API_END("pt_renderer_get_radiance")
 }
@@ -2817,7 +2837,7 @@ int pt_renderer_get_radiance_sum(pt_renderer *r, double *out) {
     PT_API_BEGIN
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
     if (r->inFlight) finishPass(r);
-    PT_HIP_TRY(hipMemcpy(out, r->accum.p, (size_t)r->W * r->H * 3 * sizeof(double), hipMemcpyDeviceToHost));
+    readToHost(out, r->accum.p, (size_t)r->W * r->H * 3 * sizeof(double), r->stream);
     return PT_OK;
     PT_API_END("pt_renderer_get_radiance_sum")
 }
@@ -2827,7 +2847,7 @@ int pt_renderer_get_rgba8(pt_renderer *r, uint8_t *out) {
     PT_API_BEGIN
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
     if (r->inFlight) finishPass(r);
-    PT_HIP_TRY(hipMemcpy(out, r->rgba.p, (size_t)r->W * r->H * 4, hipMemcpyDeviceToHost));
+    readToHost(out, r->rgba.p, (size_t)r->W * r->H * 4, r->stream);
     return PT_OK;
     PT_API_END("pt_renderer_get_rgba8")
 }
@@ -2844,6 +2864,7 @@ int pt_renderer_hit_test(pt_renderer *r, int x, int y, int *material_id, int *is
     if (r->inFlight) return fail(PT_ERR_STATE, "pt_renderer_hit_test: a pass is still running");
     PT_API_BEGIN
     ensurePool(r);
+    r->overflowStale = true;
     // one centre ray through the same extend kernel (hit_test.cu:25-47)
     const float4 *dummy = nullptr;
     (void)dummy;
@@ -3052,6 +3073,7 @@ int pt_renderer_intersect(pt_renderer *r, const float *rays, int64_t n, int any_
     if (r->inFlight) return fail(PT_ERR_STATE, "pt_renderer_intersect: a pass is still running");
     PT_API_BEGIN
     ensurePool(r);
+    r->overflowStale = true;
     for (int64_t done = 0; done < n;) {
         const int cnt = (int)std::min<int64_t>(n - done, r->pp->pool);
         std::vector<float4> o(cnt), d(cnt);
@@ -3807,11 +3829,9 @@ int pt_batch_get_radiance(pt_batch *b, int index, float *out) {
     PT_API_BEGIN
     pt_renderer *r = b->jobs[index];
     PT_HIP_TRY(hipStreamSynchronize(b->stream));
-    const size_t n = (size_t)r->W * r->H * 3;
-    std::vector<double> acc(n);
-    PT_HIP_TRY(hipMemcpy(acc.data(), r->accum.p, n * sizeof(double), hipMemcpyDeviceToHost));
-    const double inv = r->spp > 0 ? 1.0 / (double)r->spp : 0.0;
-    for (size_t i = 0; i < n; i++) out[i] = (float)(acc[i] * inv);
+    // the mean radiance of pt_renderer_get_radiance
+    tonemap(r);
+    readToHost(out, r->radiance.p, (size_t)r->W * r->H * 3 * sizeof(float), b->stream);
     return PT_OK;
     PT_API_END("pt_batch_get_radiance")
 }
