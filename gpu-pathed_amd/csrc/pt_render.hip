@@ -528,6 +528,15 @@ struct TraceCount {
     int rays = 0, nodes = 0, prims = 0;
 };
 
+__device__ __forceinline__ void addTraceCount(const TraceCount &tc, unsigned long long *tstat) {
+    int v[3] = {tc.rays, tc.nodes, tc.prims};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        for (int off = 32; off >= 1; off >>= 1) v[k] += __shfl_xor(v[k], off);
+        if (laneId() == 0) atomicAdd(&tstat[k], (unsigned long long)v[k]);
+    }
+}
+
 template <int STACK> __device__ __forceinline__ void stackStart(LaneRay &r, const TraceStack &ts) {
     r.sp = ts.column + kStackFirst * kTraceThreads;
     if (ts.spillCap > 0) ts.column[stackCountRow(STACK) * kTraceThreads] = 0;
@@ -779,14 +788,7 @@ __device__ __forceinline__ void traceQueue(const PtSceneView &sc, int *counters,
             ray = -1;
         }
     }
-    if constexpr (STATS) {
-        int v[3] = {tc.rays, tc.nodes, tc.prims};
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            for (int off = 32; off >= 1; off >>= 1) v[k] += __shfl_xor(v[k], off);
-            if (laneId() == 0) atomicAdd(&tstat[k], (unsigned long long)v[k]);
-        }
-    }
+    if constexpr (STATS) addTraceCount(tc, tstat);
 }
 
 // Persistent closest-hit kernel over the rays of `bounce`.  camO.w != 0: the rays start at
@@ -1471,17 +1473,39 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
 
 // Traces every active lane's ray to its end (lanes of a wave that wait for the longest ray idle:
 // nothing refills them here).
-template <bool ANY, int STACK>
+template <bool ANY, int STACK, bool STATS = false>
 __device__ __forceinline__ void traceLanes(const PtSceneView &sc, LaneRay &r, bool active, f3 o, f3 d, float tmin, float tmax, const TraceStack &ts,
-                                           int *overflow) {
+                                           int *overflow, TraceCount *tc = nullptr) {
     r.prim = INT32_MIN;
     bool busy = active && sc.numNodes > 0;
     if (busy) {
         laneRayStart(r, o, d, tmin, tmax);
         stackStart<STACK>(r, ts);
+        if constexpr (STATS) tc->rays++;
     }
     while (__ballot(busy) != 0)
-        if (busy) busy = !traceRound<ANY, STACK>(sc, r, ts, overflow);
+        if (busy) busy = !traceRound<ANY, STACK, STATS>(sc, r, ts, overflow, tc);
+}
+
+// What a chunk's accumulation does beside adding to the FP64 sums.
+struct PassEnd {
+    int fresh = 0;                // 1: the accumulator starts from zero here (it holds an older image)
+    float *radiance = nullptr;    // the pass's last chunk: the framebuffers (nullptr: not yet)
+    uchar4 *rgba = nullptr;
+    double invSpp = 0.0;
+    const int *overflow = nullptr;   // the pass's last kernel: traversal overflows so far,
+    int *overflowSeen = nullptr;     // and where the host reads them
+};
+
+// mean radiance + the uchar4 framebuffer of framebuffer.cu:35-40 (color.h:7-28 sRGB)
+__device__ __forceinline__ void writePixel(const double a[3], double invSpp, int p, float *radiance, uchar4 *rgba) {
+    unsigned char o[3];
+    for (int k = 0; k < 3; k++) {
+        const float v = (float)(a[k] * invSpp);
+        radiance[3 * (size_t)p + k] = v;
+        o[k] = srgbByte(v);
+    }
+    rgba[p] = make_uchar4(o[0], o[1], o[2], 255);
 }
 
 // A small chunk's paths from the camera to their end in one launch: a wave takes 64 paths and
@@ -1495,7 +1519,8 @@ __device__ __forceinline__ void traceLanes(const PtSceneView &sc, LaneRay &r, bo
 // stay idle and a wave waits for its longest ray at every bounce, which costs more than the
 // launches once the chip is full several times over: see wholePaths.  Taking new paths into idle
 // lanes between bounces did not help (2048x1024 of 327k triangles 1603 -> 1693 us: the lanes'
-// different depths spilled more state than they filled idle time).
+// different depths spilled more state than they filled idle time), nor did 8 x 8 pixel tiles
+// instead of 64 pixels of a row (327k triangles at 1024^2 882 -> 923 us, at 256^2 306 -> 289).
 static constexpr int kPathBlocksPerCU = 8;   // of two waves: four waves per SIMD
 template <int STACK>
 __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, float4 *Lpath, int *pathCounters, int *spill,
@@ -1510,10 +1535,11 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, Chun
     };
     for (int run = wave; run < (cp.nPaths + 63) / 64; run += waves) {
         const int path = run * 64 + laneId();
-        bool alive = path < cp.nPaths;
+        const bool mine = path < cp.nPaths;
         int s, col;
-        const int pixel = cp.pixBegin + chunkPixelOf(cp, alive ? path : 0, &s);
+        const int pixel = cp.pixBegin + chunkPixelOf(cp, mine ? path : 0, &s);
         const int row = divmodEst(pixel, cp.W, &col);
+        bool alive = mine;
         Rng rng = seedRng(cp.seed, (uint32_t)pixel, (uint32_t)(cp.sampleBase + s));
         const float jx = rng.uniform(), jy = rng.uniform();
         f3 o, d;
@@ -1572,8 +1598,64 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, Chun
             thr = nb;
             prevPdf = nextPdf;
         }
-        if (path < cp.nPaths) Lpath[path] = f4(acc, 0.f);
+        if (mine) Lpath[path] = f4(acc, 0.f);
     }
+}
+
+// Normals view (g_buffer.cu:27-57): colour (n + 1) / 2 of the primary hit at the pixel centre, in one
+// launch: ray, traversal, FP64 accumulator and framebuffers.  Bound by the traversal, as k_extend.
+// 1280x720 of 327k triangles: 176 us (201 us with 64 pixels of a row to a wave) against 228 us in
+// the five kernels before.
+template <int STACK, bool STATS>
+__global__ __launch_bounds__(kTraceThreads, 4) void k_normals(PtSceneView sc, PtCamera cam, double *accum, PassEnd end, int *spill,
+                                                             int spillCap, int *overflow, unsigned long long *tstat) {
+    __shared__ int sstack[stackRows(STACK) * kTraceThreads];
+    const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
+    const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), waves = (int)((gridDim.x * blockDim.x) >> 6);
+    TraceCount tc;
+    // a wave takes 8 x 8 pixels, in Morton order: where neighbouring lanes are at the same node, one
+    // L1 access serves four
+    const int tilesX = (cam.W + 7) / 8, tiles = tilesX * ((cam.H + 7) / 8);
+    for (int tile = wave; tile < tiles; tile += waves) {
+        int tx;
+        const int ty = divmodEst(tile, tilesX, &tx), l = laneId();
+        const int col = 8 * tx + ((l & 1) | (l >> 1 & 2) | (l >> 2 & 4)), row = 8 * ty + ((l >> 1 & 1) | (l >> 2 & 2) | (l >> 3 & 4));
+        const bool mine = col < cam.W && row < cam.H;
+        f3 o, d;
+        cameraRay(cam, row, col, 0.5f, 0.5f, &o, &d);
+        LaneRay r;
+        traceLanes<false, STACK, STATS>(sc, r, mine, o, d, 0.f, FLT_MAX, ts, overflow, &tc);
+        if (!mine) continue;
+        f3 c = mk(0.f);
+        if (r.prim != INT32_MIN) {
+            const TraceHit h = laneRayHit(r);
+            const SurfacePoint sp = surfaceAt(sc, h.prim, o, d, h.t, h.u, h.v);
+            c = (sp.n + mk(1.f)) / 2.f;
+        }
+        const int p = row * cam.W + col;
+        double *a = accum + 3 * (size_t)p;
+        double v[3] = {0.0, 0.0, 0.0};
+        if (!end.fresh)
+            for (int k = 0; k < 3; k++) v[k] = a[k];
+        v[0] += c.x;
+        v[1] += c.y;
+        v[2] += c.z;
+        for (int k = 0; k < 3; k++) a[k] = v[k];
+        if (end.radiance) writePixel(v, end.invSpp, p, end.radiance, end.rgba);
+    }
+    if constexpr (STATS) addTraceCount(tc, tstat);
+}
+
+// The material under one camera ray (hit_test.cu:25-47), or -1, straight to where the host reads
+// it: one launch.  A single ray is a chain of dependent node loads; everything beside it (two
+// uploads, clearing the queue counters, a grid of idle waves, two copies back) took 35 us of 55.
+template <int STACK>
+__global__ __launch_bounds__(64) void k_pick(PtSceneView sc, float4 o, float4 d, int *spill, int spillCap, int *overflow, int *out) {
+    __shared__ int sstack[stackRows(STACK) * kTraceThreads];
+    const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
+    LaneRay r;
+    traceLanes<false, STACK>(sc, r, threadIdx.x == 0, xyz(o), xyz(d), o.w, d.w, ts, overflow);
+    if (threadIdx.x == 0) *out = r.prim == INT32_MIN ? -1 : asInt(sc.prims[3 * (size_t)r.prim].w);
 }
 
 // Training targets: weight = (radiance after the vertex's sampled direction) / luminance of the
@@ -1615,27 +1697,6 @@ __global__ __launch_bounds__(256) void k_guide_finalize(float4 *records, int rec
         const float t = part[0] + part[1] + part[2] + part[3];
         if (t != 0.f) atomicAdd((float *)&counters[kWsumSlot], t);
     }
-}
-
-// What a chunk's accumulation does beside adding to the FP64 sums.
-struct PassEnd {
-    int fresh = 0;                // 1: the accumulator starts from zero here (it holds an older image)
-    float *radiance = nullptr;    // the pass's last chunk: the framebuffers (nullptr: not yet)
-    uchar4 *rgba = nullptr;
-    double invSpp = 0.0;
-    const int *overflow = nullptr;   // the pass's last kernel: traversal overflows so far,
-    int *overflowSeen = nullptr;     // and where the host reads them
-};
-
-// mean radiance + the uchar4 framebuffer of framebuffer.cu:35-40 (color.h:7-28 sRGB)
-__device__ __forceinline__ void writePixel(const double a[3], double invSpp, int p, float *radiance, uchar4 *rgba) {
-    unsigned char o[3];
-    for (int k = 0; k < 3; k++) {
-        const float v = (float)(a[k] * invSpp);
-        radiance[3 * (size_t)p + k] = v;
-        o[k] = srgbByte(v);
-    }
-    rgba[p] = make_uchar4(o[0], o[1], o[2], 255);
 }
 
 // Per pixel of the chunk: FP64 sum over the chunk's sample rows (framebuffer.cu:7-41 keeps a
@@ -1826,33 +1887,6 @@ __global__ __launch_bounds__(256) void k_tonemap(const double *accum, int npix, 
     if (end.overflow && p == 0) *end.overflowSeen = *end.overflow;
 }
 
-// Normals view (g_buffer.cu:27-57): colour (n + 1) / 2 of the primary hit at the pixel centre
-__global__ __launch_bounds__(256) void k_normals_shade(PtSceneView sc, int npix, const float4 *rayO, const float4 *rayD, const float4 *hits,
-                                                       double *accum) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npix) return;
-    const float4 h = hits[p];
-    const int slot = asInt(h.w);
-    f3 c = mk(0.f);
-    if (slot != INT32_MIN) {
-        const SurfacePoint s = surfaceAt(sc, slot, xyz(rayO[p]), xyz(rayD[p]), h.x, h.y, h.z);
-        c = (s.n + mk(1.f)) / 2.f;
-    }
-    double *a = accum + 3 * (size_t)p;
-    a[0] += c.x;
-    a[1] += c.y;
-    a[2] += c.z;
-}
-
-__global__ void k_centre_rays(PtCamera cam, int npix, int W, float4 *rayO, float4 *rayD) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npix) return;
-    f3 o, d;
-    cameraRay(cam, p / W, p % W, 0.5f, 0.5f, &o, &d);
-    rayO[p] = f4(o, 0.f);
-    rayD[p] = f4(d, FLT_MAX);
-}
-
 __global__ void k_map_prims(const PtSceneView sc, const float4 *hits, int n, float4 *out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -1939,7 +1973,7 @@ struct pt_renderer {
     DevBuf accum, radiance, rgba, stats;
     // the traversal's overflow count as of the last pass, written by its last kernel; stale after
     // traversals outside a pass
-    std::unique_ptr<HostWord> overflowSeen;
+    std::unique_ptr<HostWord> overflowSeen, picked;
     bool overflowStale = true;
     int64_t spp = 0;
     bool resetPending = false;
@@ -2708,10 +2742,6 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
     // a new image: its first chunk writes the accumulator instead of adding to it where that
     // chunk covers every pixel
     bool fresh = r->resetPending;
-    if (fresh && r->type == PT_RENDERER_NORMALS) {
-        zeroAccum(r);
-        fresh = false;
-    }
     if (fresh) {
         r->spp = 0;
         r->resetPending = false;
@@ -2723,12 +2753,17 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
         // one centre ray per pixel, added once per pass (the reference's framebuffer sees
         // spp = 1 each pass, g_buffer.cu:108-117)
         if (npix > r->poolWanted) r->poolWanted = npix;
-        ensurePool(r, npix);
-        k_centre_rays<<<(npix + 255) / 256, 256, 0, r->stream>>>(r->cam, npix, r->W, r->pp->rayO[0].as<float4>(), r->pp->rayD[0].as<float4>());
-        queueLinear(r, PT_Q_RAYS, npix);
-        launchExtend(r, 0, ptSegLen(npix), r->pp->rayO[0].as<float4>(), r->pp->rayD[0].as<float4>(), r->pp->hits.as<float4>(), TRACE_CAMERA);
-        k_normals_shade<<<(npix + 255) / 256, 256, 0, r->stream>>>(r->view, npix, r->pp->rayO[0].as<float4>(), r->pp->rayD[0].as<float4>(),
-                                                                  r->pp->hits.as<float4>(), r->accum.as<double>());
+        PassEnd end;
+        toned = !r->profile;
+        if (toned) end = passEnd(r, 1.0 / (double)(r->spp + 1));
+        end.fresh = fresh ? 1 : 0;
+        const int grid = std::min((r->W + 7) / 8 * ((r->H + 7) / 8) * 64 / kTraceThreads + 1, traceGrid(r));
+        int cap = 0;
+        int *sp = ensureSpill(r, grid, &cap), *ov = r->pp->overflow.as<int>();
+        unsigned long long *st = r->stats.as<unsigned long long>() + S_TRACE;
+        auto *kernel = r->ldsStack == 32 ? (r->traceStats ? k_normals<32, true> : k_normals<32, false>)
+                                         : (r->traceStats ? k_normals<16, true> : k_normals<16, false>);
+        kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, r->cam, r->accum.as<double>(), end, sp, cap, ov, st);
         PT_HIP_TRY(hipGetLastError());
         r->spp += 1;
         r->passSpp = spp;
@@ -2762,7 +2797,8 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
     r->lastPassPixelMajor = !r->lastChunks.empty() && r->lastChunks[0].pixelMajor;
     if (!toned) tonemap(r);
     PT_HIP_TRY(hipEventRecord(r->evEnd, r->stream));
-    r->overflowStale = !r->overflowSeen || !r->overflowSeen->p;
+    // (the normals view's one kernel still traverses when its first blocks end)
+    r->overflowStale = !r->overflowSeen || !r->overflowSeen->p || r->type == PT_RENDERER_NORMALS;
     r->inFlight = true;
     return PT_OK;
     PT_API_END("pt_renderer_render_async")
@@ -2865,9 +2901,7 @@ int pt_renderer_hit_test(pt_renderer *r, int x, int y, int *material_id, int *is
     PT_API_BEGIN
     ensurePool(r);
     r->overflowStale = true;
-    // one centre ray through the same extend kernel (hit_test.cu:25-47)
-    const float4 *dummy = nullptr;
-    (void)dummy;
+    // one centre ray (hit_test.cu:25-47)
     float4 ro, rd;
     {
         // camera.cu:24-27 generateRay(row, col) with samples (0.5, 0.5)
@@ -2881,23 +2915,21 @@ int pt_renderer_hit_test(pt_renderer *r, int x, int y, int *material_id, int *is
         ro = make_float4(c.m[0][3], c.m[1][3], c.m[2][3], 0.f);
         rd = make_float4(d[0], d[1], d[2], FLT_MAX);
     }
-    PT_HIP_TRY(hipMemcpyAsync(r->pp->rayO[0].p, &ro, 16, hipMemcpyHostToDevice, r->stream));
-    PT_HIP_TRY(hipMemcpyAsync(r->pp->rayD[0].p, &rd, 16, hipMemcpyHostToDevice, r->stream));
-    queueLinear(r, PT_Q_RAYS, 1);
-    launchExtend(r, 0, ptSegLen(1), r->pp->rayO[0].as<float4>(), r->pp->rayD[0].as<float4>(), r->pp->hits.as<float4>(), TRACE_CAMERA);
-    float4 h;
-    PT_HIP_TRY(hipMemcpyAsync(&h, r->pp->hits.p, 16, hipMemcpyDeviceToHost, r->stream));
+    if (!r->picked) r->picked = std::make_unique<HostWord>();
+    DevBuf own;   // where no pinned word was to be had
+    if (!r->picked->p) own.alloc(sizeof(int));
+    int *seen = r->picked->p ? r->picked->p : own.as<int>();
+    int cap = 0;
+    int *sp = ensureSpill(r, 1, &cap), *ov = r->pp->overflow.as<int>();
+    if (r->ldsStack == 32) k_pick<32><<<1, 64, 0, r->stream>>>(r->view, ro, rd, sp, cap, ov, seen);
+    else k_pick<16><<<1, 64, 0, r->stream>>>(r->view, ro, rd, sp, cap, ov, seen);
+    PT_HIP_TRY(hipGetLastError());
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
-    const int slot = asInt(h.w);
-    if (slot == INT32_MIN) {
-        if (material_id) *material_id = -1;
-        if (is_hit) *is_hit = 0;
-    } else {
-        float4 p0;
-        PT_HIP_TRY(hipMemcpy(&p0, r->prims.as<float4>() + 3 * (size_t)slot, 16, hipMemcpyDeviceToHost));
-        if (material_id) *material_id = asInt(p0.w);
-        if (is_hit) *is_hit = 1;
-    }
+    int mat = -1;
+    if (r->picked->p) mat = *(volatile int *)r->picked->p;
+    else PT_HIP_TRY(hipMemcpy(&mat, own.p, sizeof mat, hipMemcpyDeviceToHost));
+    if (material_id) *material_id = mat;
+    if (is_hit) *is_hit = mat >= 0 ? 1 : 0;
     return PT_OK;
     PT_API_END("pt_renderer_hit_test")
 }

@@ -367,17 +367,17 @@ class Renderer:
         return v.value
 
     def radiance(self):
-        out = np.zeros((self.H, self.W, 3), np.float32)
+        out = np.empty((self.H, self.W, 3), np.float32)
         check(lib().pt_renderer_get_radiance(self.h, _p(out)))
         return out
 
     def radiance_sum(self):
-        out = np.zeros((self.H, self.W, 3), np.float64)
+        out = np.empty((self.H, self.W, 3), np.float64)
         check(lib().pt_renderer_get_radiance_sum(self.h, _p(out)))
         return out
 
     def rgba8(self):
-        out = np.zeros((self.H, self.W, 4), np.uint8)
+        out = np.empty((self.H, self.W, 4), np.uint8)
         check(lib().pt_renderer_get_rgba8(self.h, _p(out)))
         return out
 
@@ -463,7 +463,7 @@ class Batch:
 
     def radiance(self, i):
         w, h = self.sizes[i]
-        out = np.zeros((h, w, 3), np.float32)
+        out = np.empty((h, w, 3), np.float32)
         check(lib().pt_batch_get_radiance(self.h, i, _p(out)))
         return out
 
