@@ -370,7 +370,7 @@ __device__ __forceinline__ Rng cameraRng(const ChunkParams &cp, int path) {
 // queries too: nearer occluders are found sooner).
 //
 // The stack of a lane is a column of LDS rows (kTraceThreads ints apart): a sentinel at the
-// bottom, the newest STACK or so entries above it, and below those, for trees that need them,
+// bottom, the newest entries above it, and below those, for trees that need them,
 // older entries in a spill area in global memory interleaved by lane
 // (spill[entry * lanes + lane]).  When the LDS part fills up its older half moves to the spill
 // area, and when the sentinel comes up with entries spilled the newest of them move back: both
@@ -379,7 +379,7 @@ __device__ __forceinline__ Rng cameraRng(const ChunkParams &cp, int path) {
 // What bounds the kernels is the L1's lookup rate, one access per cycle and CU: every lane's 16
 // bytes of a node are an access of their own (neighbouring lanes rarely hold the same node), seven
 // per node visit, and they fill 99% of the cycles of the icosphere's incoherent bounces (TD busy
-// 100%, VALU 69%).  The node step leaves those loads as they are and needs few instructions beside
+// 100%, VALU 69%, of 52% of their lanes).  The node step leaves those loads as they are and needs few instructions beside
 // them (about 85; the first version's, with a compare-and-select sorting network, separate push,
 // pop and leaf branches and the stack's row stride in a register, took about 150 and VALU issue was
 // the larger share: room extend 7087 -> 6594 us and shadow 4004 -> 3802 us a pass, icosphere extend
@@ -411,8 +411,27 @@ typedef __attribute__((address_space(3))) int LdsInt;
 // number of spilled entries.
 static constexpr int kStackSentinel = 1;
 static constexpr int kStackFirst = 2;
-constexpr int stackCountRow(int entries) { return kStackFirst + entries + 6; }
-constexpr int stackRows(int entries) { return stackCountRow(entries) + 1; }
+// Of `rows` rows of an LDS stack (PT_OPT_TRACE_LDS_STACK) those for entries: three fewer, so that the
+// columns and top nodes of the 11 blocks of a CU fit its LDS.
+constexpr int stackEntries(int rows) { return rows - 3; }
+constexpr int stackCountRow(int rows) { return kStackFirst + stackEntries(rows) + 6; }
+constexpr int stackRows(int rows) { return stackCountRow(rows) + 1; }
+
+// The first nodes in LDS: the tree's top levels, as the order is breadth-first.  A node's load is
+// seven L1 lookups per lane, and the L1 answers one a clock (91 to 100% busy in these kernels); 30% of
+// the visits of the 1.31M-triangle scene and 54% of the room's fall on the first 21 nodes, which LDS
+// serves beside the L1: room extend 6587 -> 6007 us a pass and shadow 3772 -> 3579, icosphere extend
+// 6941 -> 6763 and shadow 4529 -> 4476.  The queue kernels have them: a block traces many rays
+// there.  Kernels that trace a fixed 64 paths a wave keep to the L1 (with top nodes: mesh preview 318
+// -> 329 us, the copy costing more than it gives), and so do a batch's, whose renders are small.
+// Float4 k of node n is at 128 n + 16 (k ^ n % 8), so that lanes at different nodes spread over
+// the banks.
+static constexpr int kTopNodes = 21;
+typedef float V4 __attribute__((ext_vector_type(4)));
+typedef int I4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) V4 LdsV4;
+typedef __attribute__((address_space(3))) I4 LdsI4;
+typedef __attribute__((address_space(3))) char LdsChar;
 
 struct TraceStack {
     LdsInt *column;   // this lane's row 0; rows kTraceThreads apart
@@ -544,7 +563,7 @@ template <int STACK> __device__ __forceinline__ void stackStart(LaneRay &r, cons
 
 // Makes room: the older half of the LDS entries moves to the spill area.
 template <int STACK> __device__ __forceinline__ LdsInt *stackEvict(LdsInt *sp, const TraceStack ts, int *overflow) {
-    constexpr int kMove = STACK / 2;
+    constexpr int kMove = stackEntries(STACK) / 2;
     LdsInt *first = ts.column + kStackFirst * kTraceThreads;
     LdsInt *count = ts.column + stackCountRow(STACK) * kTraceThreads;
     const int n = *count;
@@ -562,7 +581,7 @@ template <int STACK> __device__ __forceinline__ LdsInt *stackEvict(LdsInt *sp, c
 // Moves the newest spilled entries back into an empty LDS part; returns its first free entry (the
 // one above the sentinel when nothing was spilled).
 template <int STACK> __device__ __forceinline__ LdsInt *stackRefill(const TraceStack ts) {
-    constexpr int kMove = STACK / 2;
+    constexpr int kMove = stackEntries(STACK) / 2;
     LdsInt *first = ts.column + kStackFirst * kTraceThreads;
     LdsInt *count = ts.column + stackCountRow(STACK) * kTraceThreads;
     const int n = *count;
@@ -580,8 +599,9 @@ template <int STACK> __device__ __forceinline__ LdsInt *stackRefill(const TraceS
 // visited only because its leaf was parked holds no primitive at or below the final tmax, so the
 // hit does not depend on the schedule.  Returns true when the ray is finished: the stack is
 // exhausted, or an any-hit query found an occluder.
-template <bool ANY, int STACK, bool STATS = false>
-__device__ __forceinline__ bool traceRound(const PtSceneView &sc, LaneRay &r, const TraceStack &ts, int *overflow, TraceCount *tc = nullptr) {
+template <bool ANY, int STACK, bool STATS = false, bool TOP = false>
+__device__ __forceinline__ bool traceRound(const PtSceneView &sc, LaneRay &r, const TraceStack &ts, int *overflow, TraceCount *tc = nullptr,
+                                           const LdsChar *top = nullptr) {
     const char *nodes = (const char *)sc.nodes;
     int leaf = 0;   // parked leaf reference (< 0), or 0
     if (r.node < 0) {
@@ -597,22 +617,41 @@ __device__ __forceinline__ bool traceRound(const PtSceneView &sc, LaneRay &r, co
         const uint64_t searching = __ballot(leaf == 0 && r.node >= 0);
         if (searching == 0) break;
         if (__popcll(searching) <= kDescentTail && __ballot(leaf != 0) != 0) break;
-        if (ts.spillCap > 0 && r.sp > ts.column + (kStackFirst + STACK - 1) * kTraceThreads) r.sp = stackEvict<STACK>(r.sp, ts, overflow);
+        if (ts.spillCap > 0 && r.sp > ts.column + (kStackFirst + stackEntries(STACK) - 1) * kTraceThreads) r.sp = stackEvict<STACK>(r.sp, ts, overflow);
         // a lane that parks a leaf in the first step keeps descending internal nodes in the next
         // (as it would while other lanes search) and idles at its second leaf
 #pragma unroll
         for (int step = 0; step < kDescentSteps; step++) {
             if (r.node >= 0) {
                 if constexpr (STATS) tc->nodes++;
-                // 32-bit offsets from the array base (a node array stays below 4 GiB); a node is
-                // 128 bytes, so the near bound's offset is an OR and the far bound of the same axis
-                // (the other float4 of the pair) is that offset XOR 16
-                const uint32_t base = (uint32_t)r.node * (uint32_t)(PT_NODE_F4 * 16);
-                const uint32_t ax = base | r.nX, ay = base | r.nY, az = base | r.nZ;
-                const float4 nx = *(const float4 *)(nodes + ax), fx = *(const float4 *)(nodes + (ax ^ 16u));
-                const float4 ny = *(const float4 *)(nodes + ay), fy = *(const float4 *)(nodes + (ay ^ 16u));
-                const float4 nz = *(const float4 *)(nodes + az), fz = *(const float4 *)(nodes + (az ^ 16u));
-                const int4 rf = *(const int4 *)(nodes + (base + 96u));
+                V4 nx, fx, ny, fy, nz, fz;
+                I4 rf;
+                const bool inLds = TOP && r.node < kTopNodes;
+                if (!inLds) {
+                    // 32-bit offsets from the array base (a node array stays below 4 GiB); a node is
+                    // 128 bytes, so the near bound's offset is an OR and the far bound of the same
+                    // axis (the other float4 of the pair) is that offset XOR 16
+                    const uint32_t base = (uint32_t)r.node * (uint32_t)(PT_NODE_F4 * 16);
+                    const uint32_t ax = base | r.nX, ay = base | r.nY, az = base | r.nZ;
+                    nx = *(const V4 *)(nodes + ax);
+                    fx = *(const V4 *)(nodes + (ax ^ 16u));
+                    ny = *(const V4 *)(nodes + ay);
+                    fy = *(const V4 *)(nodes + (ay ^ 16u));
+                    nz = *(const V4 *)(nodes + az);
+                    fz = *(const V4 *)(nodes + (az ^ 16u));
+                    rf = *(const I4 *)(nodes + (base + 96u));
+                }
+                if (inLds) {
+                    const uint32_t at = (uint32_t)r.node << 7 | ((uint32_t)r.node & 7u) << 4;
+                    const uint32_t ax = at ^ r.nX, ay = at ^ r.nY, az = at ^ r.nZ;
+                    nx = *(const LdsV4 *)(top + ax);
+                    fx = *(const LdsV4 *)(top + (ax ^ 16u));
+                    ny = *(const LdsV4 *)(top + ay);
+                    fy = *(const LdsV4 *)(top + (ay ^ 16u));
+                    nz = *(const LdsV4 *)(top + az);
+                    fz = *(const LdsV4 *)(top + (az ^ 16u));
+                    rf = *(const LdsI4 *)(top + (at ^ 96u));
+                }
                 const float bnx[4] = {nx.x, nx.y, nx.z, nx.w}, bfx[4] = {fx.x, fx.y, fx.z, fx.w};
                 const float bny[4] = {ny.x, ny.y, ny.z, ny.w}, bfy[4] = {fy.x, fy.y, fy.z, fy.w};
                 const float bnz[4] = {nz.x, nz.y, nz.z, nz.w}, bfz[4] = {fz.x, fz.y, fz.z, fz.w};
@@ -697,6 +736,13 @@ template <int STACK> __device__ __forceinline__ TraceStack traceStack(int *sstac
     return ts;
 }
 
+// Fills `top`; called by the whole block, whatever its size.
+__device__ __forceinline__ void loadTopNodes(V4 *top, const PtSceneView &sc) {
+    const int n = min(kTopNodes, sc.numNodes) * PT_NODE_F4;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) top[(k & ~7) | ((k ^ k >> 3) & 7)] = ((const V4 *)sc.nodes)[k];
+    __syncthreads();
+}
+
 // Work distribution over a segmented queue (the trace kernels and shade).  Wave w's home
 // segment is w % PT_QUEUE_SEGS; it claims records there with one atomic on that segment's
 // cursor and, once its home is exhausted, helps up to kQueueSteal following segments before
@@ -746,9 +792,9 @@ __device__ __forceinline__ int segClaim(int *counters, int bounce, int countFiel
 // rays once `refill` or more of its lanes are idle, as a contiguous run of one segment so that
 // the rays in flight on a CU stay neighbours, and leaves once its segments are exhausted and
 // its lanes idle.
-template <bool ANY, int STACK, bool STATS = false, class Load, class Finish>
+template <bool ANY, int STACK, bool STATS, bool TOP, class Load, class Finish>
 __device__ __forceinline__ void traceQueue(const PtSceneView &sc, int *counters, int bounce, int countField, int fetchField, int segLen,
-                                           int refill, const TraceStack &ts, int *overflow, Load load, Finish finish,
+                                           int refill, const TraceStack &ts, const V4 *top, int *overflow, Load load, Finish finish,
                                            unsigned long long *tstat = nullptr) {
     SegCursor cur = segStart();
     if (sc.numNodes == 0) {
@@ -783,7 +829,7 @@ __device__ __forceinline__ void traceQueue(const PtSceneView &sc, int *counters,
         }
         // all lanes idle after a refill attempt means this wave's segments are exhausted
         if (__ballot(ray >= 0) == 0) break;
-        if (ray >= 0 && traceRound<ANY, STACK, STATS>(sc, r, ts, overflow, &tc)) {
+        if (ray >= 0 && traceRound<ANY, STACK, STATS, TOP>(sc, r, ts, overflow, &tc, (const LdsChar *)top)) {
             finish(ray, r.prim >= 0, laneRayHit(r));
             ray = -1;
         }
@@ -803,9 +849,11 @@ __global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_extend(P
                                                                               int refill, int *spill, int spillCap, int *overflow,
                                                                               ChunkParams cp = ChunkParams{}, unsigned long long *tstat = nullptr) {
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
+    __shared__ V4 top[BATCH ? 1 : kTopNodes * PT_NODE_F4];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
-    traceQueue<false, STACK, STATS>(
-        sc, counters, bounce, PT_Q_RAYS, PT_Q_FETCH_EXT, segLen, refill, ts, overflow,
+    if constexpr (!BATCH) loadTopNodes(top, sc);
+    traceQueue<false, STACK, STATS, !BATCH>(
+        sc, counters, bounce, PT_Q_RAYS, PT_Q_FETCH_EXT, segLen, refill, ts, top, overflow,
         [&](int i, f3 &o, f3 &d, float &tmin, float &tmax, int &root) {
             const float4 rd = rayD[i];
             if constexpr (BATCH) {
@@ -963,13 +1011,15 @@ __global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_shadow(P
                                                                               int refill, int *spill, int spillCap, int *overflow,
                                                                               const BatchRender *renders = nullptr, unsigned long long *tstat = nullptr) {
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
+    __shared__ V4 top[BATCH ? 1 : kTopNodes * PT_NODE_F4];
     // each lane's path index, kept from the ray's load (a re-read after the traversal would be a
     // dependent round trip ahead of the radiance update)
     __shared__ int sPath[kTraceThreads];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
+    if constexpr (!BATCH) loadTopNodes(top, sc);
     int adds = 0;
-    traceQueue<true, STACK, STATS>(
-        sc, counters, bounce, PT_Q_SHADOW, PT_Q_FETCH_SHADOW, segLen, refill, ts, overflow,
+    traceQueue<true, STACK, STATS, !BATCH>(
+        sc, counters, bounce, PT_Q_SHADOW, PT_Q_FETCH_SHADOW, segLen, refill, ts, top, overflow,
         [&](int i, f3 &o, f3 &d, float &tmin, float &tmax, int &root) {
             const float4 so = sO[i], sd = sD[i];
             o = xyz(so);
@@ -2096,7 +2146,7 @@ void zeroAccum(pt_renderer *r) {
 
 // Spill area of the traversal stacks: entries beyond the LDS part for every lane of the grid.
 int *ensureSpill(pt_renderer *r, int grid, int *cap) {
-    *cap = r->stackNeed > r->ldsStack ? r->stackNeed : 0;
+    *cap = r->stackNeed > stackEntries(r->ldsStack) ? r->stackNeed : 0;
     const size_t bytes = (size_t)grid * kTraceThreads * std::max(*cap, 1) * sizeof(int);
     if (r->pp->spill.bytes < bytes) r->pp->spill.alloc(bytes);
     return r->pp->spill.as<int>();

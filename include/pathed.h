@@ -168,8 +168,8 @@ typedef enum {
     PT_OPT_GUIDE_LR_MICRO = 7,   /* guided: Adam learning rate in units of 1e-6 (default 10000) */
     PT_OPT_GUIDE_RESET = 8,      /* guided: re-initialise the network with seed = value;
                                     get: number of training steps taken */
-    PT_OPT_TRACE_LDS_STACK = 9,  /* traversal stack entries per lane kept in LDS (16 or 32);
-                                    deeper entries spill to global memory */
+    PT_OPT_TRACE_LDS_STACK = 9,  /* traversal stack rows per lane in LDS (16 or 32, holding 13
+                                    or 29 entries); deeper entries spill to global memory */
     PT_OPT_BATCH_GRAPH = 10,     /* batches only: 1 (default) = capture the whole batch in one
                                     hipGraph and launch it once; 0 = launch kernels directly */
     PT_OPT_GUIDE_MAX_FRACTION_MILLI = 11, /* guided: cap, in thousandths, on the probability of
