@@ -430,9 +430,13 @@ struct Ray {
 // own guarantees and a fused multiply-add does not.
 struct WtRay {
     f3 o;
-    int kx, ky, kz;
+    int kz;   // the direction's dominant axis; kx and ky are the two after it, cyclically
     float Sx, Sy, Sz;
 };
+// a's components on kx, ky, kz
+PT_INLINE f3 wtAxes(f3 a, int kz) {
+    return mk(kz == 0 ? a.y : kz == 1 ? a.z : a.x, kz == 0 ? a.z : kz == 1 ? a.x : a.y, kz == 0 ? a.x : kz == 1 ? a.y : a.z);
+}
 PT_INLINE WtRay wtSetup(f3 o, f3 d) {
 #pragma clang fp contract(off)
     WtRay r;
@@ -442,23 +446,22 @@ PT_INLINE WtRay wtSetup(f3 o, f3 d) {
     float m = ax;
     if (ay > m) { kz = 1; m = ay; }
     if (az > m) { kz = 2; }
-    int kx = kz + 1; if (kx == 3) kx = 0;
-    int ky = kx + 1; if (ky == 3) ky = 0;
-    const float dz = comp(d, kz);
-    if (dz < 0.f) { const int t = kx; kx = ky; ky = t; }
-    r.kx = kx; r.ky = ky; r.kz = kz;
-    r.Sx = comp(d, kx) / dz;
-    r.Sy = comp(d, ky) / dz;
-    r.Sz = 1.f / dz;
+    // (exchanging kx and ky for a negative dz, to keep the winding, would negate U, V, W, their
+    // sum and the distance's numerator exactly and change no result)
+    r.kz = kz;
+    d = wtAxes(d, kz);
+    r.Sx = d.x / d.z;
+    r.Sy = d.y / d.z;
+    r.Sz = 1.f / d.z;
     return r;
 }
 PT_INLINE bool wtHit(const WtRay &r, f3 p0, f3 p1, f3 p2, float tMin, float tMax, float *tt, float *uu, float *vv) {
 #pragma clang fp contract(off)
-    const f3 A = p0 - r.o, B = p1 - r.o, C = p2 - r.o;
-    const float Akz = comp(A, r.kz), Bkz = comp(B, r.kz), Ckz = comp(C, r.kz);
-    const float Ax = comp(A, r.kx) - r.Sx * Akz, Ay = comp(A, r.ky) - r.Sy * Akz;
-    const float Bx = comp(B, r.kx) - r.Sx * Bkz, By = comp(B, r.ky) - r.Sy * Bkz;
-    const float Cx = comp(C, r.kx) - r.Sx * Ckz, Cy = comp(C, r.ky) - r.Sy * Ckz;
+    const f3 A = wtAxes(p0 - r.o, r.kz), B = wtAxes(p1 - r.o, r.kz), C = wtAxes(p2 - r.o, r.kz);
+    const float Akz = A.z, Bkz = B.z, Ckz = C.z;
+    const float Ax = A.x - r.Sx * Akz, Ay = A.y - r.Sy * Akz;
+    const float Bx = B.x - r.Sx * Bkz, By = B.y - r.Sy * Bkz;
+    const float Cx = C.x - r.Sx * Ckz, Cy = C.y - r.Sy * Ckz;
     float U = Cx * By - Cy * Bx;
     float V = Ax * Cy - Ay * Cx;
     float W = Bx * Ay - By * Ax;

@@ -476,16 +476,6 @@ __device__ __forceinline__ void keyOrder(double &a, double &b) {
     b = lo;
 }
 
-__device__ __forceinline__ void cswap(float &ta, int &ra, float &tb, int &rb) {
-    const bool s = tb < ta;
-    const float t = s ? tb : ta;
-    const int r = s ? rb : ra;
-    tb = s ? ta : tb;
-    rb = s ? ra : rb;
-    ta = t;
-    ra = r;
-}
-
 // One ray in flight on a lane: the slab-test and watertight-test set-ups, the search interval
 // (tmax is the closest hit's distance once prim >= 0), the closest hit's primitive and
 // barycentrics, and the traversal position (node >= 0: a 4-wide node; < 0: a leaf,
@@ -885,9 +875,115 @@ __global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_extend(P
         [&](int i, bool, const TraceHit &th) { hits[i] = make_float4(th.t, th.u, th.v, asFloat(th.prim)); }, tstat);
 }
 
-// Wave stack entries of the packet traversal, and its blocks per CU.
+// Wave stack entries of the packet traversal (one per lane of a register), and its blocks per CU.
 static constexpr int kPacketStack = 64;
 static constexpr int kPacketBlocksPerCU = 16;
+
+typedef __attribute__((address_space(4))) const V4 ConstV4;
+typedef __attribute__((address_space(4))) const I4 ConstI4;
+typedef __attribute__((address_space(4))) const char ConstChar;
+
+__device__ __forceinline__ void cswap(int &ka, int &ra, int &kb, int &rb) {
+    const bool s = kb < ka;
+    const int k = ka, f = ra;
+    ka = s ? kb : ka; kb = s ? k : kb;
+    ra = s ? rb : ra; rb = s ? f : rb;
+}
+
+// One run of the packet traversal: r's closest hits, all lanes together.  KZ >= 0: the run's rays
+// have the same direction signs and this dominant axis (most runs; a primitive's coordinates then
+// need no selection); -1: any rays.
+template <int KZ> __device__ __forceinline__ void packetRun(const PtSceneView &sc, LaneRay &r, int *overflow) {
+    ConstChar *nodes = (ConstChar *)sc.nodes;
+    ConstChar *prims = (ConstChar *)sc.prims;
+    const uint32_t sX = __builtin_amdgcn_readfirstlane(r.nX), sY = __builtin_amdgcn_readfirstlane(r.nY), sZ = __builtin_amdgcn_readfirstlane(r.nZ);
+    WtRay wr = r.wr;
+    if constexpr (KZ >= 0) wr.kz = KZ;
+    // a primitive against every lane's ray (as traceRound's leaf phase)
+    auto test = [&](ConstChar *at, int prim) {
+        const V4 p0 = *(ConstV4 *)at, p1 = *(ConstV4 *)(at + 16);
+        V4 p2 = *(ConstV4 *)(at + 32);
+        asm volatile("" : "+s"(p2));   // loaded with the others, not after the branch below
+        float t, u = 0.f, v = 0.f;
+        bool h;
+        if (asInt(p1.w) == PT_TAG_SPHERE) {
+            h = sphereHit(mk(p0.x, p0.y, p0.z), p1.x, r.wr.o, r.d, r.tmin, r.tmax, &t);
+        } else {
+            h = wtHit(wr, mk(p0.x, p0.y, p0.z), mk(p1.x, p1.y, p1.z), mk(p2.x, p2.y, p2.z), r.tmin, r.tmax, &t, &u, &v);
+        }
+        if (h) {
+            r.tmax = t;
+            r.u = u;
+            r.v = v;
+            r.prim = prim;
+        }
+    };
+    const int lane = laneId();
+    int node = 0, sp = 0, stack = 0;   // wave-uniform but for the stack: entry k is lane k's
+    while (true) {
+        if (node >= 0) {
+            ConstChar *at = nodes + (size_t)(uint32_t)node * (PT_NODE_F4 * 16);
+            V4 nx, fx, ny, fy, nz, fz;
+            if constexpr (KZ >= 0) {
+                nx = *(ConstV4 *)(at + sX); fx = *(ConstV4 *)(at + (sX ^ 16u));
+                ny = *(ConstV4 *)(at + sY); fy = *(ConstV4 *)(at + (sY ^ 16u));
+                nz = *(ConstV4 *)(at + sZ); fz = *(ConstV4 *)(at + (sZ ^ 16u));
+            } else {
+                const V4 x0 = *(ConstV4 *)at, x1 = *(ConstV4 *)(at + 16), y0 = *(ConstV4 *)(at + 32), y1 = *(ConstV4 *)(at + 48),
+                         z0 = *(ConstV4 *)(at + 64), z1 = *(ConstV4 *)(at + 80);
+                nx = r.nX == 0u ? x0 : x1; fx = r.nX == 0u ? x1 : x0;
+                ny = r.nY == 32u ? y0 : y1; fy = r.nY == 32u ? y1 : y0;
+                nz = r.nZ == 64u ? z0 : z1; fz = r.nZ == 64u ? z1 : z0;
+            }
+            const I4 rf = *(ConstI4 *)(at + 96);
+            int ref[4] = {rf.x, rf.y, rf.z, rf.w}, key[4];
+            asm volatile("" : "+s"(ref[0]), "+s"(ref[1]), "+s"(ref[2]), "+s"(ref[3]));   // loaded with the planes
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float lo = max3(nx[k] * r.ix - r.ox, ny[k] * r.iy - r.oy, max2(nz[k] * r.iz - r.oz, r.tmin));
+                const float hi = min3(fx[k] * r.ix - r.ox, fy[k] * r.iy - r.oy, min2(fz[k] * r.iz - r.oz, r.tmax));
+                const bool in = lo <= hi;
+                // the run's first lane orders the children; one that only other lanes enter
+                // comes after its hits, one that no lane enters is not visited.  Distances are
+                // not negative (a camera ray's tmin is 0), so their bits order as they do
+                const int first = __builtin_amdgcn_readfirstlane(asInt(in ? lo : FLT_MAX));
+                key[k] = __ballot(in) != 0 ? first : INT32_MAX;
+            }
+            cswap(key[0], ref[0], key[1], ref[1]);
+            cswap(key[2], ref[2], key[3], ref[3]);
+            cswap(key[0], ref[0], key[2], ref[2]);
+            cswap(key[1], ref[1], key[3], ref[3]);
+            cswap(key[1], ref[1], key[2], ref[2]);
+            if (key[0] != INT32_MAX) {
+                // the farthest lowest, the second nearest on top
+                if (sp + 3 <= kPacketStack) {
+                    if (key[1] != INT32_MAX) {
+                        if (key[2] != INT32_MAX) {
+                            if (key[3] != INT32_MAX) stack = lane == sp++ ? ref[3] : stack;
+                            stack = lane == sp++ ? ref[2] : stack;
+                        }
+                        stack = lane == sp++ ? ref[1] : stack;
+                    }
+                } else if (lane == 0) {
+                    atomicAdd(overflow, 1);
+                }
+                node = ref[0];
+                continue;
+            }
+        } else {
+            // a leaf (PT_LEAF_MAX is 2)
+            const int e = ~node;
+            const int first = e & ((1 << PT_LEAF_COUNT_SHIFT) - 1);
+            const int cnt = (e >> PT_LEAF_COUNT_SHIFT) + 1;
+            ConstChar *at = prims + (size_t)(uint32_t)first * 48u;
+            test(at, first);
+            if (cnt > 1) test(at + 48, first + 1);
+        }
+        if (sp == 0) break;
+        sp--;
+        node = __builtin_amdgcn_readlane(stack, sp);
+    }
+}
 
 // Camera bounce of a pixel-major chunk whose runs of 64 camera rays are one pixel's samples
 // (or a few neighbouring pixels' samples),
@@ -901,11 +997,16 @@ static constexpr int kPacketBlocksPerCU = 16;
 // equal distances may resolve to another primitive than in the per-lane traversal).  Runs
 // are claimed 64 at a time; the wave stack holds kPacketStack entries (launched only when the
 // tree's 3 x depth + 1 fits, with an overflow counter besides).
-__global__ __launch_bounds__(kTraceThreads, 6) void k_extend_packet(PtSceneView sc, int *counters, int bounce, int segLen, const float4 *rayO,
+//
+// Nodes and primitives are the wave's, so they are scalar loads into scalar registers, which the
+// tests take as operands; the children are ordered by the scalar unit and the stack is a register.
+// A run whose rays share direction signs and dominant axis (packetRun<KZ>) needs no selection of
+// planes or coordinates either.  As vector loads, with LDS for the stack, the L1's lookups (93% of
+// the cycles) and VALU issue (100%) both bound the kernel: 1.31M triangles, 2^26 rays, 4385 us; now
+// 2780 us, VALU issue at 98% with 1436 instead of 2330 instructions a run, the scalar unit at 92%,
+// and eight waves per SIMD to cover the scalar loads (six: 3% slower).
+__global__ __launch_bounds__(kTraceThreads, 8) void k_extend_packet(PtSceneView sc, int *counters, int bounce, int segLen, const float4 *rayO,
                                                                    const float4 *rayD, float4 camO, float4 *hits, int *overflow) {
-    __shared__ int wstack[kTraceThreads / 64][kPacketStack];
-    int *ws = wstack[threadIdx.x >> 6];
-    const char *nodes = (const char *)sc.nodes;
     SegCursor cur = segStart();
     while (true) {
         int slot = 0;
@@ -919,82 +1020,12 @@ __global__ __launch_bounds__(kTraceThreads, 6) void k_extend_packet(PtSceneView 
         LaneRay r;
         // a lane without a ray gets an empty interval: every box and primitive test fails
         laneRayStart(r, xyz(ro), xyz(rd), ro.w, valid ? rd.w : -1.f, 0);
-        int node = 0, sp = 0;   // wave-uniform
-        while (true) {
-            if (node >= 0) {
-                const uint32_t base = (uint32_t)node * (uint32_t)(PT_NODE_F4 * 16);
-                const uint32_t ax = base | r.nX, ay = base | r.nY, az = base | r.nZ;
-                const float4 nx = *(const float4 *)(nodes + ax), fx = *(const float4 *)(nodes + (ax ^ 16u));
-                const float4 ny = *(const float4 *)(nodes + ay), fy = *(const float4 *)(nodes + (ay ^ 16u));
-                const float4 nz = *(const float4 *)(nodes + az), fz = *(const float4 *)(nodes + (az ^ 16u));
-                const int4 rf = *(const int4 *)(nodes + (base + 96u));
-                const float bnx[4] = {nx.x, nx.y, nx.z, nx.w}, bfx[4] = {fx.x, fx.y, fx.z, fx.w};
-                const float bny[4] = {ny.x, ny.y, ny.z, ny.w}, bfy[4] = {fy.x, fy.y, fy.z, fy.w};
-                const float bnz[4] = {nz.x, nz.y, nz.z, nz.w}, bfz[4] = {fz.x, fz.y, fz.z, fz.w};
-                int ref[4] = {__builtin_amdgcn_readfirstlane(rf.x), __builtin_amdgcn_readfirstlane(rf.y),
-                              __builtin_amdgcn_readfirstlane(rf.z), __builtin_amdgcn_readfirstlane(rf.w)};
-                float key[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const float lo = fmaxf(fmaxf(bnx[k] * r.ix - r.ox, bny[k] * r.iy - r.oy), fmaxf(bnz[k] * r.iz - r.oz, r.tmin));
-                    const float hi = fminf(fminf(bfx[k] * r.ix - r.ox, bfy[k] * r.iy - r.oy), fminf(bfz[k] * r.iz - r.oz, r.tmax));
-                    const bool in = lo <= hi;
-                    // the run's first lane orders the children; one that only other lanes enter
-                    // comes after its hits, one that no lane enters is not visited
-                    const float first = __builtin_amdgcn_readfirstlane(__float_as_int(in ? lo : INFINITY)) == __float_as_int(INFINITY)
-                                            ? FLT_MAX
-                                            : __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(in ? lo : INFINITY)));
-                    key[k] = __ballot(in) != 0 ? first : INFINITY;
-                }
-                cswap(key[0], ref[0], key[1], ref[1]);
-                cswap(key[2], ref[2], key[3], ref[3]);
-                cswap(key[0], ref[0], key[2], ref[2]);
-                cswap(key[1], ref[1], key[3], ref[3]);
-                cswap(key[1], ref[1], key[2], ref[2]);
-                if (key[0] != INFINITY) {
-                    const int more = (key[1] != INFINITY) + (key[2] != INFINITY) + (key[3] != INFINITY);
-                    if (sp + more <= kPacketStack) {
-                        // the farthest lowest, the second nearest on top
-                        if (more >= 3) ws[sp] = ref[3];
-                        if (more >= 2) ws[sp + more - 2] = ref[2];
-                        if (more >= 1) ws[sp + more - 1] = ref[1];
-                        sp += more;
-                    } else if (laneId() == 0) {
-                        atomicAdd(overflow, 1);
-                    }
-                    node = ref[0];
-                    continue;
-                }
-            } else {
-                // a leaf: every lane tests its primitives (as traceRound's leaf phase)
-                const int e = ~node;
-                const int first = e & ((1 << PT_LEAF_COUNT_SHIFT) - 1);
-                const int cnt = (e >> PT_LEAF_COUNT_SHIFT) + 1;
-                for (int j = 0; j < cnt; j++) {
-                    const uint32_t off = (uint32_t)(first + j) * 48u;
-                    const char *pr = (const char *)sc.prims;
-                    const float4 p0 = *(const float4 *)(pr + off);
-                    float4 p1 = *(const float4 *)(pr + (off + 16u)), p2 = *(const float4 *)(pr + (off + 32u));
-                    asm volatile("" : "+v"(p1.y), "+v"(p1.z), "+v"(p2.x), "+v"(p2.y), "+v"(p2.z));
-                    float t, u = 0.f, v = 0.f;
-                    bool h;
-                    if (asInt(p1.w) == PT_TAG_SPHERE) {
-                        h = sphereHit(xyz(p0), p1.x, r.wr.o, r.d, r.tmin, r.tmax, &t);
-                    } else {
-                        h = wtHit(r.wr, xyz(p0), xyz(p1), xyz(p2), r.tmin, r.tmax, &t, &u, &v);
-                    }
-                    if (h) {
-                        r.tmax = t;
-                        r.u = u;
-                        r.v = v;
-                        r.prim = first + j;
-                    }
-                }
-            }
-            if (sp == 0) break;
-            sp--;
-            node = __builtin_amdgcn_readfirstlane(ws[sp]);
-        }
+        const uint32_t kind = r.nX | r.nY << 8 | r.nZ << 16 | (uint32_t)r.wr.kz << 24;
+        const int kz = __ballot(kind != (uint32_t)__builtin_amdgcn_readfirstlane(kind)) != 0 ? -1 : __builtin_amdgcn_readfirstlane(r.wr.kz);
+        if (kz == 0) packetRun<0>(sc, r, overflow);
+        else if (kz == 1) packetRun<1>(sc, r, overflow);
+        else if (kz == 2) packetRun<2>(sc, r, overflow);
+        else packetRun<-1>(sc, r, overflow);
         if (valid) {
             const TraceHit th = laneRayHit(r);
             hits[i] = make_float4(th.t, th.u, th.v, asFloat(th.prim));
@@ -2178,9 +2209,7 @@ void launchExtend(pt_renderer *r, int bounce, int segLen, const float4 *ro, cons
     int *ctr = r->pp->counters.as<int>();
     int *ov = r->pp->overflow.as<int>();
     if (packet) {
-        // the packet kernel holds 64 registers and a 512-byte LDS stack per block: 16 two-wave
-        // blocks per CU fit (8 waves per SIMD); C1 6037-6050 against 5953-5972 Mrays/s with the
-        // per-lane kernels' 11 blocks per CU
+        // the packet kernel holds 64 registers: 16 two-wave blocks per CU fit (8 waves per SIMD)
         k_extend_packet<<<std::max(grid, r->cus * kPacketBlocksPerCU), kTraceThreads, 0, r->stream>>>(r->view, ctr, bounce, segLen, ro, rd, camO, hits, ov);
         PT_HIP_TRY(hipGetLastError());
         return;
