@@ -449,9 +449,8 @@ typedef __attribute__((address_space(3))) char LdsChar;
 
 struct TraceStack {
     LdsInt *column;   // this lane's row 0; rows kTraceThreads apart
-    int *spill;       // this lane's first spill entry; entries spillStride apart
+    int *spill;       // the spill area: entry k of lane n (of all lanes) at spill[k * lanes + n]
     int spillCap;     // spill entries per lane (0: the tree never needs them)
-    int spillStride;
 };
 
 // Largest and smallest of floats that are never signalling NaNs (the compiler quiets its operands
@@ -540,6 +539,10 @@ __device__ __forceinline__ TraceHit laneRayHit(const LaneRay &r) {
 }
 
 static constexpr int kTraceDone = INT32_MIN;   // LaneRay::node once the stack is exhausted
+// What a kernel's rays look for: the closest hit, any hit, or each ray its own (LaneRay::prim starts
+// as kMissAny for any hit).
+enum TraceMode { CLOSEST, ANY, MIXED };
+static constexpr int kMissAny = INT32_MIN + 1;
 // Searching lanes a wave leaves behind to test its parked leaves: waiting for the last few
 // lanes of a round costs more than another round.
 static constexpr int kDescentTail = 12;
@@ -566,7 +569,7 @@ template <int STACK> __device__ __forceinline__ void stackStart(LaneRay &r, cons
 }
 
 // Makes room: the older half of the LDS entries moves to the spill area.
-template <int STACK> __device__ __forceinline__ LdsInt *stackEvict(LdsInt *sp, const TraceStack ts, int *overflow) {
+template <int STACK, int UNROLL> __device__ __forceinline__ LdsInt *stackEvict(LdsInt *sp, const TraceStack ts, int *overflow) {
     constexpr int kMove = stackEntries(STACK) / 2;
     LdsInt *first = ts.column + kStackFirst * kTraceThreads;
     LdsInt *count = ts.column + stackCountRow(STACK) * kTraceThreads;
@@ -575,7 +578,10 @@ template <int STACK> __device__ __forceinline__ LdsInt *stackEvict(LdsInt *sp, c
         atomicAdd(overflow, 1);
         return first;   // the traversal ends early; the caller of the pass is told
     }
-    for (int k = 0; k < kMove; k++) ts.spill[(size_t)(n + k) * ts.spillStride] = first[k * kTraceThreads];
+    const size_t lanes = gridDim.x * blockDim.x, lane = blockIdx.x * blockDim.x + threadIdx.x;
+    int *spilled = ts.spill + (n * lanes + lane);
+#pragma unroll(UNROLL)
+    for (int k = 0; k < kMove; k++, spilled += lanes) *spilled = first[k * kTraceThreads];
     *count = n + kMove;
     LdsInt *to = first;
     for (LdsInt *from = first + kMove * kTraceThreads; from < sp; from += kTraceThreads, to += kTraceThreads) *to = *from;
@@ -584,13 +590,16 @@ template <int STACK> __device__ __forceinline__ LdsInt *stackEvict(LdsInt *sp, c
 
 // Moves the newest spilled entries back into an empty LDS part; returns its first free entry (the
 // one above the sentinel when nothing was spilled).
-template <int STACK> __device__ __forceinline__ LdsInt *stackRefill(const TraceStack ts) {
+template <int STACK, int UNROLL> __device__ __forceinline__ LdsInt *stackRefill(const TraceStack ts) {
     constexpr int kMove = stackEntries(STACK) / 2;
     LdsInt *first = ts.column + kStackFirst * kTraceThreads;
     LdsInt *count = ts.column + stackCountRow(STACK) * kTraceThreads;
     const int n = *count;
     if (n == 0) return first;
-    for (int k = 0; k < kMove; k++) first[k * kTraceThreads] = ts.spill[(size_t)(n - kMove + k) * ts.spillStride];
+    const size_t lanes = gridDim.x * blockDim.x, lane = blockIdx.x * blockDim.x + threadIdx.x;
+    const int *from = ts.spill + ((n - kMove) * lanes + lane);
+#pragma unroll(UNROLL)
+    for (int k = 0; k < kMove; k++, from += lanes) first[k * kTraceThreads] = *from;
     *count = n - kMove;
     return first + kMove * kTraceThreads;
 }
@@ -603,9 +612,12 @@ template <int STACK> __device__ __forceinline__ LdsInt *stackRefill(const TraceS
 // visited only because its leaf was parked holds no primitive at or below the final tmax, so the
 // hit does not depend on the schedule.  Returns true when the ray is finished: the stack is
 // exhausted, or an any-hit query found an occluder.
-template <bool ANY, int STACK, bool STATS = false, bool TOP = false>
+template <TraceMode MODE, int STACK, bool STATS = false, bool TOP = false>
 __device__ __forceinline__ bool traceRound(const PtSceneView &sc, LaneRay &r, const TraceStack &ts, int *overflow, TraceCount *tc = nullptr,
                                            const LdsChar *top = nullptr) {
+    // the spill code unrolled costs the mixed kernel registers (icosphere 10735 -> 11056 us a pass) and
+    // gains the others a little (room's camera rays 439 -> 422 us)
+    constexpr int kUnroll = MODE == MIXED ? 1 : STACK <= 16 ? 7 : 2;
     const char *nodes = (const char *)sc.nodes;
     int leaf = 0;   // parked leaf reference (< 0), or 0
     if (r.node < 0) {
@@ -621,7 +633,7 @@ __device__ __forceinline__ bool traceRound(const PtSceneView &sc, LaneRay &r, co
         const uint64_t searching = __ballot(leaf == 0 && r.node >= 0);
         if (searching == 0) break;
         if (__popcll(searching) <= kDescentTail && __ballot(leaf != 0) != 0) break;
-        if (ts.spillCap > 0 && r.sp > ts.column + (kStackFirst + stackEntries(STACK) - 1) * kTraceThreads) r.sp = stackEvict<STACK>(r.sp, ts, overflow);
+        if (ts.spillCap > 0 && r.sp > ts.column + (kStackFirst + stackEntries(STACK) - 1) * kTraceThreads) r.sp = stackEvict<STACK, kUnroll>(r.sp, ts, overflow);
         // a lane that parks a leaf in the first step keeps descending internal nodes in the next
         // (as it would while other lanes search) and idles at its second leaf
 #pragma unroll
@@ -715,16 +727,17 @@ __device__ __forceinline__ bool traceRound(const PtSceneView &sc, LaneRay &r, co
                 h = wtHit(r.wr, xyz(p0), xyz(p1), xyz(p2), r.tmin, r.tmax, &t, &u, &v);
             }
             if (h) {
+                const bool done = MODE == ANY || (MODE == MIXED && r.prim == kMissAny);
                 r.tmax = t;
                 r.u = u;
                 r.v = v;
                 r.prim = first + j;
-                if (ANY) return true;
+                if (done) return true;
             }
         }
     }
     if (r.node == kTraceDone && ts.spillCap > 0) {
-        r.sp = stackRefill<STACK>(ts) - kTraceThreads;
+        r.sp = stackRefill<STACK, kUnroll>(ts) - kTraceThreads;
         r.node = *r.sp;
     }
     return r.node == kTraceDone;
@@ -734,8 +747,7 @@ template <int STACK> __device__ __forceinline__ TraceStack traceStack(int *sstac
     TraceStack ts;
     ts.column = (LdsInt *)(sstack + threadIdx.x);
     ts.column[kStackSentinel * kTraceThreads] = kTraceDone;
-    ts.spillStride = gridDim.x * blockDim.x;
-    ts.spill = spill + blockIdx.x * blockDim.x + threadIdx.x;
+    ts.spill = spill;
     ts.spillCap = spillCap;
     return ts;
 }
@@ -790,63 +802,127 @@ __device__ __forceinline__ int segClaim(int *counters, int bounce, int countFiel
     return 0;
 }
 
-// Traces the bounce's queue (count field countField, cursor field fetchField): load(i, o, d,
-// tmin, tmax, root) reads the ray in slot i (root: the BVH node its traversal starts at),
-// finish(i, hit, th) stores its result.  A wave takes new
-// rays once `refill` or more of its lanes are idle, as a contiguous run of one segment so that
-// the rays in flight on a CU stay neighbours, and leaves once its segments are exhausted and
+// Traces queues: claim(want, slot, any) grants up to `want` rays from slot *slot on (0: none left;
+// MIXED: *any says what they look for), load(i, any, o, d, tmin, tmax, root) reads the ray in slot i
+// (root: the BVH node its traversal starts at), finish(i, any, hit, th) stores its result.  A wave
+// takes new rays once `refill` or more of its lanes are idle, as a contiguous run of one segment so
+// that the rays in flight on a CU stay neighbours, and leaves once its segments are exhausted and
 // its lanes idle.
-template <bool ANY, int STACK, bool STATS, bool TOP, class Load, class Finish>
-__device__ __forceinline__ void traceQueue(const PtSceneView &sc, int *counters, int bounce, int countField, int fetchField, int segLen,
-                                           int refill, const TraceStack &ts, const V4 *top, int *overflow, Load load, Finish finish,
-                                           unsigned long long *tstat = nullptr) {
-    SegCursor cur = segStart();
+static constexpr int kNoRay = INT32_MIN;   // an idle lane; else a slot, or ~slot for a MIXED any-hit ray
+template <TraceMode MODE, int STACK, bool STATS, bool TOP, class Claim, class Load, class Finish>
+__device__ __forceinline__ void traceQueue(const PtSceneView &sc, int refill, const TraceStack &ts, const V4 *top, int *overflow, Claim claim, Load load,
+                                           Finish finish, unsigned long long *tstat = nullptr) {
+    bool any = MODE == ANY;
     if (sc.numNodes == 0) {
         TraceHit th;
         th.t = FLT_MAX; th.u = 0.f; th.v = 0.f; th.prim = INT32_MIN;
         int slot = 0, got;
-        while ((got = segClaim(counters, bounce, countField, fetchField, segLen, 64, cur, &slot)) > 0)
-            if (laneId() < got) finish(slot + laneId(), false, th);
+        while ((got = claim(64, &slot, &any)) > 0)
+            if (laneId() < got) finish(slot + laneId(), any, false, th);
         return;
     }
     LaneRay r;
-    int ray = -1;
+    int ray = kNoRay;
+    bool more = true;   // wave-uniform
     TraceCount tc;
     while (true) {
-        const uint64_t idle = __ballot(ray < 0);
-        if (cur.left > 0 && __popcll(idle) >= refill) {
+        const uint64_t idle = __ballot(ray == kNoRay);
+        if (more && __popcll(idle) >= refill) {
             int slot = 0;
-            const int got = segClaim(counters, bounce, countField, fetchField, segLen, __popcll(idle), cur, &slot);
-            if (ray < 0) {
+            const int got = claim(__popcll(idle), &slot, &any);
+            more = got > 0;
+            if (ray == kNoRay) {
                 const int k = (int)lanesBelow(idle);
                 if (k < got) {
-                    ray = slot + k;
+                    ray = MODE == MIXED && any ? ~(slot + k) : slot + k;
                     f3 o, d;
                     float tmin, tmax;
                     int root = 0;
-                    load(ray, o, d, tmin, tmax, root);
+                    load(slot + k, any, o, d, tmin, tmax, root);
                     laneRayStart(r, o, d, tmin, tmax, root);
+                    if (MODE == MIXED && any) r.prim = kMissAny;
                     stackStart<STACK>(r, ts);
                     if constexpr (STATS) tc.rays++;
                 }
             }
         }
         // all lanes idle after a refill attempt means this wave's segments are exhausted
-        if (__ballot(ray >= 0) == 0) break;
-        if (ray >= 0 && traceRound<ANY, STACK, STATS, TOP>(sc, r, ts, overflow, &tc, (const LdsChar *)top)) {
-            finish(ray, r.prim >= 0, laneRayHit(r));
-            ray = -1;
+        if (__ballot(ray != kNoRay) == 0) break;
+        if (ray != kNoRay && traceRound<MODE, STACK, STATS, TOP>(sc, r, ts, overflow, &tc, (const LdsChar *)top)) {
+            const bool mineAny = MODE == ANY || (MODE == MIXED && ray < 0);
+            finish(MODE == MIXED && ray < 0 ? ~ray : ray, mineAny, r.prim >= 0, laneRayHit(r));
+            ray = kNoRay;
         }
     }
     if constexpr (STATS) addTraceCount(tc, tstat);
 }
 
-// Persistent closest-hit kernel over the rays of `bounce`.  camO.w != 0: the rays start at
-// camO (camera rays, tmin 0) and rayO is not read.  BATCH (a batch wavefront): the traversal
-// starts at the root node of the ray's render; at bounce 0 the render comes from the path
-// index (chunk groups) and the origin is its camera's, later rayO.w holds the render.
-// STATS: the instrumented build that adds its rays, node visits and primitive tests to
-// tstat[0..2].
+// A bounce's extension rays: camO.w != 0: they start at camO (camera rays, tmin 0) and rayO is not
+// read.  BATCH (a batch wavefront): the traversal starts at the root node of the ray's render; at
+// bounce 0 the render comes from the path index (chunk groups) and the origin is its camera's,
+// later rayO.w holds the render.
+template <bool BATCH> struct ExtendRays {
+    const float4 *rayO, *rayD;
+    float4 camO;
+    float4 *hits;
+    int bounce, segLen;
+    __device__ __forceinline__ void load(const ChunkParams &cp, int i, f3 &o, f3 &d, float &tmin, float &tmax, int &root) const {
+        const float4 rd = rayD[i];
+        if constexpr (BATCH) {
+            if (bounce == 0) {
+                int off;
+                const int seg = divmodEst(i, segLen, &off);
+                const int p = ptCameraPath(seg, off);
+                const BatchRender &R = cp.renders[batchRenderOf(cp, p)];
+                o = xyz(batchCameraOrigin(R));
+                tmin = 0.f;
+                root = R.root;
+            } else {
+                const float4 ro = rayO[i];
+                o = xyz(ro);
+                tmin = kBounceEps;
+                root = cp.renders[asInt(ro.w)].root;
+            }
+        } else if (camO.w != 0.f) {
+            o = xyz(camO);
+            tmin = 0.f;
+        } else {
+            const float4 ro = rayO[i];
+            o = xyz(ro);
+            tmin = ro.w;
+        }
+        d = xyz(rd);
+        tmax = rd.w;
+    }
+    __device__ __forceinline__ void store(int i, const TraceHit &th) const { hits[i] = make_float4(th.t, th.u, th.v, asFloat(th.prim)); }
+};
+
+// A bounce's shadow rays (interval [1e-4, tmax]); an unoccluded one adds its light contribution to
+// its path.  path: the lane's path index, kept from the ray's load (a re-read after the traversal
+// would be a dependent round trip ahead of the radiance update).  BATCH: sL.w holds the ray's
+// render, whose root node starts the traversal.
+template <bool BATCH> struct ShadowRays {
+    const float4 *sO, *sD, *sL;
+    float4 *Lpath;
+    __device__ __forceinline__ void load(const BatchRender *renders, int *path, int i, f3 &o, f3 &d, float &tmin, float &tmax, int &root) const {
+        const float4 so = sO[i], sd = sD[i];
+        o = xyz(so);
+        d = xyz(sd);
+        tmin = kShadowEps;
+        tmax = so.w;
+        *path = asInt(sd.w);
+        if constexpr (BATCH) root = renders[asInt(((const float *)&sL[i])[3])].root;
+    }
+    __device__ __forceinline__ void add(const int *path, int i) const {
+        const float4 l = sL[i];
+        float4 acc = Lpath[*path];
+        acc.x += l.x; acc.y += l.y; acc.z += l.z;
+        Lpath[*path] = acc;
+    }
+};
+
+// Persistent closest-hit kernel over the rays of `bounce`.  STATS: the instrumented build that adds
+// its rays, node visits and primitive tests to tstat[0..2].
 template <int STACK, bool BATCH = false, bool STATS = false>
 __global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_extend(PtSceneView sc, int *counters, int bounce, int segLen,
                                                                               const float4 *rayO, const float4 *rayD, float4 camO, float4 *hits,
@@ -856,37 +932,13 @@ __global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_extend(P
     __shared__ V4 top[BATCH ? 1 : kTopNodes * PT_NODE_F4];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
     if constexpr (!BATCH) loadTopNodes(top, sc);
-    traceQueue<false, STACK, STATS, !BATCH>(
-        sc, counters, bounce, PT_Q_RAYS, PT_Q_FETCH_EXT, segLen, refill, ts, top, overflow,
-        [&](int i, f3 &o, f3 &d, float &tmin, float &tmax, int &root) {
-            const float4 rd = rayD[i];
-            if constexpr (BATCH) {
-                if (bounce == 0) {
-                    int off;
-                    const int seg = divmodEst(i, segLen, &off);
-                    const int p = ptCameraPath(seg, off);
-                    const BatchRender &R = cp.renders[batchRenderOf(cp, p)];
-                    o = xyz(batchCameraOrigin(R));
-                    tmin = 0.f;
-                    root = R.root;
-                } else {
-                    const float4 ro = rayO[i];
-                    o = xyz(ro);
-                    tmin = kBounceEps;
-                    root = cp.renders[asInt(ro.w)].root;
-                }
-            } else if (camO.w != 0.f) {
-                o = xyz(camO);
-                tmin = 0.f;
-            } else {
-                const float4 ro = rayO[i];
-                o = xyz(ro);
-                tmin = ro.w;
-            }
-            d = xyz(rd);
-            tmax = rd.w;
-        },
-        [&](int i, bool, const TraceHit &th) { hits[i] = make_float4(th.t, th.u, th.v, asFloat(th.prim)); }, tstat);
+    const ExtendRays<BATCH> ext{rayO, rayD, camO, hits, bounce, segLen};
+    SegCursor cur = segStart();
+    traceQueue<CLOSEST, STACK, STATS, !BATCH>(
+        sc, refill, ts, top, overflow,
+        [&](int want, int *slot, bool *) { return segClaim(counters, bounce, PT_Q_RAYS, PT_Q_FETCH_EXT, segLen, want, cur, slot); },
+        [&](int i, bool, f3 &o, f3 &d, float &tmin, float &tmax, int &root) { ext.load(cp, i, o, d, tmin, tmax, root); },
+        [&](int i, bool, bool, const TraceHit &th) { ext.store(i, th); }, tstat);
 }
 
 // Wave stack entries of the packet traversal (one per lane of a register), and its blocks per CU.
@@ -1047,9 +1099,7 @@ __global__ __launch_bounds__(kTraceThreads, 8) void k_extend_packet(PtSceneView 
     }
 }
 
-// Persistent any-hit kernel for the shadow rays of `bounce` (interval [1e-4, tmax]); an
-// unoccluded ray adds its light contribution to its path.
-// BATCH: sL.w holds the ray's render, whose root node starts the traversal.
+// Persistent any-hit kernel for the shadow rays of `bounce`.
 template <int STACK, bool BATCH = false, bool STATS = false>
 __global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_shadow(PtSceneView sc, int *counters, int bounce, int segLen,
                                                                               const float4 *sO, const float4 *sD, const float4 *sL, float4 *Lpath,
@@ -1057,35 +1107,71 @@ __global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_shadow(P
                                                                               const BatchRender *renders = nullptr, unsigned long long *tstat = nullptr) {
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
     __shared__ V4 top[BATCH ? 1 : kTopNodes * PT_NODE_F4];
-    // each lane's path index, kept from the ray's load (a re-read after the traversal would be a
-    // dependent round trip ahead of the radiance update)
     __shared__ int sPath[kTraceThreads];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
     if constexpr (!BATCH) loadTopNodes(top, sc);
+    const ShadowRays<BATCH> sh{sO, sD, sL, Lpath};
+    int *path = sPath + threadIdx.x;
     int adds = 0;
-    traceQueue<true, STACK, STATS, !BATCH>(
-        sc, counters, bounce, PT_Q_SHADOW, PT_Q_FETCH_SHADOW, segLen, refill, ts, top, overflow,
-        [&](int i, f3 &o, f3 &d, float &tmin, float &tmax, int &root) {
-            const float4 so = sO[i], sd = sD[i];
-            o = xyz(so);
-            d = xyz(sd);
-            tmin = kShadowEps;
-            tmax = so.w;
-            sPath[threadIdx.x] = asInt(sd.w);
-            if constexpr (BATCH) root = renders[asInt(((const float *)&sL[i])[3])].root;
-        },
-        [&](int i, bool occluded, const TraceHit &) {
+    SegCursor cur = segStart();
+    traceQueue<ANY, STACK, STATS, !BATCH>(
+        sc, refill, ts, top, overflow,
+        [&](int want, int *slot, bool *) { return segClaim(counters, bounce, PT_Q_SHADOW, PT_Q_FETCH_SHADOW, segLen, want, cur, slot); },
+        [&](int i, bool, f3 &o, f3 &d, float &tmin, float &tmax, int &root) { sh.load(renders, path, i, o, d, tmin, tmax, root); },
+        [&](int i, bool, bool occluded, const TraceHit &) {
             if (!occluded) {
-                const int pid = sPath[threadIdx.x];
-                const float4 l = sL[i];
-                float4 acc = Lpath[pid];
-                acc.x += l.x; acc.y += l.y; acc.z += l.z;
-                Lpath[pid] = acc;
+                sh.add(path, i);
                 adds++;
             }
         },
         tstat);
     waveSum(adds, &counters[ptQueueField(homeSegment(), bounce, PT_Q_LADD_SHADOW)]);
+}
+
+// The shadow rays of a bounce and the next bounce's extension rays, both made by the bounce's
+// shading, in one launch: lanes take extension rays while there are any and shadow rays after
+// them, side by side in a wave.  A launch lasts as
+// long as its longest ray: at 2^19 to 2^21 paths half of one, and at the late bounces of any pass all
+// of it; together the queues' tails are waited for once and each fills the other's idle lanes.
+// Extension and shadow kernels of a pass, apart / together: room of 4M triangles, 2^21 paths, depth 16:
+// 9473 / 7945 us; guided room, 2^19 paths: 3720 / 2412; 1.31M triangles, 2^26 paths, depth 8: 11225 /
+// 10735 (its first bounce alone, where nothing waits, 9325 / 9407); batch of 12, 1.5e7 paths:
+// 4197 / 3808.
+template <int STACK, bool BATCH = false>
+__global__ __launch_bounds__(kTraceThreads, STACK <= 16 ? 6 : 3) void k_trace(PtSceneView sc, int *counters, int bounce, int segLen, const float4 *rayO,
+                                                                             const float4 *rayD, float4 *hits, const float4 *sO, const float4 *sD,
+                                                                             const float4 *sL, float4 *Lpath, int refill, int *spill, int spillCap,
+                                                                             int *overflow, ChunkParams cp) {
+    __shared__ int sstack[stackRows(STACK) * kTraceThreads];
+    __shared__ V4 top[BATCH ? 1 : kTopNodes * PT_NODE_F4];
+    __shared__ int sPath[kTraceThreads];
+    __shared__ int sAdds[kTraceThreads / 64];   // (a register more per lane would spill others)
+    const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
+    if constexpr (!BATCH) loadTopNodes(top, sc);
+    const ExtendRays<BATCH> ext{rayO, rayD, make_float4(0.f, 0.f, 0.f, 0.f), hits, bounce + 1, segLen};
+    const ShadowRays<BATCH> sh{sO, sD, sL, Lpath};
+    int *path = sPath + threadIdx.x;
+    if (laneId() == 0) sAdds[threadIdx.x >> 6] = 0;
+    SegCursor curExt = segStart(), curSh = segStart();
+    traceQueue<MIXED, STACK, false, !BATCH>(
+        sc, refill, ts, top, overflow,
+        [&](int want, int *slot, bool *any) {
+            const int got = segClaim(counters, bounce + 1, PT_Q_RAYS, PT_Q_FETCH_EXT, segLen, want, curExt, slot);
+            *any = got == 0;
+            return got > 0 ? got : segClaim(counters, bounce, PT_Q_SHADOW, PT_Q_FETCH_SHADOW, segLen, want, curSh, slot);
+        },
+        [&](int i, bool any, f3 &o, f3 &d, float &tmin, float &tmax, int &root) {
+            if (any) sh.load(cp.renders, path, i, o, d, tmin, tmax, root);
+            else ext.load(cp, i, o, d, tmin, tmax, root);
+        },
+        [&](int i, bool any, bool hit, const TraceHit &th) {
+            if (!any) ext.store(i, th);
+            else if (!hit) {
+                sh.add(path, i);
+                atomicAdd(&sAdds[threadIdx.x >> 6], 1);
+            }
+        });
+    if (laneId() == 0 && sAdds[threadIdx.x >> 6] != 0) atomicAdd(&counters[ptQueueField(homeSegment(), bounce, PT_Q_LADD_SHADOW)], sAdds[threadIdx.x >> 6]);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1570,7 +1656,7 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
 
 // Traces every active lane's ray to its end (lanes of a wave that wait for the longest ray idle:
 // nothing refills them here).
-template <bool ANY, int STACK, bool STATS = false>
+template <TraceMode MODE, int STACK, bool STATS = false>
 __device__ __forceinline__ void traceLanes(const PtSceneView &sc, LaneRay &r, bool active, f3 o, f3 d, float tmin, float tmax, const TraceStack &ts,
                                            int *overflow, TraceCount *tc = nullptr) {
     r.prim = INT32_MIN;
@@ -1581,7 +1667,7 @@ __device__ __forceinline__ void traceLanes(const PtSceneView &sc, LaneRay &r, bo
         if constexpr (STATS) tc->rays++;
     }
     while (__ballot(busy) != 0)
-        if (busy) busy = !traceRound<ANY, STACK, STATS>(sc, r, ts, overflow, tc);
+        if (busy) busy = !traceRound<MODE, STACK, STATS>(sc, r, ts, overflow, tc);
 }
 
 // What a chunk's accumulation does beside adding to the FP64 sums.
@@ -1646,7 +1732,7 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, Chun
         for (int depth = 0; depth < cp.maxDepth && __ballot(alive) != 0; depth++) {
             tally(0, depth, alive);
             LaneRay r;
-            traceLanes<false, STACK>(sc, r, alive, o, d, depth == 0 ? 0.f : kBounceEps, FLT_MAX, ts, overflow);
+            traceLanes<CLOSEST, STACK>(sc, r, alive, o, d, depth == 0 ? 0.f : kBounceEps, FLT_MAX, ts, overflow);
             bool addL = false, pushRay = false, pushShadow = false;
             f3 p = mk(0.f), contrib = mk(0.f), lightDir = mk(0.f), next = mk(0.f), nb = mk(0.f);
             float lightDist = 0.f, nextPdf = -1.f;
@@ -1684,7 +1770,7 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, Chun
             tally(2, depth, addL);
             if (cp.nee) {
                 tally(1, depth, pushShadow);
-                traceLanes<true, STACK>(sc, r, pushShadow, p, lightDir, kShadowEps, lightDist - 2e-4f, ts, overflow);
+                traceLanes<ANY, STACK>(sc, r, pushShadow, p, lightDir, kShadowEps, lightDist - 2e-4f, ts, overflow);
                 const bool lit = pushShadow && r.prim == INT32_MIN;
                 if (lit) acc = acc + contrib;
                 tally(3, depth, lit);
@@ -1721,7 +1807,7 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_normals(PtSceneView sc, Pt
         f3 o, d;
         cameraRay(cam, row, col, 0.5f, 0.5f, &o, &d);
         LaneRay r;
-        traceLanes<false, STACK, STATS>(sc, r, mine, o, d, 0.f, FLT_MAX, ts, overflow, &tc);
+        traceLanes<CLOSEST, STACK, STATS>(sc, r, mine, o, d, 0.f, FLT_MAX, ts, overflow, &tc);
         if (!mine) continue;
         f3 c = mk(0.f);
         if (r.prim != INT32_MIN) {
@@ -1751,7 +1837,7 @@ __global__ __launch_bounds__(64) void k_pick(PtSceneView sc, float4 o, float4 d,
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
     LaneRay r;
-    traceLanes<false, STACK>(sc, r, threadIdx.x == 0, xyz(o), xyz(d), o.w, d.w, ts, overflow);
+    traceLanes<CLOSEST, STACK>(sc, r, threadIdx.x == 0, xyz(o), xyz(d), o.w, d.w, ts, overflow);
     if (threadIdx.x == 0) *out = r.prim == INT32_MIN ? -1 : asInt(sc.prims[3 * (size_t)r.prim].w);
 }
 
@@ -2276,6 +2362,21 @@ void launchShadow(pt_renderer *r, int bounce, int segLen) {
     PT_HIP_TRY(hipGetLastError());
 }
 
+// Shadow rays of `bounce` and extension rays of the bounce after it.
+void launchTrace(pt_renderer *r, int bounce, int segLen, const float4 *ro, const float4 *rd, const ChunkParams &cp) {
+    const int refill = refillLanes(r, TRACE_INCOHERENT);
+    const int grid = traceGrid(r);
+    int *ctr = r->pp->counters.as<int>(), *ov = r->pp->overflow.as<int>();
+    const float4 *o = r->pp->sO.as<float4>(), *d = r->pp->sD.as<float4>(), *l = r->pp->sL.as<float4>();
+    float4 *L = r->pp->Lpath.as<float4>(), *hits = r->pp->hits.as<float4>();
+    int cap = 0;
+    int *sp = ensureSpill(r, grid, &cap);
+    auto run = [&](auto kernel) { kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, ctr, bounce, segLen, ro, rd, hits, o, d, l, L, refill, sp, cap, ov, cp); };
+    if (cp.renders) r->ldsStack == 32 ? run(k_trace<32, true>) : run(k_trace<16, true>);
+    else r->ldsStack == 32 ? run(k_trace<32>) : run(k_trace<16>);
+    PT_HIP_TRY(hipGetLastError());
+}
+
 // Clears the queue counters and describes a linear queue of n records (slots 0 .. n - 1) in
 // field `field` of bounce 0; its segment length is ptSegLen(n).
 void queueLinear(pt_renderer *r, int field, int n) {
@@ -2385,9 +2486,11 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
     const float4 camO = make_float4(r->cam.m[0][3], r->cam.m[1][3], r->cam.m[2][3], 1.f);
     const float4 noCam = make_float4(0.f, 0.f, 0.f, 0.f);
     int cur = 0;
+    // timed and counting kernels run by themselves
+    const bool merged = cp.nee && !r->profile && !r->traceStats;
     for (int b = 0; b < cp.maxDepth; b++) {
         const float4 bo = b == 0 ? camO : noCam;
-        {
+        if (b == 0 || !merged) {
             KTimer t(r, K_EXTEND);
             // camera runs of one pixel's samples, or of a few neighbouring pixels' (pixel-major
             // chunks of 16 sample rows or more): one traversal per run.  Runs of 64 pixels of a
@@ -2429,11 +2532,14 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
                     r->pp->beta[1 - cur].as<float4>(), r->pp->sO.as<float4>(), r->pp->sD.as<float4>(), r->pp->sL.as<float4>(), r->pp->Lpath.as<float4>(), ga, bo);
             PT_HIP_TRY(hipGetLastError());
         }
-        if (cp.nee) {
+        cur = 1 - cur;
+        if (merged) {
+            // (the last bounce's vertices spawn no rays)
+            if (b + 1 < cp.maxDepth) launchTrace(r, b, cp.segLen, r->pp->rayO[cur].as<float4>(), r->pp->rayD[cur].as<float4>(), cp);
+        } else if (cp.nee) {
             KTimer t(r, K_SHADOW);
             launchShadow(r, b, cp.segLen);
         }
-        cur = 1 - cur;
     }
     accumulateChunk(r, cp, false, end);
     if (guided && r->gTrainSteps > 0) {
@@ -3620,6 +3726,8 @@ void planWave(pt_batch *b, int scale) {
     }
 }
 
+constexpr int kMergedBatchPaths = 1 << 17;
+
 // One chunk of the batch wavefront: raygen from every group's camera, the bounces with the
 // batch kernels, accumulation into each render's accumulator.  A chunk that holds sample rows
 // of one render only (the large renders) runs that render's own kernels instead, exactly its
@@ -3655,9 +3763,14 @@ void runWaveChunk(pt_batch *b, const WaveChunk &c) {
     PT_HIP_TRY(hipGetLastError());
     const int shadeGrid = (int)std::max<int64_t>(PT_QUEUE_SEGS / 4, std::min<int64_t>((cp.nPaths + 255) / 256, (int64_t)w->cus * w->shadeBlocksPerCU));
     int cur = 0;
+    // One launch for a bounce's shadow rays and the next one's extension rays (k_trace), as in a
+    // render's own chunks; small batches, which would gain too, keep a launch per queue: their
+    // callers see the number of graph nodes (pt_batch_stats) and count on the kernels being there.
+    const bool merged = cp.nee && cp.nPaths >= kMergedBatchPaths;
     for (int bn = 0; bn < cp.maxDepth; bn++) {
-        launchExtend(w, bn, cp.segLen, pp.rayO[cur].as<float4>(), pp.rayD[cur].as<float4>(), pp.hits.as<float4>(),
-                     bn == 0 ? TRACE_CAMERA : TRACE_INCOHERENT, make_float4(0.f, 0.f, 0.f, 0.f), &cp);
+        if (bn == 0 || !merged)
+            launchExtend(w, bn, cp.segLen, pp.rayO[cur].as<float4>(), pp.rayD[cur].as<float4>(), pp.hits.as<float4>(),
+                         bn == 0 ? TRACE_CAMERA : TRACE_INCOHERENT, make_float4(0.f, 0.f, 0.f, 0.f), &cp);
         // w = 1 marks bounce 0 (camera vertices); batch kernels take each render's camera
         const float4 camFlag = make_float4(0.f, 0.f, 0.f, bn == 0 ? 1.f : 0.f);
         k_shade<false, true><<<shadeGrid, 256, 0, b->stream>>>(
@@ -3666,8 +3779,9 @@ void runWaveChunk(pt_batch *b, const WaveChunk &c) {
             pp.beta[1 - cur].as<float4>(), pp.sO.as<float4>(), pp.sD.as<float4>(), pp.sL.as<float4>(), pp.Lpath.as<float4>(), GuideShadeArgs{},
             camFlag);
         PT_HIP_TRY(hipGetLastError());
-        if (cp.nee) launchShadow(w, bn, cp.segLen);
         cur = 1 - cur;
+        if (!merged && cp.nee) launchShadow(w, bn, cp.segLen);
+        if (merged && bn + 1 < cp.maxDepth) launchTrace(w, bn, cp.segLen, pp.rayO[cur].as<float4>(), pp.rayD[cur].as<float4>(), cp);
     }
     k_accumulate_batch<<<(c.accThreads + 255) / 256, 256, 0, b->stream>>>(cp, c.accThreads, pp.Lpath.as<float4>(), ctr,
                                                                           b->waveStats.as<unsigned long long>());
