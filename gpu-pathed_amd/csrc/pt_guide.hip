@@ -407,6 +407,12 @@ __device__ float lossGradientQ(const float *v, f3 w, float pb, float wt, int g, 
     return g == 0 ? -wt * (__logf(qq) + __logf(mix)) : 0.f;
 }
 
+// A lane's pair of features of its record, and its neighbour lane's, as one feature of both records.
+__device__ __forceinline__ uint32_t pairRows(uint32_t own, uint32_t pick) {
+    const uint32_t other = __builtin_amdgcn_mov_dpp(own, 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true);
+    return __builtin_amdgcn_perm(own, other, pick);
+}
+
 // Training step in one kernel: blocks of eight waves, persistent over iterations of
 // GUIDE_TRAIN_ROWS records (16 rows per wave).  Per iteration each wave runs the forward pass
 // of its rows with the activations in registers (as inference), the loss gradient at the
@@ -419,6 +425,10 @@ __device__ float lossGradientQ(const float *v, f3 w, float pb, float wt, int g, 
 // delta fragments.  Each block keeps its gradient in registers across iterations and writes it
 // once as a partial, summed in block order by k_guide_reduce: the result does not depend on
 // scheduling.  Rows past the batch get weight 0 and so zero deltas.
+// Bound by VALU issue and the matrix cores together (52% and about 30% of the cycles, two waves per
+// SIMD between barriers): 2^18 records 92.8 us with each iteration's record search and load at its
+// start and 16-bit transposing stores, 84.0 with the records loaded an iteration ahead and paired
+// stores; 16 waves a block over two tiles 97 (more fragment reads, spills).
 constexpr int TRAIN_WAVES = 8;
 constexpr int TRAIN_TILE = 16;                        // rows per wave per iteration
 constexpr int FM_PITCH = GUIDE_TRAIN_ROWS + 8;        // bf16 per feature of a feature-major tile
@@ -438,6 +448,7 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_guide_train(GuideNet net, 
     __shared__ float4 sB[GUIDE_LAYERS * GUIDE_W / 4];
     __shared__ float4 sRec[TRAIN_WAVES][TRAIN_TILE][GUIDE_TREC_F4];
     __shared__ float sLoss[TRAIN_WAVES];
+    __shared__ int sPrefix[PT_QUEUE_SEGS];
     __shared__ __align__(16) TrainGradLds gs;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = lane >> 4, lr = lane & 15;
@@ -445,6 +456,7 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_guide_train(GuideNet net, 
     for (int c = threadIdx.x; c < GUIDE_LAYERS * 8 * 64; c += blockDim.x) sWf[c] = ld8(net.w + 8 * (size_t)c);
     for (int c = threadIdx.x; c < (GUIDE_LAYERS - 1) * 8 * 64; c += blockDim.x) sWb[c] = ld8(net.wt + 8 * (size_t)(8 * 64 + c));
     stageBiases(net.b, (float *)sB);
+    if (prefix && threadIdx.x < PT_QUEUE_SEGS) sPrefix[threadIdx.x] = prefix[threadIdx.x];
     __syncthreads();
     const int count = *countPtr;
     const float wsum = wsumPtr ? *wsumPtr : 0.f;
@@ -457,31 +469,36 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_guide_train(GuideNet net, 
         db[L] = 0.f;
         dW[L][0] = dW[L][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    const uint32_t pick = lane & 1 ? 0x07060302u : 0x01000504u;   // pairRows: the odd lane's halves, or the even lane's
     float lossAcc = 0.f;
     const int iters = (batch + GUIDE_TRAIN_ROWS - 1) / GUIDE_TRAIN_ROWS;
-    for (int it = blockIdx.x; it < iters; it += gridDim.x) {
-        {
-            // the tile's records: lane (g, lr) loads float4 g of row lr
-            const int r = it * GUIDE_TRAIN_ROWS + wave * TRAIN_TILE + lr;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (r < batch && count > 0) {
-                const int vi = (int)(((int64_t)base + r) % count);
-                size_t idx = (size_t)vi;
-                if (prefix) {
-                    // the last segment whose prefix does not exceed vi holds record vi
-                    int lo = 0, hi = PT_QUEUE_SEGS;
-                    while (hi - lo > 1) {
-                        const int mid = (lo + hi) >> 1;
-                        if (prefix[mid] <= vi) lo = mid;
-                        else hi = mid;
-                    }
-                    idx = (size_t)lo * recSeg + (vi - prefix[lo]);
+    // lane (g, lr)'s float4 of the tile of iteration `it`: float4 g of row lr's record
+    auto loadRecord = [&](int it) {
+        const int r = it * GUIDE_TRAIN_ROWS + wave * TRAIN_TILE + lr;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (r < batch && count > 0) {
+            const int vi = (int)(((uint32_t)base + (uint32_t)r) % (uint32_t)count);
+            size_t idx = (size_t)vi;
+            if (prefix) {
+                // the last segment whose prefix does not exceed vi holds record vi
+                int lo = 0, hi = PT_QUEUE_SEGS;
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (sPrefix[mid] <= vi) lo = mid;
+                    else hi = mid;
                 }
-                v = recs[idx * GUIDE_TREC_F4 + g];
-                if (g == 3) v.w = fminf(v.w * wscale, 64.f);
+                idx = (size_t)lo * recSeg + (vi - sPrefix[lo]);
             }
-            sRec[wave][lr][g] = v;
+            v = recs[idx * GUIDE_TREC_F4 + g];
+            if (g == 3) v.w = fminf(v.w * wscale, 64.f);
         }
+        return v;
+    };
+    // each iteration's records are loaded during the one before
+    float4 next = loadRecord(blockIdx.x);
+    for (int it = blockIdx.x; it < iters; it += gridDim.x) {
+        sRec[wave][lr][g] = next;
+        if (it + (int)gridDim.x < iters) next = loadRecord(it + gridDim.x);
         WAVE_SYNC();
         // forward; act[L] = the input of layer L as B fragments [K step]
         bf16x8 act[GUIDE_LAYERS][2];
@@ -549,13 +566,15 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_guide_train(GuideNet net, 
         }
 #pragma unroll
         for (int L = GUIDE_LAYERS - 1; L >= 0; L--) {
+            // feature-major, two records a store: neighbouring lanes (records) exchange halves, the
+            // even one writes the pair's feature p, the odd one p + 1
 #pragma unroll
             for (int ks = 0; ks < 2; ks++)
 #pragma unroll
-                for (int p = 0; p < 8; p++) {
-                    const int kf = kFeature(g, p, ks), col = wave * TRAIN_TILE + lr;
-                    gs.a[kf][col] = act[L][ks][p];
-                    gs.d[kf][col] = dl[ks][p];
+                for (int h = 0; h < 4; h++) {
+                    const int kf = kFeature(g, 2 * h, ks) + (lr & 1), col = wave * TRAIN_TILE + (lr & ~1);
+                    *(uint32_t *)&gs.a[kf][col] = pairRows(__builtin_bit_cast(u32x4, act[L][ks])[h], pick);
+                    *(uint32_t *)&gs.d[kf][col] = pairRows(__builtin_bit_cast(u32x4, dl[ks])[h], pick);
                 }
             if (L > 0) {
                 // delta of layer L - 1's outputs: W_L^T delta_L, masked by ReLU'
