@@ -2499,12 +2499,16 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
         const float4 bo = b == 0 ? camO : noCam;
         if (b == 0 || !merged) {
             KTimer t(r, K_EXTEND);
-            // camera runs of one pixel's samples, or of a few neighbouring pixels' (pixel-major
-            // chunks of 16 sample rows or more): one traversal per run.  Runs of 64 pixels of a
-            // row (one sample row) trace faster per lane (the room at 1 spp: 3444 against 3254
-            // Mrays/s); the 48-render batch gains 0.5% from 16 rows against 64.
+            // Camera runs of one pixel's samples, or of a few neighbouring pixels' (pixel-major
+            // chunks of 16 sample rows or more), in scenes of few primitives per run's pixels: one
+            // traversal per run.  Camera bounce per lane / as packets, us: 1.31M triangles at 1024^2,
+            // 2, 4, 8, 16 samples (40 to 5 primitives a run): 402 / 738, 595 / 789, 928 / 928, 1597 /
+            // 1163; rooms differ: 100k at 1024^2, 8, 32 samples: 382 / 689, 899 / 723.  Passes: 1.31M
+            // triangles at 256^2, 64 samples (20 a run) 2490 / 2431, at 300 x 200, 48 samples (29)
+            // 1792 / 1973; room of 4M at 512 x 256, 32 samples (61) 15937 / 16289.
             const bool packet = b == 0 && cp.pixelMajor && cp.samples >= 16 && !r->traceStats && r->view.numNodes > 0 &&
-                                r->stackNeed <= kPacketStack && r->packetCamera;
+                                r->stackNeed <= kPacketStack && r->packetCamera &&
+                                (int64_t)r->view.numPrims * 64 <= 20 * (int64_t)cp.samples * r->W * r->H;
             launchExtend(r, b, cp.segLen, r->pp->rayO[cur].as<float4>(), r->pp->rayD[cur].as<float4>(), r->pp->hits.as<float4>(),
                          b == 0 ? TRACE_CAMERA : TRACE_INCOHERENT, bo, nullptr, packet);
         }
