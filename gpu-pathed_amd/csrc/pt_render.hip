@@ -1699,8 +1699,8 @@ __device__ __forceinline__ void writePixel(const double a[3], double invSpp, int
 }
 
 // A small chunk's paths from the camera to their end in one launch: a wave takes 64 paths and
-// alternates between tracing its lanes' rays, shading their hits and tracing their shadow rays,
-// with the path state in registers.  The arithmetic is the queue kernels' own, step by step, so a
+// alternates between shading its lanes' hits and tracing the shadow rays this made together with the
+// next extension rays (traceBoth), with the path state in registers.  The arithmetic is the queue kernels' own, step by step, so a
 // path's radiance is theirs bit for bit.
 //
 // The queue kernels need their queues long: each launch lasts at least as long as its longest ray
@@ -1712,11 +1712,74 @@ __device__ __forceinline__ void writePixel(const double a[3], double invSpp, int
 // different depths spilled more state than they filled idle time), nor did 8 x 8 pixel tiles
 // instead of 64 pixels of a row (327k triangles at 1024^2 882 -> 923 us, at 256^2 306 -> 289).
 static constexpr int kPathBlocksPerCU = 8;   // of two waves: four waves per SIMD
+// A wave's shadow rays of a bounce and what came of them.
+struct ShadowList {
+    float o[3][64], d[3][64], tmax[64], contrib[3][64];
+    int hit[64];
+    __device__ __forceinline__ void put(int k, f3 from, f3 dir, float dist, f3 c) {
+        o[0][k] = from.x; o[1][k] = from.y; o[2][k] = from.z;
+        d[0][k] = dir.x; d[1][k] = dir.y; d[2][k] = dir.z;
+        tmax[k] = dist;
+        contrib[0][k] = c.x; contrib[1][k] = c.y; contrib[2][k] = c.z;
+        hit[k] = 0;
+    }
+};
+
+// The lanes' extension rays (of those alive) and the wave's shadow rays, together: lanes without a
+// ray, or done with their own, take the next shadow rays of the list once kShadowRefill of them can,
+// so the wave waits once a bounce, and lanes whose path has ended work too.  us, shadow rays traced by
+// their paths' lanes after the extension rays / together from 1, 16, 32 lanes on: 327k triangles at
+// 641 x 359 320 / 278, 282, 282; 1.31M at 256^2 400 / 331, 336, 341; Cornell box at 256^2, 16 samples
+// (bound by VALU issue) 356 / 352, 349, 343.
+static constexpr int kShadowRefill = 32;
 template <int STACK>
+__device__ __forceinline__ TraceHit traceBoth(const PtSceneView &sc, bool alive, f3 o, f3 d, float tmin, ShadowList &sh, int shadows, const TraceStack &ts,
+                                              int *overflow) {
+    TraceHit h;
+    h.t = FLT_MAX; h.u = 0.f; h.v = 0.f; h.prim = INT32_MIN;
+    if (sc.numNodes == 0) return h;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    constexpr int kOwn = 64;
+    LaneRay r;
+    int job = kNoRay;   // kOwn: the lane's extension ray; else a shadow ray
+    if (alive) {
+        laneRayStart(r, o, d, tmin, FLT_MAX);
+        stackStart<STACK>(r, ts);
+        job = kOwn;
+    }
+    int taken = 0;
+    while (true) {
+        const uint64_t idle = __ballot(job == kNoRay);
+        if (taken < shadows && __popcll(idle) >= kShadowRefill) {
+            const int k = taken + (int)lanesBelow(idle);
+            if (job == kNoRay && k < shadows) {
+                job = k;
+                laneRayStart(r, mk(sh.o[0][k], sh.o[1][k], sh.o[2][k]), mk(sh.d[0][k], sh.d[1][k], sh.d[2][k]), kShadowEps, sh.tmax[k]);
+                r.prim = kMissAny;
+                stackStart<STACK>(r, ts);
+            }
+            taken = min(shadows, taken + __popcll(idle));
+        }
+        if (__ballot(job != kNoRay) == 0) break;
+        if (job != kNoRay && traceRound<MIXED, STACK>(sc, r, ts, overflow)) {
+            if (job == kOwn) h = laneRayHit(r);
+            else if (r.prim >= 0) sh.hit[job] = 1;
+            job = kNoRay;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return h;
+}
+
+template <int STACK, bool NEE>
 __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, float4 *Lpath, int *pathCounters, int *spill,
                                                            int spillCap, int *overflow) {
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
+    __shared__ ShadowList lists[NEE ? kTraceThreads / 64 : 1];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
+    ShadowList &sh = lists[NEE ? threadIdx.x >> 6 : 0];
     const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), waves = (int)((gridDim.x * blockDim.x) >> 6);
     int *count = pathCounters + (wave % kPathSegs) * kPathCounters;
     auto tally = [&](int field, int bounce, bool mine) {
@@ -1736,36 +1799,46 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, Chun
         cameraRay(cam, row, col, jx, jy, &o, &d);
         f3 thr = mk(1.f), acc = mk(0.f);
         float prevPdf = -1.f;
-        for (int depth = 0; depth < cp.maxDepth && __ballot(alive) != 0; depth++) {
+        int shadows = 0;     // in the list (wave-uniform)
+        int myShadow = -1;   // this lane's place there
+        for (int depth = 0; depth < cp.maxDepth && (__ballot(alive) != 0 || shadows > 0); depth++) {
             tally(0, depth, alive);
-            LaneRay r;
-            traceLanes<CLOSEST, STACK>(sc, r, alive, o, d, depth == 0 ? 0.f : kBounceEps, FLT_MAX, ts, overflow);
+            TraceHit h;
+            if constexpr (NEE) {
+                h = traceBoth<STACK>(sc, alive, o, d, depth == 0 ? 0.f : kBounceEps, sh, shadows, ts, overflow);
+            } else {
+                LaneRay r;
+                traceLanes<CLOSEST, STACK>(sc, r, alive, o, d, depth == 0 ? 0.f : kBounceEps, FLT_MAX, ts, overflow);
+                h = laneRayHit(r);
+            }
+            if (NEE && shadows > 0) {
+                const bool lit = myShadow >= 0 && sh.hit[myShadow] == 0;
+                if (lit) acc = acc + mk(sh.contrib[0][myShadow], sh.contrib[1][myShadow], sh.contrib[2][myShadow]);
+                tally(3, depth - 1, lit);
+            }
             bool addL = false, pushRay = false, pushShadow = false;
-            f3 p = mk(0.f), contrib = mk(0.f), lightDir = mk(0.f), next = mk(0.f), nb = mk(0.f);
-            float lightDist = 0.f, nextPdf = -1.f;
+            f3 p = mk(0.f), contrib = mk(0.f), next = mk(0.f), nb = mk(0.f);
+            LightSample ls;
+            float nextPdf = -1.f;
             if (alive) {
                 f3 L;
-                if (r.prim == INT32_MIN) {
-                    L = missRadiance(sc, cp.nee, depth, prevPdf, thr, d);
+                if (h.prim == INT32_MIN) {
+                    L = missRadiance(sc, NEE, depth, prevPdf, thr, d);
                 } else {
-                    const TraceHit h = laneRayHit(r);
                     const SurfacePoint sp = surfaceAt(sc, h.prim, o, d, h.t, h.u, h.v);
                     const Frame fr = makeFrame(sp.n);
                     const f3 wo = normalize(toLocal(fr, -d));
                     const PtMaterial m = sc.materials[sp.mat];
                     const int type = matType(m);
-                    L = surfaceRadiance(sc, cp.nee, depth, prevPdf, thr, o, sp, wo, m, type);
+                    L = surfaceRadiance(sc, NEE, depth, prevPdf, thr, o, sp, wo, m, type);
                     if (depth + 1 < cp.maxDepth) {
                         const BsdfSample bs = sampleDirection(m, type, wo, rng);
                         pushRay = continuePath(bs, thr, &nb);
                         nextPdf = bs.delta ? -1.f : bs.pdf;
-                        if (cp.nee && !bs.delta) {
-                            LightSample ls;
+                        if (NEE && !bs.delta) {
                             pushShadow = lightSample(
                                 sc, rng, sp, fr, wo, m, thr, [&](f3 wiL, f3) { return cp.misSample ? bsdfSamplePdf(m, wo, wiL) : bsdfPdf(m, wo, wiL); }, &ls,
                                 &contrib);
-                            lightDir = ls.wi;
-                            lightDist = ls.dist;
                         }
                         p = sp.p;
                         next = toWorld(fr, bs.wi);
@@ -1775,12 +1848,15 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, Chun
                 if (depth == 0 || addL) acc = acc + L;
             }
             tally(2, depth, addL);
-            if (cp.nee) {
+            if constexpr (NEE) {
+                const uint64_t pushing = __ballot(pushShadow);
+                shadows = __popcll(pushing);
+                myShadow = -1;
+                if (pushShadow) {
+                    myShadow = (int)lanesBelow(pushing);
+                    sh.put(myShadow, p, ls.wi, ls.dist - 2e-4f, contrib);
+                }
                 tally(1, depth, pushShadow);
-                traceLanes<ANY, STACK>(sc, r, pushShadow, p, lightDir, kShadowEps, lightDist - 2e-4f, ts, overflow);
-                const bool lit = pushShadow && r.prim == INT32_MIN;
-                if (lit) acc = acc + contrib;
-                tally(3, depth, lit);
             }
             alive = pushRay;
             o = p;
@@ -2441,16 +2517,16 @@ GuideSceneNorm guideNorm(pt_renderer *r) {
 }
 
 // Whether a chunk's paths are traced whole (k_paths) or through the queues.  us a pass, queues /
-// whole: 256^2 pixels of 327k triangles 847 / 323, of the Cornell box 361 / 97, 1 sample each;
-// 2^20 paths: Cornell box 728 / 415, 5k triangles 775 / 464, 1.31M triangles 1816 / 1154, room of
-// 1M at depth 16 6534 / 5473; 2^21 paths: 5k triangles 936 / 821, 1.31M at depth 4 1931 / 1990,
-// room of 1M at depth 16 9526 / 10978; 2^23 paths: Cornell box 3727 / 2761, 17 nodes 1606 / 1401,
-// 304 nodes 2122 / 2106, 1229 nodes 2483 / 2710.  The timed and the counting kernels are the
+// whole: 2^16 paths: Cornell box (3 nodes) 342 / 86, 1.31M triangles (319k nodes) 857 / 359; 2^20:
+// 1.31M 1516 / 991, room of 1M (246k nodes, depth 16) 4787 / 4225; 2^21: 82k triangles (20k nodes)
+// 1295 / 1034, room of 100k (25k nodes) 5852 / 5522, 1.31M 1879 / 1643, room of 1M 7233 / 8299; 2^22:
+// 294 nodes 1195 / 1036, 1226 nodes 1366 / 1260, 20k nodes 1855 / 1888; 2^23: Cornell box 3424 /
+// 2585, 17 nodes 1256 / 1229, 294 nodes 1785 / 1939.  The timed and the counting kernels are the
 // queues', and so are a batch's: its chunks are filled with paths of several renders.
 bool wholePaths(const pt_renderer *r, const ChunkParams &cp) {
     if (r->type == PT_RENDERER_GUIDED || r->profile || r->traceStats || !r->ownsStream) return false;
     const int nodes = r->view.numNodes;
-    return cp.nPaths <= (nodes <= 16 ? 1 << 23 : nodes <= 4096 ? 1 << 21 : 1 << 20);
+    return cp.nPaths <= (nodes <= 16 ? 1 << 23 : nodes <= 4096 ? 1 << 22 : nodes <= 32768 ? 1 << 21 : 1 << 20);
 }
 
 void accumulateChunk(pt_renderer *r, const ChunkParams &cp, bool whole, const PassEnd &end) {
@@ -2469,8 +2545,9 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
         int *sp = ensureSpill(r, grid, &cap);
         float4 *L = r->pp->Lpath.as<float4>();
         int *pc = r->pp->pathCounters.as<int>(), *ov = r->pp->overflow.as<int>();
-        if (r->ldsStack == 32) k_paths<32><<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, L, pc, sp, cap, ov);
-        else k_paths<16><<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, L, pc, sp, cap, ov);
+        auto run = [&](auto kernel) { kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, L, pc, sp, cap, ov); };
+        if (cp.nee) r->ldsStack == 32 ? run(k_paths<32, true>) : run(k_paths<16, true>);
+        else r->ldsStack == 32 ? run(k_paths<32, false>) : run(k_paths<16, false>);
         PT_HIP_TRY(hipGetLastError());
         accumulateChunk(r, cp, true, end);
         return;
