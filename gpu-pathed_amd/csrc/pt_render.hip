@@ -578,6 +578,7 @@ template <int STACK> __device__ __forceinline__ void stackStart(LaneRay &r, cons
 // Makes room: the older half of the LDS entries moves to the spill area.
 template <int STACK, int UNROLL> __device__ __forceinline__ LdsInt *stackEvict(LdsInt *sp, const TraceStack ts, int *overflow) {
     constexpr int kMove = stackEntries(STACK) / 2;
+    static_assert(kMove >= 3 * kDescentSteps, "an eviction makes room for what the steps before it added");
     LdsInt *first = ts.column + kStackFirst * kTraceThreads;
     LdsInt *count = ts.column + stackCountRow(STACK) * kTraceThreads;
     const int n = *count;
@@ -2373,13 +2374,13 @@ int *ensureSpill(pt_renderer *r, int grid, int *cap) {
 // wave takes a whole run at a time: refilling early would mix in a pixel 64 runs away.  The
 // incoherent queues refill earlier, which shortens the wait for a batch's longest ray.
 // Per-launch optima on the 1.31M-triangle icosphere at 1024^2, 64 spp: camera rays 64
-// (extend 1773 -> 1678 us per launch against 48; 40 and 56 as 48), the later closest-hit
-// queues and the shadow rays 40 (whole batches of 64 take 1.9x as long on the first bounce's
-// queue; 16 idle lanes cost 6% of the pass).
+// (extend 1773 -> 1678 us per launch against 48; 40 and 56 as 48); later queues 32 (passes with 40, 32,
+// 24, 16 there: icosphere 17637, 17602, 17715, 18375 us, room of 4M 9722, 9627, 9596, 9594; whole
+// batches of 64 take 1.9x as long on the first bounce's queue).
 enum { TRACE_CAMERA = 0, TRACE_INCOHERENT = 1, TRACE_SHADOW = 2 };
 int refillLanes(const pt_renderer *r, int kind) {
     if (r->refillLanes > 0) return r->refillLanes;
-    return kind == TRACE_CAMERA ? 64 : 40;
+    return kind == TRACE_CAMERA ? 64 : 32;
 }
 
 // Trace grids hold at least PT_QUEUE_SEGS waves: every queue segment needs home waves.
