@@ -535,6 +535,11 @@ __device__ __forceinline__ const float *boxOf(const BinTree &t, int c) {
 // consecutive leaf positions and notes the nodes it leaves its tile at, the next launch's
 // workgroups carry on from those in tiles kClimbFan times as long, until one tile holds the
 // tree (1.31M leaves: three launches).
+//
+// Then it is the chain of dependent loads per level that counts.  In global memory it was parent,
+// its range, arrival, children, their results, 3 us a level (295 + 157 + 162 us); a node's place is
+// now loaded while its child is computed, the first launch's results, nine in ten, meet in LDS, and
+// a climb keeps the child that it comes from (81 + 111 us).
 constexpr int kClimbTile = 1024;
 constexpr int kClimbFan = 64;
 
@@ -549,33 +554,37 @@ struct ClimbArgs {
     int *left[2], *leftCount[2];
 };
 
-// cost of child c given `slots` of its parent
-__device__ float slotCost(const ClimbArgs &a, int c, int slots, float leafCost) {
-    if (!liveChild(a.t, c)) return leafCost;
-    return (slots == 1 ? a.tb.W : slots == 2 ? a.tb.S2 : a.tb.S3)[c];
-}
+// What a parent needs of a child: a leaf, or an internal node that has been computed.
+struct Subtree {
+    float box[6];
+    float W, S2, S3;
+    int cnt, height;   // leaves, and internal nodes on the longest path down
+    __device__ __forceinline__ float cost(int slots, float leafCost) const {
+        return cnt <= PT_LEAF_MAX ? leafCost : slots == 1 ? W : slots == 2 ? S2 : S3;
+    }
+};
 
-template <bool BOXES> __device__ void climbNode(const ClimbArgs &a, int p) {
-    const int2 c = a.t.children[p];
-    float x[6], y[6];
-    for (int k = 0; k < 6; k++) x[k] = c.x >= 0 ? a.nodeBoxes[6 * (size_t)c.x + k] : a.t.leafBoxes[6 * (size_t)(~c.x) + k];
-    for (int k = 0; k < 6; k++) y[k] = c.y >= 0 ? a.nodeBoxes[6 * (size_t)c.y + k] : a.t.leafBoxes[6 * (size_t)(~c.y) + k];
-    float u[6];
+// Internal node p from its children x and y; its results go to the global tables, and back.
+template <bool BOXES> __device__ __forceinline__ Subtree climbNode(const ClimbArgs &a, int p, int cnt, const Subtree &x, const Subtree &y) {
+    Subtree r;
     for (int k = 0; k < 3; k++) {
-        u[k] = fminf(x[k], y[k]);
-        u[3 + k] = fmaxf(x[3 + k], y[3 + k]);
+        r.box[k] = fminf(x.box[k], y.box[k]);
+        r.box[3 + k] = fmaxf(x.box[3 + k], y.box[3 + k]);
     }
     if constexpr (BOXES)
-        for (int k = 0; k < 6; k++) a.nodeBoxes[6 * (size_t)p + k] = u[k];
-    a.height[p] = 1 + max(c.x >= 0 ? a.height[c.x] : 0, c.y >= 0 ? a.height[c.y] : 0);
-    if (a.t.cnt[p] <= PT_LEAF_MAX) return;
-    const float lx = kPrimCost * boxArea6(x) * (float)childCount(a.t, c.x), ly = kPrimCost * boxArea6(y) * (float)childCount(a.t, c.y);
+        for (int k = 0; k < 6; k++) a.nodeBoxes[6 * (size_t)p + k] = r.box[k];
+    r.cnt = cnt;
+    r.height = 1 + max(x.height, y.height);
+    a.height[p] = r.height;
+    r.W = r.S2 = r.S3 = 0.f;
+    if (cnt <= PT_LEAF_MAX) return r;
+    const float lx = kPrimCost * boxArea6(x.box) * (float)x.cnt, ly = kPrimCost * boxArea6(y.box) * (float)y.cnt;
     float share[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     for (int j = 2; j <= 4; j++) {
         float best = INFINITY;
         int bi = 1;
         for (int i = 1; i < j; i++) {
-            const float v = slotCost(a, c.x, min(i, 3), lx) + slotCost(a, c.y, min(j - i, 3), ly);
+            const float v = x.cost(min(i, 3), lx) + y.cost(min(j - i, 3), ly);
             if (v < best) {
                 best = v;
                 bi = i;
@@ -584,11 +593,102 @@ template <bool BOXES> __device__ void climbNode(const ClimbArgs &a, int p) {
         share[j] = best;
         a.tb.split[3 * (size_t)p + (j - 2)] = (unsigned char)bi;
     }
-    const float w = kNodeCost * boxArea6(u) + share[4];
-    a.tb.W[p] = w;
-    a.tb.S2[p] = fminf(w, share[2]);
-    a.tb.S3[p] = fminf(w, share[3]);
-    a.tb.opened[p] = (unsigned char)((share[2] < w ? 1 : 0) | (share[3] < w ? 2 : 0));
+    r.W = kNodeCost * boxArea6(r.box) + share[4];
+    r.S2 = fminf(r.W, share[2]);
+    r.S3 = fminf(r.W, share[3]);
+    a.tb.W[p] = r.W;
+    a.tb.S2[p] = r.S2;
+    a.tb.S3[p] = r.S3;
+    a.tb.opened[p] = (unsigned char)((share[2] < r.W ? 1 : 0) | (share[3] < r.W ? 2 : 0));
+    return r;
+}
+
+// A node's place in the tree.  A climb loads its next node's while it waits for the present one.
+struct Place {
+    int first, cnt, parent;
+    int2 children;
+};
+__device__ __forceinline__ Place placeOf(const BinTree &t, int p) {
+    if (p < 0) return Place{0, 0, -1, make_int2(0, 0)};
+    return Place{t.first[p], t.cnt[p], t.parentNode[p], t.children[p]};
+}
+
+__device__ __forceinline__ Subtree leafSubtree(const ClimbArgs &a, int leaf) {
+    Subtree s;
+    for (int k = 0; k < 6; k++) s.box[k] = a.t.leafBoxes[6 * (size_t)leaf + k];
+    s.W = s.S2 = s.S3 = 0.f;
+    s.cnt = 1;
+    s.height = 0;
+    return s;
+}
+__device__ __forceinline__ Subtree globalSubtree(const ClimbArgs &a, int c) {
+    if (c < 0) return leafSubtree(a, ~c);
+    Subtree s;
+    for (int k = 0; k < 6; k++) s.box[k] = a.nodeBoxes[6 * (size_t)c + k];
+    s.W = a.tb.W[c];
+    s.S2 = a.tb.S2[c];
+    s.S3 = a.tb.S3[c];
+    s.cnt = a.t.cnt[c];
+    s.height = a.height[c];
+    return s;
+}
+
+// The first launch over an LBVH, whose node numbers are positions of their subtrees' ends: a tile's
+// nodes meet in LDS, and the global tables are only written, without a wait.
+__global__ __launch_bounds__(kClimbTile) void k_climb_tiles(ClimbArgs a) {
+    __shared__ float box[6][kClimbTile], cost[3][kClimbTile];
+    __shared__ int cnt[kClimbTile], height[kClimbTile], arrivals[kClimbTile];
+    __shared__ int out;
+    if (threadIdx.x == 0) out = 0;
+    arrivals[threadIdx.x] = 0;
+    __syncthreads();
+    const int begin = (int)(blockIdx.x * kClimbTile), end = min(begin + kClimbTile, a.t.n);
+    const int pos = begin + (int)threadIdx.x;
+    if (pos < end) {
+        int p = a.t.parentLeaf[pos], from = ~pos;
+        Subtree s = leafSubtree(a, pos);
+        Place at = placeOf(a.t, p);
+        // a node inside the tile has all its leaves there, so its two arrivals are of this workgroup
+        while (p >= 0 && at.first >= begin && at.first + at.cnt <= end) {
+            if (from >= 0) {
+                const int k = from - begin;
+                for (int j = 0; j < 6; j++) box[j][k] = s.box[j];
+                cost[0][k] = s.W;
+                cost[1][k] = s.S2;
+                cost[2][k] = s.S3;
+                cnt[k] = s.cnt;
+                height[k] = s.height;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            if (__hip_atomic_fetch_add(&arrivals[p - begin], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) {
+                p = -1;
+                break;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            const Place next = placeOf(a.t, at.parent);
+            const bool left = at.children.x == from;
+            const int c = left ? at.children.y : at.children.x;
+            Subtree o;
+            if (c < 0) {
+                o = leafSubtree(a, ~c);
+            } else {
+                const int k = c - begin;
+                for (int j = 0; j < 6; j++) o.box[j] = box[j][k];
+                o.W = cost[0][k];
+                o.S2 = cost[1][k];
+                o.S3 = cost[2][k];
+                o.cnt = cnt[k];
+                o.height = height[k];
+            }
+            s = left ? climbNode<true>(a, p, at.cnt, s, o) : climbNode<true>(a, p, at.cnt, o, s);
+            from = p;
+            p = at.parent;
+            at = next;
+        }
+        if (p >= 0) a.left[1][begin + atomicAdd(&out, 1)] = p;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) a.leftCount[1][blockIdx.x] = out;
 }
 
 // One launch of the pass over tiles of `tile` leaf positions; in: the parity of the launch before,
@@ -600,13 +700,15 @@ template <bool BOXES> __global__ __launch_bounds__(kClimbTile) void k_climb(Clim
     const int64_t begin64 = (int64_t)blockIdx.x * tile;
     const int begin = (int)begin64, end = (int)min(begin64 + tile, (int64_t)a.t.n);
     auto climb = [&](int p) {
-        // a node inside the tile has all its leaves there, so its two arrivals are of this workgroup
-        while (p >= 0 && a.t.first[p] >= begin && a.t.first[p] + a.t.cnt[p] <= end) {
+        Place at = placeOf(a.t, p);
+        while (p >= 0 && at.first >= begin && at.first + at.cnt <= end) {
             __threadfence_block();
             if (__hip_atomic_fetch_add(&a.arrivals[p], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) return;
             __threadfence_block();
-            climbNode<BOXES>(a, p);
-            p = a.t.parentNode[p];
+            const Place next = placeOf(a.t, at.parent);
+            climbNode<BOXES>(a, p, at.cnt, globalSubtree(a, at.children.x), globalSubtree(a, at.children.y));
+            p = at.parent;
+            at = next;
         }
         // a tile of n positions is left at most n times: every time for another subtree
         if (p >= 0) a.left[1 - in][begin + atomicAdd(&out, 1)] = p;
@@ -631,7 +733,9 @@ template <bool BOXES> void climbTree(const ClimbArgs &a, hipStream_t stream) {
     int in = 0;
     int64_t sub = 0;
     for (int64_t tile = kClimbTile;; tile *= kClimbFan) {
-        k_climb<BOXES><<<blocks(a.t.n, (int)std::min<int64_t>(tile, INT32_MAX)), kClimbTile, 0, stream>>>(a, (int)std::min<int64_t>(tile, INT32_MAX), (int)sub, in);
+        const int len = (int)std::min<int64_t>(tile, INT32_MAX);
+        if (BOXES && sub == 0) k_climb_tiles<<<blocks(a.t.n, len), kClimbTile, 0, stream>>>(a);
+        else k_climb<BOXES><<<blocks(a.t.n, len), kClimbTile, 0, stream>>>(a, len, (int)sub, in);
         PT_HIP_TRY(hipGetLastError());
         if (tile >= a.t.n) return;
         sub = tile;
