@@ -672,13 +672,25 @@ __global__ void k_guide_pack(const float *params, __bf16 *w, __bf16 *wt, float *
     storeParam(p, liveParam(p) ? params[p] : 0.f, w, wt, b);
 }
 
+__device__ __forceinline__ void adamStep(const AdamState &st, int p, float g) {
+    const float mm = 0.9f * st.m[p] + 0.1f * g;
+    const float vv = 0.999f * st.v[p] + 0.001f * g * g;
+    st.m[p] = mm;
+    st.v[p] = vv;
+    const float val = st.params[p] - st.lr * (mm * st.c1) / (sqrtf(vv * st.c2) + 1e-8f);
+    st.params[p] = val;
+    storeParam(p, val, st.w, st.wt, st.b);
+}
+
 // Sum of the per-block partial gradients: 64 parameters per block, REDUCE_SLICES slices of the
 // partials per parameter (k = slice, slice + REDUCE_SLICES, ...), the slices added in a fixed
 // tree, so the result does not depend on scheduling.  The last block sums the per-block losses
-// the same way (fixed strided partial sums, then a fixed tree).
+// the same way (fixed strided partial sums, then a fixed tree).  ADAM: a parameter's step follows in
+// the thread that has its gradient (as a kernel of its own 4.8 us and a launch more per step).
 constexpr int REDUCE_SLICES = 16;
+template <bool ADAM>
 __global__ __launch_bounds__(64 * REDUCE_SLICES) void k_guide_reduce(const float *partials, int nblocks, const float *lossPart, int nloss,
-                                                                    float invBatch, float *grad, float *lossOut) {
+                                                                    float invBatch, float *grad, float *lossOut, AdamState st) {
     __shared__ float part[REDUCE_SLICES][64];
     __shared__ float lsum[64 * REDUCE_SLICES];
     const int t = threadIdx.x;
@@ -706,22 +718,16 @@ __global__ __launch_bounds__(64 * REDUCE_SLICES) void k_guide_reduce(const float
         if (slice < half) part[slice][t & 63] += part[slice + half][t & 63];
         __syncthreads();
     }
-    if (slice == 0 && p < GUIDE_PARAMS) grad[p] = liveParam(p) ? part[0][t] * invBatch : 0.f;
+    if (slice == 0 && p < GUIDE_PARAMS) {
+        const float g = liveParam(p) ? part[0][t] * invBatch : 0.f;
+        grad[p] = g;
+        if (ADAM && liveParam(p)) adamStep(st, p, g);
+    }
 }
 
-__global__ void k_guide_adam(float *params, float *m, float *v, const float *grad, float c1, float c2, float lr, __bf16 *w, __bf16 *wt,
-                             float *b) {
+__global__ void k_guide_adam(AdamState st, const float *grad) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= GUIDE_PARAMS) return;
-    if (!liveParam(p)) return;
-    const float g = grad[p];
-    const float mm = 0.9f * m[p] + 0.1f * g;
-    const float vv = 0.999f * v[p] + 0.001f * g * g;
-    m[p] = mm;
-    v[p] = vv;
-    const float val = params[p] - lr * (mm * c1) / (sqrtf(vv * c2) + 1e-8f);
-    params[p] = val;
-    storeParam(p, val, w, wt, b);
+    if (p < GUIDE_PARAMS && liveParam(p)) adamStep(st, p, grad[p]);
 }
 
 __global__ void k_mfma_tile(const float *A, const float *B, float *C) {
@@ -814,17 +820,24 @@ void guideInferRaw(GuideNet net, const float *feats, int n, float *rawOut, hipSt
 }
 
 void guideGradients(GuideNet net, const float4 *records, const int *count, const int *prefix, int recSeg, int base, int batch,
-                    const float *wsum, const GuideTrainBufs &tb, float *grad, float *lossOut, hipStream_t s) {
+                    const float *wsum, const GuideTrainBufs &tb, float *grad, float *lossOut, hipStream_t s, const AdamState *step) {
     k_guide_train<<<tb.blocks, 64 * TRAIN_WAVES, 0, s>>>(net, records, count, prefix, recSeg, wsum, base, batch, tb.partials, tb.lossPart);
-    k_guide_reduce<<<(GUIDE_PARAMS + 63) / 64 + 1, 64 * REDUCE_SLICES, 0, s>>>(tb.partials, tb.blocks, tb.lossPart, tb.blocks,
-                                                                              1.f / (float)std::max(batch, 1), grad, lossOut);
+    auto reduce = [&](auto kernel) {
+        kernel<<<(GUIDE_PARAMS + 63) / 64 + 1, 64 * REDUCE_SLICES, 0, s>>>(tb.partials, tb.blocks, tb.lossPart, tb.blocks, 1.f / (float)std::max(batch, 1),
+                                                                          grad, lossOut, step ? *step : AdamState{});
+    };
+    step ? reduce(k_guide_reduce<true>) : reduce(k_guide_reduce<false>);
     PT_HIP_TRY(hipGetLastError());
 }
 
-void guideAdam(float *params, float *m, float *v, const float *grad, int step, float lr, __bf16 *dW, __bf16 *dWt, float *dB, hipStream_t s) {
+AdamState guideAdamState(float *params, float *m, float *v, int step, float lr, __bf16 *dW, __bf16 *dWt, float *dB) {
     const float c1 = 1.f / (1.f - powf(0.9f, (float)step));
     const float c2 = 1.f / (1.f - powf(0.999f, (float)step));
-    k_guide_adam<<<(GUIDE_PARAMS + 255) / 256, 256, 0, s>>>(params, m, v, grad, c1, c2, lr, dW, dWt, dB);
+    return AdamState{params, m, v, c1, c2, lr, dW, dWt, dB};
+}
+
+void guideAdam(float *params, float *m, float *v, const float *grad, int step, float lr, __bf16 *dW, __bf16 *dWt, float *dB, hipStream_t s) {
+    k_guide_adam<<<(GUIDE_PARAMS + 255) / 256, 256, 0, s>>>(guideAdamState(params, m, v, step, lr, dW, dWt, dB), grad);
     PT_HIP_TRY(hipGetLastError());
 }
 

@@ -1930,14 +1930,20 @@ __global__ __launch_bounds__(64) void k_pick(PtSceneView sc, float4 o, float4 d,
 // Records live in per-segment parts of recSeg entries; block 0 also writes the exclusive prefix
 // sums of the kept counts, through which training reads the records as one sequence.
 __global__ __launch_bounds__(256) void k_guide_finalize(float4 *records, int recSeg, int *counters, const float4 *Lpath) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        int acc = 0;
-        for (int s = 0; s < PT_QUEUE_SEGS; s++) {
-            counters[kRecPrefixSlot + s] = acc;
-            acc += min(counters[ptQueueField(s, 0, PT_Q_RECORDS)], recSeg);
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        static_assert(PT_QUEUE_SEGS == 64, "a lane per segment");
+        const int s = (int)threadIdx.x;
+        const int n = min(counters[ptQueueField(s, 0, PT_Q_RECORDS)], recSeg);
+        int upTo = n;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int other = __shfl_up(upTo, off);
+            if (s >= off) upTo += other;
         }
-        counters[kRecPrefixSlot + PT_QUEUE_SEGS] = acc;
-        counters[kRecValidSlot] = acc;
+        counters[kRecPrefixSlot + s] = upTo - n;
+        if (s == 63) {
+            counters[kRecPrefixSlot + PT_QUEUE_SEGS] = upTo;
+            counters[kRecValidSlot] = upTo;
+        }
     }
     // grid-stride over the record slots; the weight sum is reduced per block so that the
     // shared accumulator takes one atomic per block
@@ -2647,10 +2653,10 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
         tb.lossPart = r->gLossPart.as<float>();
         for (int s = 0; s < r->gTrainSteps; s++) {
             const int base = (int)((r->gTrainTotal * (int64_t)r->gBatch) & 0x3fffffff);
+            const AdamState step = guideAdamState(r->gParams.as<float>(), r->gM.as<float>(), r->gV.as<float>(), ++r->gAdamStep, r->gLr, r->gW.as<__bf16>(),
+                                                  r->gWt.as<__bf16>(), r->gB.as<float>());
             guideGradients(guideNet(r), r->gRecords.as<float4>(), &ctr[kRecValidSlot], &ctr[kRecPrefixSlot], (int)(r->gRecCap / PT_QUEUE_SEGS),
-                           base, r->gBatch, (const float *)&ctr[kWsumSlot], tb, r->gGrad.as<float>(), r->gLoss.as<float>(), r->stream);
-            guideAdam(r->gParams.as<float>(), r->gM.as<float>(), r->gV.as<float>(), r->gGrad.as<float>(), ++r->gAdamStep, r->gLr,
-                      r->gW.as<__bf16>(), r->gWt.as<__bf16>(), r->gB.as<float>(), r->stream);
+                           base, r->gBatch, (const float *)&ctr[kWsumSlot], tb, r->gGrad.as<float>(), r->gLoss.as<float>(), r->stream, &step);
             r->gTrainTotal++;
         }
     }
