@@ -367,16 +367,6 @@ __global__ __launch_bounds__(256) void k_raygen_batch(ChunkParams cp, float4 *ra
 // The camera origin of a batch render.
 __device__ __forceinline__ float4 batchCameraOrigin(const BatchRender &R) { return make_float4(R.cam.m[0][3], R.cam.m[1][3], R.cam.m[2][3], 0.f); }
 
-// The camera-ray state k_raygen does not store: the RNG after the pixel's two jitter draws.
-__device__ __forceinline__ Rng cameraRng(const ChunkParams &cp, int path) {
-    int s;
-    const int pixel = cp.pixBegin + chunkPixelOf(cp, path, &s);
-    Rng rng = seedRng(cp.seed, (uint32_t)pixel, (uint32_t)(cp.sampleBase + s));
-    rng.next();
-    rng.next();
-    return rng;
-}
-
 // ------------------------------------------------------------------------------------------
 // BVH traversal (closest hit / any hit) over the 4-wide BVH: one 128-byte node fetch tests
 // four child boxes; the hit children are ordered near to far (a 5-exchange sorting network),
@@ -1393,15 +1383,17 @@ template <bool GUIDED, bool BATCH = false>
 __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, ChunkParams cp, int bounce, int *counters, const float4 *rayO, const float4 *rayD,
                                                const uint4 *state, const float4 *beta, const float4 *hits, float4 *nRayO, float4 *nRayD,
                                                uint4 *nState, float4 *nBeta, float4 *sO, float4 *sD, float4 *sL, float4 *Lpath,
-                                               GuideShadeArgs ga, float4 camO) {
+                                               GuideShadeArgs ga, PtCamera cam, int cameraRays) {
     // Waves claim 64 rays at a time from one queue segment and append the continuation and
     // shadow rays to the same segment of the next queues.  Appends happen where each record is
     // complete (one atomic per wave and branch: the lanes taking a branch append together), so
     // no output record stays live across the rest of the vertex.
     //
-    // camO.w != 0 (bounce 0): the camera rays' origin, throughput, previous pdf, path index and
-    // RNG state are recomputed here instead of read (k_raygen stores only the directions), and
-    // the path's radiance is written instead of added to.
+    // cameraRays (bounce 0): the camera rays, their throughput, previous pdf, path index and RNG state
+    // are recomputed here instead of read, and the path's radiance is written instead of added to.
+    // (Reading the directions that k_raygen stores for the traversal cost more than making them
+    // again: the kernel is bound by what passes the L2; 2^26 paths of 1.31M triangles 3907 -> 3716 us
+    // a pass.)
     //
     // BATCH (a batch wavefront): every path belongs to one render of the batch (state.w above
     // the depth; at bounce 0 found from the path index), whose camera, lights, environment,
@@ -1413,7 +1405,7 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
     // together), parks the slots of hits and of misses in two LDS lists and shades either 64
     // at a time, so both codes run on full waves.  Every vertex is shaded exactly once (the
     // last partial batches when the queue is exhausted); results do not depend on the order.
-    const bool camera = camO.w != 0.f;
+    const bool camera = cameraRays != 0;
     // per wave: parked slots (the segment is slot / segLen), each list below 64 + one claim
     // (at most 63 left over plus the claim)
     __shared__ int sHit[4][64 * (kShadeClaimWords + 1)], sMiss[4][64 * (kShadeClaimWords + 1)];
@@ -1472,26 +1464,32 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
         bool addL = false;
         int rid = 0, spawned = 0;   // batch wavefront: the path's render, rays its vertex spawned
         if (active) {
-            const float4 rd = streamLoad(&rayD[i]), h = streamLoad(&hits[i]);
+            const float4 h = streamLoad(&hits[i]);
             float4 ro, bp;
             uint4 st;
+            f3 d;
             if (camera) {
+                // the ray from its jitter draws, as k_raygen makes it
                 const int p = ptCameraPath(seg, i - seg * cp.segLen);
                 bp = make_float4(1.f, 1.f, 1.f, -1.f);
+                PathSource ps{0, 0, 0, cp.seed};
                 if constexpr (BATCH) {
-                    const PathSource ps = batchPathSource(cp, p);
-                    const BatchRender &R = cp.renders[ps.render];
-                    Rng g = seedRng(ps.seed, (uint32_t)ps.pixel, (uint32_t)ps.sample);
-                    g.next();
-                    g.next();
-                    ro = batchCameraOrigin(R);
-                    st = make_uint4((uint32_t)g.state, (uint32_t)(g.state >> 32), (uint32_t)p, packDepth(0, ps.render));
+                    ps = batchPathSource(cp, p);
                 } else {
-                    const Rng g = cameraRng(cp, p);
-                    ro = camO;
-                    st = make_uint4((uint32_t)g.state, (uint32_t)(g.state >> 32), (uint32_t)p, 0u);
+                    ps.pixel = cp.pixBegin + chunkPixelOf(cp, p, &ps.sample);
+                    ps.sample += cp.sampleBase;
                 }
+                const PtCamera &c = BATCH ? cp.renders[ps.render].cam : cam;
+                Rng g = seedRng(ps.seed, (uint32_t)ps.pixel, (uint32_t)ps.sample);
+                const float jx = g.uniform(), jy = g.uniform();
+                int col;
+                const int row = divmodEst(ps.pixel, BATCH ? cp.renders[ps.render].W : cp.W, &col);
+                f3 from;
+                cameraRay(c, row, col, jx, jy, &from, &d);
+                ro = f4(from, 0.f);
+                st = make_uint4((uint32_t)g.state, (uint32_t)(g.state >> 32), (uint32_t)p, BATCH ? packDepth(0, ps.render) : 0u);
             } else {
+                d = xyz(streamLoad(&rayD[i]));
                 ro = streamLoad(&rayO[i]);
                 bp = streamLoad(&beta[i]);
                 st = streamLoad(&state[i]);
@@ -1509,7 +1507,7 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
                 lv.env = R.env;
                 maxDepth = R.maxDepth;
             }
-            const f3 o = xyz(ro), d = xyz(rd), thr = xyz(bp);
+            const f3 o = xyz(ro), thr = xyz(bp);
             const float prevPdf = bp.w;
             f3 L = mk(0.f);
             if constexpr (GUIDED) {
@@ -2619,12 +2617,12 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
                 k_shade<true><<<shadeGrid, 256, 0, r->stream>>>(
                     r->view, cp, b, ctr, r->pp->rayO[cur].as<float4>(), r->pp->rayD[cur].as<float4>(), r->pp->st[cur].as<uint4>(), r->pp->beta[cur].as<float4>(),
                     r->pp->hits.as<float4>(), r->pp->rayO[1 - cur].as<float4>(), r->pp->rayD[1 - cur].as<float4>(), r->pp->st[1 - cur].as<uint4>(),
-                    r->pp->beta[1 - cur].as<float4>(), r->pp->sO.as<float4>(), r->pp->sD.as<float4>(), r->pp->sL.as<float4>(), r->pp->Lpath.as<float4>(), ga, bo);
+                    r->pp->beta[1 - cur].as<float4>(), r->pp->sO.as<float4>(), r->pp->sD.as<float4>(), r->pp->sL.as<float4>(), r->pp->Lpath.as<float4>(), ga, r->cam, b == 0);
             else
                 k_shade<false><<<shadeGrid, 256, 0, r->stream>>>(
                     r->view, cp, b, ctr, r->pp->rayO[cur].as<float4>(), r->pp->rayD[cur].as<float4>(), r->pp->st[cur].as<uint4>(), r->pp->beta[cur].as<float4>(),
                     r->pp->hits.as<float4>(), r->pp->rayO[1 - cur].as<float4>(), r->pp->rayD[1 - cur].as<float4>(), r->pp->st[1 - cur].as<uint4>(),
-                    r->pp->beta[1 - cur].as<float4>(), r->pp->sO.as<float4>(), r->pp->sD.as<float4>(), r->pp->sL.as<float4>(), r->pp->Lpath.as<float4>(), ga, bo);
+                    r->pp->beta[1 - cur].as<float4>(), r->pp->sO.as<float4>(), r->pp->sD.as<float4>(), r->pp->sL.as<float4>(), r->pp->Lpath.as<float4>(), ga, r->cam, b == 0);
             PT_HIP_TRY(hipGetLastError());
         }
         cur = 1 - cur;
@@ -3866,13 +3864,11 @@ void runWaveChunk(pt_batch *b, const WaveChunk &c) {
         if (bn == 0 || !merged)
             launchExtend(w, bn, cp.segLen, pp.rayO[cur].as<float4>(), pp.rayD[cur].as<float4>(), pp.hits.as<float4>(),
                          bn == 0 ? TRACE_CAMERA : TRACE_INCOHERENT, make_float4(0.f, 0.f, 0.f, 0.f), &cp);
-        // w = 1 marks bounce 0 (camera vertices); batch kernels take each render's camera
-        const float4 camFlag = make_float4(0.f, 0.f, 0.f, bn == 0 ? 1.f : 0.f);
         k_shade<false, true><<<shadeGrid, 256, 0, b->stream>>>(
             w->view, cp, bn, ctr, pp.rayO[cur].as<float4>(), pp.rayD[cur].as<float4>(), pp.st[cur].as<uint4>(), pp.beta[cur].as<float4>(),
             pp.hits.as<float4>(), pp.rayO[1 - cur].as<float4>(), pp.rayD[1 - cur].as<float4>(), pp.st[1 - cur].as<uint4>(),
             pp.beta[1 - cur].as<float4>(), pp.sO.as<float4>(), pp.sD.as<float4>(), pp.sL.as<float4>(), pp.Lpath.as<float4>(), GuideShadeArgs{},
-            camFlag);
+            PtCamera{}, bn == 0);
         PT_HIP_TRY(hipGetLastError());
         cur = 1 - cur;
         if (!merged && cp.nee) launchShadow(w, bn, cp.segLen);
