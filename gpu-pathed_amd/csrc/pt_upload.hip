@@ -17,7 +17,6 @@
 #include <cmath>
 #include <memory>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 #include "pt_gpu.h"
@@ -309,12 +308,17 @@ struct ReadStage {
         if (p) (void)hipHostFree(p);
         for (hipEvent_t e : events) (void)hipEventDestroy(e);
     }
-    void prepare(size_t n, size_t pieces) {
+    // false: no pinned memory to be had
+    bool prepare(size_t n, size_t pieces) {
         if (bytes < n) {
             if (p) (void)hipHostFree(p);
             p = nullptr;
             bytes = 0;
-            PT_HIP_TRY(hipHostMalloc((void **)&p, n, hipHostMallocPortable));
+            if (hipHostMalloc((void **)&p, n, hipHostMallocPortable) != hipSuccess) {
+                (void)hipGetLastError();
+                p = nullptr;
+                return false;
+            }
             bytes = n;
         }
         while (events.size() < pieces) {
@@ -322,6 +326,7 @@ struct ReadStage {
             PT_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             events.push_back(e);
         }
+        return true;
     }
 };
 
@@ -393,7 +398,11 @@ void readToHost(void *dst, const void *src, size_t bytes, hipStream_t stream) {
     // about six pieces
     const size_t piece = std::clamp<size_t>(bytes / 6 / 256 * 256, kReadPieceMin, kReadPieceMax);
     std::unique_ptr<ReadStage> stage = stageKeeper().take(device);
-    stage->prepare(std::min(bytes, kReadStage), (std::min(bytes, kReadStage) + piece - 1) / piece);
+    if (!stage->prepare(std::min(bytes, kReadStage), (std::min(bytes, kReadStage) + piece - 1) / piece)) {
+        PT_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
+        PT_HIP_TRY(hipStreamSynchronize(stream));
+        return;
+    }
     for (size_t done = 0; done < bytes;) {
         const size_t part = std::min(bytes - done, kReadStage);
         const int n = (int)((part + piece - 1) / piece);
@@ -416,8 +425,8 @@ void readToHost(void *dst, const void *src, size_t bytes, hipStream_t stream) {
         const size_t wanted = std::min<size_t>(4, part / kReadPerThread);
         try {
             while (helpers.size() < wanted) helpers.emplace_back(copyOut);
-        } catch (const std::system_error &) {
-            // no thread to be had: this one copies what is left
+        } catch (...) {
+            // no thread (or no memory for one) to be had: this one copies what is left
         }
         copyOut();
         for (std::thread &t : helpers) t.join();
