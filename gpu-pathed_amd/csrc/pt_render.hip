@@ -2,17 +2,20 @@
 //
 // One progressive pass of `spp` samples per pixel is cut into chunks of at most `pool`
 // paths (whole sample rows of the image, or pixel ranges when the image alone exceeds the
-// pool).  A chunk runs:
+// pool).  A small chunk is traced whole in one launch (k_paths); a large one, and any that is guided,
+// timed or part of a batch, runs:
 //
-//   raygen            one thread per path: PCG32 stream, camera ray, path record
+//   raygen            one thread per path: PCG32 stream, camera ray's direction
+//   extend            camera rays: closest hit through the BVH, as packets where runs of them stay
+//                     together, else persistent waves, a ray per lane
 //   for each bounce:
-//     extend          persistent waves fetch 64 rays at a time; closest hit through the BVH
-//                     with a traversal stack in LDS
 //     shade           emission with MIS weight, BSDF sample, light sample; appends the
 //                     continuation ray and the shadow ray to compacted queues (one atomic
 //                     per wave, slots from the wave's ballot prefix)
-//     shadow          persistent any-hit traversal; adds the unoccluded light contribution
-//   accumulate        per pixel: FP64 sum of the chunk's sample radiances
+//     trace           the shadow rays (any hit; adds the unoccluded light contribution) and the
+//                     next bounce's extension rays, lanes of a wave taking either
+//   accumulate        per pixel: FP64 sum of the chunk's sample radiances; at the pass's end the
+//                     framebuffers
 //
 // Path state is structure-of-arrays in HBM, double-buffered between bounces so every queue
 // kernel reads and writes contiguously:
@@ -3312,15 +3315,15 @@ int pt_renderer_get_kernel_stats(pt_renderer *r, pt_kernel_stat *out, int cap, i
     const double npix = (double)r->W * r->H * (double)r->kstat[K_TONEMAP].launches;
     // algorithmic bytes per unit (record sizes above)
     pt_kernel_stat *k = r->kstat;
-    // camera rays (bounce 0) carry only a direction: no origin, state or throughput reads, and
-    // shade writes their paths' radiance once instead of a read-modify-write
+    // camera rays (bounce 0) carry only a direction, which shade makes itself: it reads their hits
+    // alone, and writes their paths' radiance once instead of a read-modify-write
     const double camRays = (double)s[S_RAYS], camAdds = (double)s[S_LADD_SHADE];
     k[K_RAYGEN].units = (int64_t)paths;
     k[K_RAYGEN].bytes = 16.0 * paths;                    // writes rayD
     k[K_EXTEND].units = (int64_t)rays;
     k[K_EXTEND].bytes = 48.0 * rays - 16.0 * camRays;    // reads rayO (not for camera rays), rayD; writes hit
     k[K_SHADE].units = (int64_t)rays;
-    k[K_SHADE].bytes = 80.0 * rays - 48.0 * camRays + 64.0 * nextRays + 48.0 * shadows + 32.0 * (addShade - camAdds) + 16.0 * camRays;
+    k[K_SHADE].bytes = 80.0 * rays - 64.0 * camRays + 64.0 * nextRays + 48.0 * shadows + 32.0 * (addShade - camAdds) + 16.0 * camRays;
     k[K_SHADOW].units = (int64_t)shadows;
     k[K_SHADOW].bytes = 48.0 * shadows + 32.0 * addShadow;
     k[K_ACCUM].units = (int64_t)pixelsAcc;
