@@ -1471,6 +1471,7 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
             float4 ro, bp;
             uint4 st;
             f3 d;
+            uint64_t cameraInc = 0;
             if (camera) {
                 // the ray from its jitter draws, as k_raygen makes it
                 const int p = ptCameraPath(seg, i - seg * cp.segLen);
@@ -1485,6 +1486,7 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
                 const PtCamera &c = BATCH ? cp.renders[ps.render].cam : cam;
                 Rng g = seedRng(ps.seed, (uint32_t)ps.pixel, (uint32_t)ps.sample);
                 const float jx = g.uniform(), jy = g.uniform();
+                cameraInc = g.inc;
                 int col;
                 const int row = divmodEst(ps.pixel, BATCH ? cp.renders[ps.render].W : cp.W, &col);
                 f3 from;
@@ -1531,7 +1533,9 @@ __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, C
                 L = surfaceRadiance(lv, cp.nee, depth, prevPdf, thr, o, sp, wo, m, type);
                 if (depth + 1 < maxDepth) {
                     Rng rng;
-                    if constexpr (BATCH) {
+                    if (camera) {
+                        rng.inc = cameraInc;
+                    } else if constexpr (BATCH) {
                         const PathSource ps = batchPathSource(cp, pathId);
                         rng.inc = streamInc(ps.seed, (uint32_t)ps.pixel, (uint32_t)ps.sample);
                     } else {

@@ -57,3 +57,20 @@ def test_merged_trace_in_a_batch():
         for i, want in enumerate(ref):
             assert np.array_equal(b.radiance(i), want), i
     b.close()
+
+
+def test_merged_trace_of_a_plain_pass_too_large_to_trace_whole():
+    scene = P.Scene.preset(4, 3, 100000)
+    out = []
+    for profile in (0, 1):
+        r = P.Renderer(1536, 1400)
+        r.set_scene(scene)
+        r.set_max_depth(4)
+        r.set_option(P.OPT_PROFILE_KERNELS, profile)
+        r.render(1)
+        st = r.stats()
+        out.append([r.radiance_sum(), np.array(st.bounce_rays), np.array(st.bounce_shadow)])
+        assert st.bvh_nodes > 4096 and st.stack_overflows == 0
+        r.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
