@@ -1704,7 +1704,7 @@ __device__ __forceinline__ void writePixel(const double a[3], double invSpp, int
     rgba[p] = make_uchar4(o[0], o[1], o[2], 255);
 }
 
-// A small chunk's paths from the camera to their end in one launch: a wave takes 64 paths and
+// A small chunk's paths from the camera to their end in one launch: a wave takes up to 64 paths and
 // alternates between shading its lanes' hits and tracing the shadow rays this made together with the
 // next extension rays (traceBoth), with the path state in registers.  The arithmetic is the queue kernels' own, step by step, so a
 // path's radiance is theirs bit for bit.
@@ -1780,8 +1780,8 @@ __device__ __forceinline__ TraceHit traceBoth(const PtSceneView &sc, bool alive,
 }
 
 template <int STACK, bool NEE>
-__global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, float4 *Lpath, int *pathCounters, int *spill,
-                                                           int spillCap, int *overflow) {
+__global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, int runPaths, float4 *Lpath, int *pathCounters,
+                                                           int *spill, int spillCap, int *overflow) {
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
     __shared__ ShadowList lists[NEE ? kTraceThreads / 64 : 1];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
@@ -1792,9 +1792,9 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, Chun
         const int n = __popcll(__ballot(mine));
         if (n > 0 && laneId() == 0) atomicAdd(&count[field * kMaxBounces + bounce], n);
     };
-    for (int run = wave; run < (cp.nPaths + 63) / 64; run += waves) {
-        const int path = run * 64 + laneId();
-        const bool mine = path < cp.nPaths;
+    for (int run = wave; run < (cp.nPaths + runPaths - 1) / runPaths; run += waves) {
+        const int path = run * runPaths + laneId();
+        const bool mine = laneId() < runPaths && path < cp.nPaths;
         int s, col;
         const int pixel = cp.pixBegin + chunkPixelOf(cp, mine ? path : 0, &s);
         const int row = divmodEst(pixel, cp.W, &col);
@@ -2541,6 +2541,22 @@ bool wholePaths(const pt_renderer *r, const ChunkParams &cp) {
     return cp.nPaths <= (nodes <= 16 ? 1 << 23 : nodes <= 4096 ? 1 << 22 : nodes <= 32768 ? 1 << 21 : 1 << 20);
 }
 
+// Paths per wave of k_paths.  A pass too small to fill the chip lasts as long as its slowest wave: with
+// fewer paths that wave waits for fewer, and its other lanes take the shadow rays at once instead of
+// after their own.  So as few as still fit the chip in one go (two goes cost more: 1.31M triangles,
+// 2.3e5 paths 424 us against 634).  us a pass with 64 / with 4 to 32: 1.31M triangles, 1024, 16384, 65536,
+// 1.3e5 paths 191 / 143, 275 / 205, 357 / 291, 377 / 366; room of 1M, 1024 and 65536 paths 801 / 397,
+// 957 / 823; 40k triangles 151 / 96, 197 / 184.  In small trees, whose rays are short, shading the same
+// paths in more waves costs more (Cornell box, 65536 paths: 84 / 97).
+constexpr int kMinPathsPerWave = 4;
+int pathsPerWave(const ChunkParams &cp, int nodes, int cus) {
+    if (!cp.nee || nodes <= 4096) return 64;
+    const int slots = cus * kPathBlocksPerCU * (kTraceThreads / 64);
+    for (int n = kMinPathsPerWave; n < 64; n *= 2)
+        if (cp.nPaths <= slots * n) return n;
+    return 64;
+}
+
 void accumulateChunk(pt_renderer *r, const ChunkParams &cp, bool whole, const PassEnd &end) {
     KTimer t(r, K_ACCUM);
     k_accumulate<<<(cp.npix + 255) / 256, 256, 0, r->stream>>>(cp, r->pp->Lpath.as<float4>(), r->accum.as<double>(), r->pp->counters.as<int>(),
@@ -2552,12 +2568,13 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
     int *ctr = r->pp->counters.as<int>();
     const bool guided = r->type == PT_RENDERER_GUIDED;
     if (wholePaths(r, cp)) {
-        const int grid = std::min((cp.nPaths + kTraceThreads - 1) / kTraceThreads, r->cus * kPathBlocksPerCU);
+        const int runPaths = pathsPerWave(cp, r->view.numNodes, r->cus), perBlock = runPaths * (kTraceThreads / 64);
+        const int grid = std::min((cp.nPaths + perBlock - 1) / perBlock, r->cus * kPathBlocksPerCU);
         int cap = 0;
         int *sp = ensureSpill(r, grid, &cap);
         float4 *L = r->pp->Lpath.as<float4>();
         int *pc = r->pp->pathCounters.as<int>(), *ov = r->pp->overflow.as<int>();
-        auto run = [&](auto kernel) { kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, L, pc, sp, cap, ov); };
+        auto run = [&](auto kernel) { kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, runPaths, L, pc, sp, cap, ov); };
         if (cp.nee) r->ldsStack == 32 ? run(k_paths<32, true>) : run(k_paths<16, true>);
         else r->ldsStack == 32 ? run(k_paths<32, false>) : run(k_paths<16, false>);
         PT_HIP_TRY(hipGetLastError());

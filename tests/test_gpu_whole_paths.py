@@ -76,3 +76,13 @@ def test_spilling_stacks_find_the_closest_hit(n, lds):
     assert np.array_equal(r.intersect(rays, any_hit=True)[3] == P.MISS, o.intersect(shadow, tri_test=1)[3] == P.MISS)
     assert r.stats().stack_overflows == 0
     r.close()
+
+
+@pytest.mark.parametrize("W,H", [(128, 128), (128, 129), (256, 128), (257, 128), (256, 256), (362, 362), (512, 257)])
+@pytest.mark.parametrize("kind", ["mesh", "room"])
+def test_waves_of_few_paths_equal_the_queues(W, H, kind):
+    print(f"case: {kind} {W}x{H}", flush=True)
+    scene = P.Scene.preset({"mesh": 4, "room": 2}[kind], 3, 100000)
+    args = (scene, W, H, 1, 6, True, 0, 0)
+    for k, (a, b) in enumerate(zip(_images(*args, 0), _images(*args, 1))):
+        assert np.array_equal(a, b), k
