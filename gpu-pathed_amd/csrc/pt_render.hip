@@ -2303,6 +2303,20 @@ hipEvent_t takeEvent(pt_renderer *r) {
     return r->eventPool[r->eventNext++];
 }
 
+// A pass under way.  One that fails leaves a reset that it had begun pending: the sums of the old
+// image are still there, or those of a part of the new one.
+struct PassScope {
+    pt_renderer *r;
+    bool fresh;
+    bool queued = false;
+    explicit PassScope(pt_renderer *rr) : r(rr), fresh(rr->resetPending) {}
+    ~PassScope() {
+        if (queued) return;
+        if (fresh) r->resetPending = true;
+        r->overflowStale = true;
+    }
+};
+
 struct KTimer {
     pt_renderer *r;
     int k;
@@ -3057,9 +3071,10 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
     if (spp <= 0) return fail(PT_ERR_INVALID, "pt_renderer_render_async: spp must be positive");
     PT_API_BEGIN
     const int npix = r->W * r->H;
+    PassScope pass(r);
     // a new image: its first chunk writes the accumulator instead of adding to it where that
     // chunk covers every pixel
-    bool fresh = r->resetPending;
+    bool fresh = pass.fresh;
     if (fresh) {
         r->spp = 0;
         r->resetPending = false;
@@ -3118,6 +3133,7 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
     // (the normals view's one kernel still traverses when its first blocks end)
     r->overflowStale = !r->overflowSeen || !r->overflowSeen->p || r->type == PT_RENDERER_NORMALS;
     r->inFlight = true;
+    pass.queued = true;
     return PT_OK;
     PT_API_END("pt_renderer_render_async")
 }

@@ -1,0 +1,91 @@
+"""What the renderer's host code does after a call has failed, and what it hands to kernels, on a HIP
+runtime double (host/hip_double.cpp): no GPU, allocations that fail on request, launches that are
+recorded and do not run."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+import pathed_capi as P
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as C, os, struct, sys
+double = C.CDLL({double!r}, mode=C.RTLD_GLOBAL)
+double.double_name.restype = C.c_char_p
+double.double_room.restype = C.c_size_t
+double.double_watch.argtypes = [C.c_char_p, C.c_int, C.c_size_t]
+double.double_room.argtypes = [C.c_void_p]
+sys.path.insert(0, {package!r})
+import numpy as np
+import pathed_capi as P
+
+def watch(name, index, size):
+    double.double_watch(name.encode(), index, size)
+    watch.size = size
+
+def launches():
+    # (kernel, blocks, threads, the watched argument's bytes) of each watched launch so far
+    out = []
+    for k in range(double.double_launches()):
+        grid, arg = (C.c_uint * 2)(), C.create_string_buffer(watch.size)
+        double.double_grid(k, grid)
+        double.double_arg(k, arg)
+        out.append((double.double_name(k).decode(), grid[0], grid[1], arg.raw))
+    return out
+
+def fails(code, f, *args):
+    try:
+        f(*args)
+    except P.PtError:
+        return
+    raise AssertionError("the call did not fail")
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("double") / "hip_double.so")
+    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                           os.path.join(HERE, "host", "hip_double.cpp"), "-o", lib])
+    prelude = PRELUDE.format(double=lib, package=os.path.dirname(P.__file__))
+
+    def go(body, *args):
+        res = subprocess.run([sys.executable, "-c", prelude + textwrap.dedent(body), *map(str, args)], capture_output=True, text=True, timeout=120)
+        assert res.returncode == 0, res.stdout + res.stderr
+
+    return go
+
+
+@pytest.mark.parametrize("kind", [P.RENDERER_OPTIX, P.RENDERER_GUIDED])
+def test_a_failed_pass_keeps_the_reset_pending(run, kind):
+    """A new image's first pass fails for want of memory; the next one still starts from empty sums
+    (k_accumulate's PassEnd::fresh, its last argument's first member)."""
+    run("""
+    s = P.Scene.preset(0)
+    failed = 0
+    for n in range(1, 100):
+        r = P.Renderer(8, 8)
+        r.set_type(int(sys.argv[1]))
+        r.set_scene(s)
+        watch("12k_accumulateE", 6, 4)
+        r.render(1)
+        r.reset()
+        double.double_fail_at(n)
+        try:
+            r.render(100000)   # the path pool grows
+            break
+        except P.PtError:
+            failed += 1
+        double.double_fail_at(0)
+        assert r.spp() == 0
+        r.set_option(P.OPT_POOL_PATHS, 4096)
+        r.render(1)
+        fresh = [struct.unpack("i", a)[0] for _, _, _, a in launches()]
+        assert fresh == [0, 1], (n, fresh)   # loading the scene cleared the sums for the first
+        assert r.spp() == 1
+    assert failed >= 13, failed
+    """, kind)
