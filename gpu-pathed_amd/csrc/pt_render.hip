@@ -2364,6 +2364,7 @@ void ensurePool(pt_renderer *r, int64_t need = 4096) {
     const int64_t want = ptPoolCapacity(need, r->poolWanted);
     if (r->pp->pool >= want) return;
     const size_t n = (size_t)want;
+    r->pp->pool = 0;   // until every array is there: one that fails has lost its old memory
     for (int k = 0; k < 2; k++) {
         r->pp->rayO[k].alloc(n * 16);
         r->pp->rayD[k].alloc(n * 16);

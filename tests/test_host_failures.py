@@ -37,7 +37,7 @@ def launches():
         out.append((double.double_name(k).decode(), grid[0], grid[1], arg.raw))
     return out
 
-def fails(code, f, *args):
+def fails(f, *args):
     try:
         f(*args)
     except P.PtError:
@@ -89,3 +89,25 @@ def test_a_failed_pass_keeps_the_reset_pending(run, kind):
         assert r.spp() == 1
     assert failed >= 13, failed
     """, kind)
+
+
+def test_a_pool_that_could_not_grow_is_allocated_again(run):
+    """The path pool fails to grow at each of its arrays in turn; the next pass, which the old capacity
+    would hold, gets arrays that exist and hold its queues (k_shade's path state, arguments 4 to 16)."""
+    run("""
+    s = P.Scene.preset(0)
+    for n in range(1, 14):
+        r = P.Renderer(8, 8)
+        r.set_scene(s)
+        r.set_option(P.OPT_PROFILE_KERNELS, 1)
+        r.render(1)
+        double.double_fail_at(n)
+        fails(r.render, 100000)
+        double.double_fail_at(0)
+        for arg in range(4, 17):
+            watch("7k_shade", arg, 8)
+            r.render(1)
+            assert launches()
+            for _, _, _, a in launches():
+                assert double.double_room(struct.unpack("P", a)[0]) >= 64 * 64 * 16, (n, arg)
+    """)
