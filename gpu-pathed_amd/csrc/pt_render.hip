@@ -2516,12 +2516,13 @@ void ensureGuide(pt_renderer *r) {
         PT_HIP_TRY(hipStreamSynchronize(r->stream));
         r->gAdamStep = 0;
     }
+    r->gRecCap = 0;   // until every array is there
     r->gMix.alloc((size_t)r->pp->pool * GUIDE_REC_F4 * sizeof(float4));
     r->gFeat.alloc((size_t)r->pp->pool * 2 * sizeof(float4));
-    r->gRecCap = 2 * r->pp->pool;
-    r->gRecords.alloc((size_t)r->gRecCap * GUIDE_TREC_F4 * sizeof(float4));
+    r->gRecords.alloc((size_t)(2 * r->pp->pool) * GUIDE_TREC_F4 * sizeof(float4));
     r->gRecIdx[0].alloc((size_t)r->pp->pool * 4);
     r->gRecIdx[1].alloc((size_t)r->pp->pool * 4);
+    r->gRecCap = 2 * r->pp->pool;
     r->guideReady = true;
 }
 

@@ -111,3 +111,26 @@ def test_a_pool_that_could_not_grow_is_allocated_again(run):
             for _, _, _, a in launches():
                 assert double.double_room(struct.unpack("P", a)[0]) >= 64 * 64 * 16, (n, arg)
     """)
+
+
+def test_guiding_memory_that_could_not_grow_is_allocated_again(run):
+    """The same for the arrays of a guided pass: the mixtures, features, training records and record
+    indices of the next pass (k_shade's GuideShadeArgs, argument 17)."""
+    run("""
+    s = P.Scene.preset(0)
+    for n in range(14, 19):   # after the pool's thirteen
+        r = P.Renderer(8, 8)
+        r.set_type(P.RENDERER_GUIDED)
+        r.set_option(P.OPT_GUIDE_TRAIN_STEPS, 0)
+        r.set_scene(s)
+        r.render(1)
+        double.double_fail_at(n)
+        fails(r.render, 100000)
+        double.double_fail_at(0)
+        watch("7k_shade", 17, 56)
+        r.render(1)
+        mix, feat, records, seg, rec_in, rec_out, _ = struct.unpack("PPPi4xPPf4x", launches()[0][3])   # a guided bounce
+        assert seg > 0 and double.double_room(records) >= 64 * seg * 64, n
+        for p, size in ((mix, 64), (feat, 32), (rec_in, 4), (rec_out, 4)):
+            assert double.double_room(p) >= 64 * 64 * size, (n, size)
+    """)
