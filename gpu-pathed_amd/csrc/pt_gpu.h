@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "pt_internal.h"
@@ -44,6 +45,10 @@ struct DevBuf {
         if (n == 0) return;
         PT_HIP_TRY(hipMalloc(&p, n));
         bytes = n;
+    }
+    void swap(DevBuf &o) {
+        std::swap(p, o.p);
+        std::swap(bytes, o.bytes);
     }
     template <class T> T *as() const { return (T *)p; }
 };
@@ -135,6 +140,17 @@ struct SceneArrays {
     void buildMaterials(DevBuf &records, hipStream_t stream) const;
     // Emitter records (3 float4 each) in the reference's light order; returns their number.
     int buildEmitters(DevBuf &records, hipStream_t stream) const;
+    void swap(SceneArrays &o) {
+        arrays.buf.swap(o.arrays.buf);
+        std::swap(nTri, o.nTri);
+        std::swap(nSph, o.nSph);
+        std::swap(nMat, o.nMat);
+        std::swap(pos, o.pos);
+        std::swap(sph, o.sph);
+        std::swap(triMat, o.triMat);
+        std::swap(sphMat, o.sphMat);
+        std::swap(mats, o.mats);
+    }
 };
 
 }  // namespace pt

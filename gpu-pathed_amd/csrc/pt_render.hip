@@ -2860,12 +2860,22 @@ int pt_renderer_set_scene(pt_renderer *r, const pt_scene *s) {
     if (s->mats.empty()) return fail(PT_ERR_INVALID, "pt_renderer_set_scene: scene has no materials");
     PT_API_BEGIN
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
-    r->camHost = s->cam;
-    computeCamera(r);
     // primitive records in input order (triangles, then spheres)
     const int64_t n = nt + ns;
     float lo[3], hi[3];
-    r->scene.load(*s, r->primsIn, r->normals, lo, hi, r->stream);
+    {
+        // beside the old scene, which stays where there is no memory for the new one's description
+        SceneArrays next;
+        DevBuf records, normals;
+        next.load(*s, records, normals, lo, hi, r->stream);
+        r->scene.swap(next);
+        r->primsIn.swap(records);
+        r->normals.swap(normals);
+    }
+    // from here on the old scene goes: a load that fails leaves none
+    r->hasScene = false;
+    r->camHost = s->cam;
+    computeCamera(r);
     r->prims.alloc(sizeof(float4) * 3 * (size_t)std::max<int64_t>(n, 1));
     for (int k = 0; k < 3; k++) {
         r->sceneLo[k] = std::isfinite(lo[k]) ? lo[k] : 0.f;

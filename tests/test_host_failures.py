@@ -134,3 +134,49 @@ def test_guiding_memory_that_could_not_grow_is_allocated_again(run):
         for p, size in ((mix, 64), (feat, 32), (rec_in, 4), (rec_out, 4)):
             assert double.double_room(p) >= 64 * 64 * size, (n, size)
     """)
+
+
+def test_a_scene_that_could_not_be_loaded_leaves_no_freed_memory_in_use(run):
+    """A scene load fails at each of its allocations in turn: what the renderer then does, it does with
+    memory that is there (the old scene's), or it says that it has no scene."""
+    run("""
+    def scene(n):
+        s = P.Scene()
+        m = s.add_material(P.LAMBERTIAN, (0.5, 0.5, 0.5))
+        e = s.add_material(P.LAMBERTIAN, (0, 0, 0), (1, 1, 1))
+        for _ in range(100 * n):
+            s.add_material(P.MIRROR, (1, 1, 1))   # no array of the old scene's size fits the new one's
+        tri = np.arange(9 * n, dtype=np.float32).reshape(n, 9) % 7
+        s.add_triangles(tri, np.arange(n) % 2, normals=np.ones((n, 9), np.float32))
+        s.set_environment(np.ones((4, 8, 4), np.float32))
+        return s
+
+    old, new = scene(1), scene(2)   # (trees of one node, which need no kernel to be built)
+    kept = 0
+    for n in range(1, 100):
+        r = P.Renderer(8, 8)
+        r.set_scene(old)
+        r.render(1)
+        double.double_fail_at(n)
+        try:
+            r.set_scene(new)
+            break
+        except P.PtError:
+            pass
+        double.double_fail_at(0)
+        for kernel, index, call in (("k_paths", 0, lambda: r.render(1)), ("k_materials", 0, lambda: r.set_material(1, P.LAMBERTIAN, emit=(2, 2, 2))),
+                                    ("k_emitter_flags", 0, lambda: r.set_material(1, P.LAMBERTIAN, emit=(1, 1, 1))),
+                                    ("k_emitter_flags", 1, lambda: r.set_material(1, P.LAMBERTIAN, emit=(2, 2, 2)))):
+            size = 40 if kernel == "k_paths" else 8
+            watch("%d%s" % (len(kernel), kernel), index, size)
+            try:
+                call()
+            except P.PtError as e:
+                assert "no scene" in str(e), (n, e)
+                continue
+            kept += 1
+            assert launches()
+            for p in struct.unpack("%dP" % (size // 8), launches()[-1][3]):
+                assert double.double_room(p) > 0, (n, kernel, index)
+    assert n > 10 and kept >= 8, (n, kept)
+    """)
