@@ -3680,7 +3680,7 @@ void buildWave(pt_batch *b) {
     w->cus = b->jobs[0]->cus;
     int64_t nN = 0, nP = 0, nNrm = 0, nM = 0, nE = 0;
     for (pt_renderer *r : b->jobs) {
-        nN += r->bvh.numNodes;
+        nN += std::max(r->bvh.numNodes, 1);
         nP += r->view.numPrims;
         nNrm += (int64_t)(r->normals.bytes / sizeof(float4));
         nM += r->scene.nMat;
@@ -3694,6 +3694,11 @@ void buildWave(pt_batch *b) {
     w->normals.alloc(sizeof(float4) * (size_t)std::max<int64_t>(nNrm, 1));
     w->materials.alloc(sizeof(PtMaterial) * (size_t)std::max<int64_t>(nM, 1));
     w->emitters.alloc(sizeof(float4) * 3 * (size_t)std::max<int64_t>(nE, 1));
+    // A render without primitives has a node without children (boxes that nothing hits): its rays
+    // start at its root as any other's do.
+    float empty[4 * PT_NODE_F4] = {};
+    for (int k = 0; k < 24; k++) empty[k] = k / 4 % 2 == 0 ? 1e30f : -1e30f;
+    for (int k = 24; k < 28; k++) empty[k] = asFloat(PT_EMPTY_CHILD);
     std::vector<BatchRender> table(b->jobs.size());
     int64_t oN = 0, oP = 0, oNrm = 0, oM = 0, oE = 0;
     for (size_t j = 0; j < b->jobs.size(); j++) {
@@ -3702,7 +3707,8 @@ void buildWave(pt_batch *b) {
         const int64_t nrm = (int64_t)(r->normals.bytes / sizeof(float4)), nm = r->scene.nMat;
         float4 *dn = w->nodes.as<float4>() + (size_t)PT_NODE_F4 * oN, *dp = w->prims.as<float4>() + 3 * (size_t)oP;
         float4 *de = w->emitters.as<float4>() + 3 * (size_t)oE;
-        PT_HIP_TRY(hipMemcpyAsync(dn, r->nodes.p, sizeof(float4) * PT_NODE_F4 * (size_t)nn, hipMemcpyDeviceToDevice, b->stream));
+        if (nn > 0) PT_HIP_TRY(hipMemcpyAsync(dn, r->nodes.p, sizeof(float4) * PT_NODE_F4 * (size_t)nn, hipMemcpyDeviceToDevice, b->stream));
+        else PT_HIP_TRY(hipMemcpyAsync(dn, empty, sizeof empty, hipMemcpyHostToDevice, b->stream));
         PT_HIP_TRY(hipMemcpyAsync(dp, r->prims.p, sizeof(float4) * 3 * (size_t)np, hipMemcpyDeviceToDevice, b->stream));
         if (nrm > 0)
             PT_HIP_TRY(hipMemcpyAsync(w->normals.as<float4>() + oNrm, r->normals.p, sizeof(float4) * (size_t)nrm, hipMemcpyDeviceToDevice, b->stream));
@@ -3725,7 +3731,7 @@ void buildWave(pt_batch *b) {
         R.env = r->view.env;
         R.cam = r->cam;
         R.accum = r->accum.as<double>();
-        oN += nn;
+        oN += std::max(nn, 1);
         oP += np;
         oNrm += nrm;
         oM += nm;

@@ -180,3 +180,35 @@ def test_a_scene_that_could_not_be_loaded_leaves_no_freed_memory_in_use(run):
                 assert double.double_room(p) > 0, (n, kernel, index)
     assert n > 10 and kept >= 8, (n, kept)
     """)
+
+
+@pytest.mark.parametrize("empty", [(0,), (1,), (2,), (0, 2), (0, 1, 2)])
+def test_a_batch_render_without_primitives_has_a_node_of_its_own(run, empty):
+    """Renders of an environment alone in a batch: their rays start at a node of theirs, inside the merged
+    array, that has no children (k_extend's scene view, k_raygen_batch's chunk)."""
+    run("""
+    empty = [int(a) for a in sys.argv[1:]]
+    b = P.Batch()
+    for k in range(3):
+        s = P.Scene()
+        m = s.add_material(P.LAMBERTIAN, (0.5, 0.5, 0.5))
+        if k not in empty:
+            s.add_triangles([[0, 0, 0, 1, 0, 0, 0, 1, 0]], [m])
+        s.set_environment(np.ones((2, 4, 4), np.float32))
+        b.add(s, 8, 8, 1, 2)
+    b.set_option(P.OPT_BATCH_GRAPH, 0)
+    watch("8k_extend", 0, 56)
+    b.run()
+    nodes, n_nodes = struct.unpack("5P4i", launches()[0][3])[0:7:6]
+    watch("14k_raygen_batch", 0, 96)
+    b.run()
+    renders = struct.unpack("12Q", launches()[0][3])[10]
+    size = double.double_room(renders) // 3
+    roots = [struct.unpack("i", C.string_at(renders + k * size, 4))[0] for k in range(3)]
+    assert len(set(roots)) == 3 and 0 <= min(roots) and max(roots) < n_nodes and double.double_room(nodes) >= 128 * n_nodes, (roots, n_nodes)
+    for k in empty:
+        node = C.string_at(nodes + 128 * roots[k], 128)
+        boxes = np.frombuffer(node, np.float32, 24).reshape(3, 2, 4)
+        assert np.all(boxes[:, 0] == np.float32(1e30)) and np.all(boxes[:, 1] == np.float32(-1e30))   # inverted: nothing hits them
+        assert struct.unpack("4i", node[96:112]) == (0x7fffffff,) * 4
+    """, *empty)
