@@ -3102,7 +3102,8 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
         toned = !r->profile;
         if (toned) end = passEnd(r, 1.0 / (double)(r->spp + 1));
         end.fresh = fresh ? 1 : 0;
-        const int grid = std::min((r->W + 7) / 8 * ((r->H + 7) / 8) * 64 / kTraceThreads + 1, traceGrid(r));
+        const int tiles = (r->W + 7) / 8 * ((r->H + 7) / 8);   // a wave each
+        const int grid = std::min(tiles / (kTraceThreads / 64) + 1, traceGrid(r));
         int cap = 0;
         int *sp = ensureSpill(r, grid, &cap), *ov = r->pp->overflow.as<int>();
         unsigned long long *st = r->stats.as<unsigned long long>() + S_TRACE;

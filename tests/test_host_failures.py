@@ -212,3 +212,17 @@ def test_a_batch_render_without_primitives_has_a_node_of_its_own(run, empty):
         assert np.all(boxes[:, 0] == np.float32(1e30)) and np.all(boxes[:, 1] == np.float32(-1e30))   # inverted: nothing hits them
         assert struct.unpack("4i", node[96:112]) == (0x7fffffff,) * 4
     """, *empty)
+
+
+@pytest.mark.parametrize("width,height", [(1, 1), (1 << 28, 1), (1, 1 << 28), (1 << 14, 1 << 14)])
+def test_the_normals_view_of_the_largest_images_has_a_grid(run, width, height):
+    run("""
+    r = P.Renderer(int(sys.argv[1]), int(sys.argv[2]))
+    r.set_scene(P.Scene.preset(0))
+    r.set_type(P.RENDERER_NORMALS)
+    watch("9k_normals", 0, 8)
+    r.render(1)
+    (name, blocks, threads, _), = launches()
+    assert 1 <= blocks <= 11 * 256 and threads == 128, blocks
+    assert int(sys.argv[1]) * int(sys.argv[2]) == 1 or blocks == 11 * 256
+    """, width, height)
