@@ -3097,7 +3097,6 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
     if (r->type == PT_RENDERER_NORMALS) {
         // one centre ray per pixel, added once per pass (the reference's framebuffer sees
         // spp = 1 each pass, g_buffer.cu:108-117)
-        if (npix > r->poolWanted) r->poolWanted = npix;
         PassEnd end;
         toned = !r->profile;
         if (toned) end = passEnd(r, 1.0 / (double)(r->spp + 1));

@@ -226,3 +226,18 @@ def test_the_normals_view_of_the_largest_images_has_a_grid(run, width, height):
     assert 1 <= blocks <= 11 * 256 and threads == 128, blocks
     assert int(sys.argv[1]) * int(sys.argv[2]) == 1 or blocks == 11 * 256
     """, width, height)
+
+
+def test_the_normals_view_leaves_the_pool_option(run):
+    run("""
+    r = P.Renderer(128, 96)
+    r.set_scene(P.Scene.preset(0))
+    r.set_option(P.OPT_POOL_PATHS, 4096)
+    r.set_type(P.RENDERER_NORMALS)
+    r.render(1)
+    assert r.get_option(P.OPT_POOL_PATHS) == 4096
+    r.set_type(P.RENDERER_OPTIX)
+    watch("12k_accumulateE", 0, 4)
+    r.render(1)
+    assert len(launches()) == 3   # chunks of 4096 paths
+    """)
