@@ -833,7 +833,7 @@ __global__ __launch_bounds__(256) void k_level_write(BinTree t, CollapseTables t
     o[28] = 0.f;
 }
 
-constexpr int kMaxLevels = 4096;   // of 4-wide nodes
+constexpr int kLevelGroup = 32;   // levels queued without a look at the last one's size, at most
 // Working arrays of the collapse of a tree of ni internal nodes.
 struct CollapseWork {
     unsigned *live[2], *scanTmp;
@@ -846,7 +846,7 @@ struct CollapseWork {
             w.want(live[k], (size_t)ni + 1);
             w.want(front[k], (size_t)ni);
         }
-        w.want(levels, (size_t)kMaxLevels + 1);
+        w.want(levels, (size_t)ni + kLevelGroup + 1);   // a level has a node at least
         w.want(nodes, (size_t)PT_NODE_F4 * ni);
     }
 };
@@ -861,11 +861,12 @@ int collapseWide(const BinTree &t, const CollapseTables &tb, const CollapseWork 
     // a full tree of n / 2 two-primitive leaves has this many levels; a group more where it is deeper
     int group = 1;
     for (int64_t w = 4; w * 2 < t.n; w *= 4) group++;
+    group = std::min(group, kLevelGroup);
     int level = 0, cur = 0;
     int64_t most = 1;
     WideLevel lv{1, 0};
     while (lv.m > 0) {
-        if (level + group > kMaxLevels) throw HipFailure("BVH collapse: the tree is too deep");
+        if (level > ni) throw HipFailure("BVH collapse: more levels than internal nodes");
         for (int k = 0; k < group; k++, level++) {
             exclusiveScan<unsigned>(cw.live[cur], (int)most, cw.scanTmp, stream, &cw.levels[level].m);
             k_level_write<<<blocks(4 * most, 256), 256, 0, stream>>>(t, tb, cw.front[cur], cw.levels + level, cw.live[cur], cw.front[1 - cur],
