@@ -298,6 +298,22 @@ void faultIn(char *p, size_t len) {
 
 namespace {
 
+// Makes a device current until it goes.
+struct DeviceScope {
+    int before = 0;
+    bool other = false;
+    explicit DeviceScope(int device) {
+        PT_HIP_TRY(hipGetDevice(&before));
+        other = before != device;
+        if (other) PT_HIP_TRY(hipSetDevice(device));
+    }
+    ~DeviceScope() {
+        if (other) (void)hipSetDevice(before);
+    }
+    DeviceScope(const DeviceScope &) = delete;
+    DeviceScope &operator=(const DeviceScope &) = delete;
+};
+
 // Staging memory and its events, of one device.
 struct ReadStage {
     int device = 0;
@@ -393,8 +409,10 @@ HostWord::~HostWord() {
 
 void readToHost(void *dst, const void *src, size_t bytes, hipStream_t stream) {
     if (bytes == 0) return;
+    // a stream takes events of its own device only, which need not be this thread's
     int device = 0;
-    PT_HIP_TRY(hipGetDevice(&device));
+    PT_HIP_TRY(hipStreamGetDevice(stream, &device));
+    const DeviceScope on(device);
     // about six pieces
     const size_t piece = std::clamp<size_t>(bytes / 6 / 256 * 256, kReadPieceMin, kReadPieceMax);
     std::unique_ptr<ReadStage> stage = stageKeeper().take(device);

@@ -241,3 +241,28 @@ def test_the_normals_view_leaves_the_pool_option(run):
     r.render(1)
     assert len(launches()) == 3   # chunks of 4096 paths
     """)
+
+
+def test_images_are_read_from_any_thread_and_device(run):
+    """A renderer of one device read while another is current, and from a thread that never chose one: the
+    events of the copy are of the stream's device, and the caller's device stays what it was."""
+    run("""
+    import threading
+    double.double_devices(2)
+    current = C.c_int()
+    for own, other in ((0, 1), (1, 0)):
+        assert double.hipSetDevice(own) == 0
+        r = P.Renderer(40, 30)
+        r.set_scene(P.Scene.preset(0))
+        r.render(1)
+        assert double.hipSetDevice(other) == 0
+        for read in (r.radiance, r.radiance_sum, r.rgba8):
+            read()
+            double.hipGetDevice(C.byref(current))
+            assert current.value == other
+        read = []
+        t = threading.Thread(target=lambda: read.append(r.radiance()))
+        t.start()
+        t.join()
+        assert len(read) == 1
+    """)
