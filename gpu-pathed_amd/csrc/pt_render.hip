@@ -1717,7 +1717,9 @@ __device__ __forceinline__ void writePixel(const double a[3], double invSpp, int
 // lanes between bounces did not help (2048x1024 of 327k triangles 1603 -> 1693 us: the lanes'
 // different depths spilled more state than they filled idle time), nor did 8 x 8 pixel tiles
 // instead of 64 pixels of a row (327k triangles at 1024^2 882 -> 923 us, at 256^2 306 -> 289).
-static constexpr int kPathBlocksPerCU = 8;   // of two waves: four waves per SIMD
+// Blocks of two waves per CU: eight, four waves per SIMD, as the registers allow; 32 stack rows and the
+// shadow lists take 25 KB of LDS a block, which leaves room for six.
+constexpr int pathBlocksPerCU(int rows, bool nee) { return rows > 16 && nee ? 6 : 8; }
 // A wave's shadow rays of a bounce and what came of them.
 struct ShadowList {
     float o[3][64], d[3][64], tmax[64], contrib[3][64];
@@ -1780,7 +1782,7 @@ __device__ __forceinline__ TraceHit traceBoth(const PtSceneView &sc, bool alive,
 }
 
 template <int STACK, bool NEE>
-__global__ __launch_bounds__(kTraceThreads, 4) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, int runPaths, float4 *Lpath, int *pathCounters,
+__global__ __launch_bounds__(kTraceThreads, pathBlocksPerCU(STACK, NEE) / 2) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, int runPaths, float4 *Lpath, int *pathCounters,
                                                            int *spill, int spillCap, int *overflow) {
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
     __shared__ ShadowList lists[NEE ? kTraceThreads / 64 : 1];
@@ -2565,9 +2567,9 @@ bool wholePaths(const pt_renderer *r, const ChunkParams &cp) {
 // 957 / 823; 40k triangles 151 / 96, 197 / 184.  In small trees, whose rays are short, shading the same
 // paths in more waves costs more (Cornell box, 65536 paths: 84 / 97).
 constexpr int kMinPathsPerWave = 4;
-int pathsPerWave(const ChunkParams &cp, int nodes, int cus) {
+int pathsPerWave(const ChunkParams &cp, int nodes, int resident) {
     if (!cp.nee || nodes <= 4096) return 64;
-    const int slots = cus * kPathBlocksPerCU * (kTraceThreads / 64);
+    const int slots = resident * (kTraceThreads / 64);
     for (int n = kMinPathsPerWave; n < 64; n *= 2)
         if (cp.nPaths <= slots * n) return n;
     return 64;
@@ -2584,8 +2586,9 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
     int *ctr = r->pp->counters.as<int>();
     const bool guided = r->type == PT_RENDERER_GUIDED;
     if (wholePaths(r, cp)) {
-        const int runPaths = pathsPerWave(cp, r->view.numNodes, r->cus), perBlock = runPaths * (kTraceThreads / 64);
-        const int grid = std::min((cp.nPaths + perBlock - 1) / perBlock, r->cus * kPathBlocksPerCU);
+        const int resident = r->cus * pathBlocksPerCU(r->ldsStack, cp.nee != 0);
+        const int runPaths = pathsPerWave(cp, r->view.numNodes, resident), perBlock = runPaths * (kTraceThreads / 64);
+        const int grid = std::min((cp.nPaths + perBlock - 1) / perBlock, resident);
         int cap = 0;
         int *sp = ensureSpill(r, grid, &cap);
         float4 *L = r->pp->Lpath.as<float4>();

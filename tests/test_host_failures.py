@@ -266,3 +266,20 @@ def test_images_are_read_from_any_thread_and_device(run):
         t.join()
         assert len(read) == 1
     """)
+
+
+@pytest.mark.parametrize("lds,nee,blocks", [(16, 1, 8), (16, 0, 8), (32, 1, 6), (32, 0, 8)])
+def test_whole_path_grids_are_what_fits_the_chip(run, lds, nee, blocks):
+    """Blocks of k_paths per CU by their LDS (160 KB; 11 KB of 16 stack rows, 19 KB of 32, 5.5 KB of shadow
+    lists) and registers: a second go of a few blocks takes as long as the first."""
+    run("""
+    lds, nee, blocks = (int(a) for a in sys.argv[1:])
+    r = P.Renderer(1024, 1024)
+    r.set_scene(P.Scene.preset(0))
+    r.set_option(P.OPT_TRACE_LDS_STACK, lds)
+    r.set_nee(nee)
+    watch("7k_paths", 3, 4)
+    r.render(1)
+    (_, grid, threads, _), = launches()
+    assert grid == 256 * blocks and threads == 128, grid
+    """, lds, nee, blocks)
