@@ -2546,17 +2546,18 @@ GuideSceneNorm guideNorm(pt_renderer *r) {
     return nm;
 }
 
-// Whether a chunk's paths are traced whole (k_paths) or through the queues.  us a pass, queues /
-// whole: 2^16 paths: Cornell box (3 nodes) 342 / 86, 1.31M triangles (319k nodes) 857 / 359; 2^20:
-// 1.31M 1516 / 991, room of 1M (246k nodes, depth 16) 4787 / 4225; 2^21: 82k triangles (20k nodes)
-// 1295 / 1034, room of 100k (25k nodes) 5852 / 5522, 1.31M 1879 / 1643, room of 1M 7233 / 8299; 2^22:
-// 294 nodes 1195 / 1036, 1226 nodes 1366 / 1260, 20k nodes 1855 / 1888; 2^23: Cornell box 3424 /
-// 2585, 17 nodes 1256 / 1229, 294 nodes 1785 / 1939.  The timed and the counting kernels are the
-// queues', and so are a batch's: its chunks are filled with paths of several renders.
+// Whether a chunk's paths are traced whole (k_paths) or through the queues.  Above these sizes it depends
+// on the scene, not on its size, which is faster: queues / whole time at 2^20, 2^21 and 2^22 paths of
+// triangle or sphere soups (rays of a wave part early) 0.98 to 1.7, 0.72 to 1.1 and 0.45 to 0.87, of
+// displaced spheres of 1k to 100k triangles 1.5 to 2.0, 1.2 to 1.5 and 0.84 to 1.2, of rooms 1.1 to 1.7,
+// 0.82 to 1.1 and 0.64 to 0.96.  Trees of 5 to 16 nodes 1.2 to 3.8, 0.89 to 2.8 and 0.61 to 1.9; of up to
+// 4 1.9 to 5.0, 1.4 to 3.9 and 0.90 to 2.6, Cornell box (3 nodes) 2.0, 1.6 and 1.4, at 2^23 0.79.  The
+// timed and the counting kernels are the queues', and so are a batch's: its chunks are filled with paths
+// of several renders.
 bool wholePaths(const pt_renderer *r, const ChunkParams &cp) {
     if (r->type == PT_RENDERER_GUIDED || r->profile || r->traceStats || !r->ownsStream) return false;
     const int nodes = r->view.numNodes;
-    return cp.nPaths <= (nodes <= 16 ? 1 << 23 : nodes <= 4096 ? 1 << 22 : nodes <= 32768 ? 1 << 21 : 1 << 20);
+    return cp.nPaths <= (nodes <= 4 ? 1 << 22 : nodes <= 16 ? 1 << 21 : 1 << 20);
 }
 
 // Paths per wave of k_paths.  A pass too small to fill the chip lasts as long as its slowest wave: with

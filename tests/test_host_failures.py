@@ -283,3 +283,16 @@ def test_whole_path_grids_are_what_fits_the_chip(run, lds, nee, blocks):
     (_, grid, threads, _), = launches()
     assert grid == 256 * blocks and threads == 128, grid
     """, lds, nee, blocks)
+
+
+def test_whole_paths_up_to_the_limit(run):
+    run("""
+    s = P.Scene()
+    s.add_triangles([[0, 0, 0, 1, 0, 0, 0, 1, 0]], [s.add_material(P.LAMBERTIAN, (0.5, 0.5, 0.5))])   # one node
+    for height, whole in ((2048, 1), (2049, 0)):
+        r = P.Renderer(2048, height)
+        r.set_scene(s)
+        watch("7k_paths", 3, 4)
+        r.render(1)
+        assert len(launches()) == whole
+    """)
