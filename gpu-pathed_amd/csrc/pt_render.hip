@@ -1876,12 +1876,17 @@ __global__ __launch_bounds__(kTraceThreads, pathBlocksPerCU(STACK, NEE) / 2) voi
     }
 }
 
+// Waves' worth of pixels of an image, in 8 x 8 tiles or in order.
+__host__ __device__ constexpr int normalsRuns(int W, int H, int tiled) { return tiled ? (W + 7) / 8 * ((H + 7) / 8) : (W * H + 63) / 64; }
+
 // Normals view (g_buffer.cu:27-57): colour (n + 1) / 2 of the primary hit at the pixel centre, in one
 // launch: ray, traversal, FP64 accumulator and framebuffers.  Bound by the traversal, as k_extend.
 // 1280x720 of 327k triangles: 176 us (201 us with 64 pixels of a row to a wave) against 228 us in
-// the five kernels before.
+// the five kernels before.  An image whose edge tiles leave more than an eighth of the lanes without a
+// pixel goes by 64 pixels in order instead (one column of 2^20 pixels, 100k triangles: 655 us in tiles,
+// 132 in order, 176 in the five kernels; one row 124, 44, 79).
 template <int STACK, bool STATS>
-__global__ __launch_bounds__(kTraceThreads, 4) void k_normals(PtSceneView sc, PtCamera cam, double *accum, PassEnd end, int *spill,
+__global__ __launch_bounds__(kTraceThreads, 4) void k_normals(PtSceneView sc, PtCamera cam, int tiled, double *accum, PassEnd end, int *spill,
                                                              int spillCap, int *overflow, unsigned long long *tstat) {
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
@@ -1889,12 +1894,21 @@ __global__ __launch_bounds__(kTraceThreads, 4) void k_normals(PtSceneView sc, Pt
     TraceCount tc;
     // a wave takes 8 x 8 pixels, in Morton order: where neighbouring lanes are at the same node, one
     // L1 access serves four
-    const int tilesX = (cam.W + 7) / 8, tiles = tilesX * ((cam.H + 7) / 8);
-    for (int tile = wave; tile < tiles; tile += waves) {
-        int tx;
-        const int ty = divmodEst(tile, tilesX, &tx), l = laneId();
-        const int col = 8 * tx + ((l & 1) | (l >> 1 & 2) | (l >> 2 & 4)), row = 8 * ty + ((l >> 1 & 1) | (l >> 2 & 2) | (l >> 3 & 4));
-        const bool mine = col < cam.W && row < cam.H;
+    const int npix = cam.W * cam.H, tilesX = (cam.W + 7) / 8, runs = normalsRuns(cam.W, cam.H, tiled);
+    for (int run = wave; run < runs; run += waves) {
+        const int l = laneId();
+        int row, col;
+        bool mine;
+        if (tiled) {
+            int tx;
+            const int ty = divmodEst(run, tilesX, &tx);
+            col = 8 * tx + ((l & 1) | (l >> 1 & 2) | (l >> 2 & 4));
+            row = 8 * ty + ((l >> 1 & 1) | (l >> 2 & 2) | (l >> 3 & 4));
+            mine = col < cam.W && row < cam.H;
+        } else {
+            mine = 64 * run + l < npix;
+            row = divmodEst(mine ? 64 * run + l : 0, cam.W, &col);
+        }
         f3 o, d;
         cameraRay(cam, row, col, 0.5f, 0.5f, &o, &d);
         LaneRay r;
@@ -3105,14 +3119,14 @@ int pt_renderer_render_async(pt_renderer *r, int spp) {
         toned = !r->profile;
         if (toned) end = passEnd(r, 1.0 / (double)(r->spp + 1));
         end.fresh = fresh ? 1 : 0;
-        const int tiles = (r->W + 7) / 8 * ((r->H + 7) / 8);   // a wave each
-        const int grid = std::min(tiles / (kTraceThreads / 64) + 1, traceGrid(r));
+        const int tiled = 8 * (int64_t)npix >= 7 * 64 * (int64_t)normalsRuns(r->W, r->H, 1) ? 1 : 0;
+        const int grid = std::min(normalsRuns(r->W, r->H, tiled) / (kTraceThreads / 64) + 1, traceGrid(r));
         int cap = 0;
         int *sp = ensureSpill(r, grid, &cap), *ov = r->pp->overflow.as<int>();
         unsigned long long *st = r->stats.as<unsigned long long>() + S_TRACE;
         auto *kernel = r->ldsStack == 32 ? (r->traceStats ? k_normals<32, true> : k_normals<32, false>)
                                          : (r->traceStats ? k_normals<16, true> : k_normals<16, false>);
-        kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, r->cam, r->accum.as<double>(), end, sp, cap, ov, st);
+        kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, r->cam, tiled, r->accum.as<double>(), end, sp, cap, ov, st);
         PT_HIP_TRY(hipGetLastError());
         r->spp += 1;
         r->passSpp = spp;
