@@ -91,6 +91,25 @@ public:
     int *p = nullptr;
 };
 
+// An int that a kernel writes and the host reads once the stream is idle.
+class HostInt {
+public:
+    int *target() {
+        if (!word.p) own.alloc(sizeof(int));
+        return word.p ? word.p : own.as<int>();
+    }
+    int read() const {
+        int v = 0;
+        if (word.p) v = *(volatile int *)word.p;
+        else PT_HIP_TRY(hipMemcpy(&v, own.p, sizeof v, hipMemcpyDeviceToHost));
+        return v;
+    }
+
+private:
+    HostWord word;
+    DevBuf own;   // where no pinned word was to be had
+};
+
 struct BvhInfo {
     int numNodes = 0;      // 4-wide nodes
     int depth = 0;         // levels of 4-wide nodes
@@ -135,11 +154,13 @@ struct SceneArrays {
     // Uploads s and writes its primitive records (triangles, then spheres), the per-vertex
     // normals that differ from the flat ones, and the bounds (+-infinity without primitives).
     void load(const pt_scene &s, DevBuf &records, DevBuf &normals, float lo[3], float hi[3], hipStream_t stream);
-    HostMaterial material(int id, hipStream_t stream) const;
-    void setMaterial(int id, const HostMaterial &m, DevBuf &records, hipStream_t stream);
     void buildMaterials(DevBuf &records, hipStream_t stream) const;
     // Emitter records (3 float4 each) in the reference's light order; returns their number.
-    int buildEmitters(DevBuf &records, hipStream_t stream) const;
+    int buildEmitters(DevBuf &records, HostInt &answer, hipStream_t stream) const;
+    // A material's new values, in place; null colours stay.  The emitters' number: they are listed again
+    // where the material is emissive now or was.
+    int editMaterial(int id, int type, const float *albedo, const float *emit, float ior, float alpha, DevBuf &materials, DevBuf &emitters,
+                     int emittersNow, HostInt &answer, hipStream_t stream);
     void swap(SceneArrays &o) {
         arrays.buf.swap(o.arrays.buf);
         std::swap(nTri, o.nTri);

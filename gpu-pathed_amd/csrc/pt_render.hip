@@ -2267,8 +2267,9 @@ struct pt_renderer {
     DevBuf accum, radiance, rgba, stats;
     // the traversal's overflow count as of the last pass, written by its last kernel; stale after
     // traversals outside a pass
-    std::unique_ptr<HostWord> overflowSeen, picked;
+    std::unique_ptr<HostWord> overflowSeen;
     bool overflowStale = true;
+    HostInt answer;   // of a pick or a material edit
     int64_t spp = 0;
     bool resetPending = false;
     // pass tracking
@@ -2367,7 +2368,7 @@ void computeCamera(pt_renderer *r) {
 
 // The emitter list, rebuilt after edits so that emission changes also change it.
 void buildEmitters(pt_renderer *r) {
-    r->view.numEmitters = r->scene.buildEmitters(r->emitters, r->stream);
+    r->view.numEmitters = r->scene.buildEmitters(r->emitters, r->answer, r->stream);
     r->view.emitters = r->emitters.as<float4>();
 }
 
@@ -2970,15 +2971,8 @@ int pt_renderer_set_material(pt_renderer *r, int id, int type, const float albed
     if (r->inFlight) return fail(PT_ERR_STATE, "pt_renderer_set_material: a pass is still running");
     PT_API_BEGIN
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
-    HostMaterial m = r->scene.material(id, r->stream);
-    const bool wasEmissive = isEmissive(m);
-    m.type = type;
-    if (albedo) memcpy(m.albedo, albedo, 12);
-    if (emit) memcpy(m.emit, emit, 12);
-    m.ior = ior;
-    m.alpha = alpha;
-    r->scene.setMaterial(id, m, r->materials, r->stream);
-    if (wasEmissive || isEmissive(m)) buildEmitters(r);
+    r->view.numEmitters = r->scene.editMaterial(id, type, albedo, emit, ior, alpha, r->materials, r->emitters, r->view.numEmitters, r->answer, r->stream);
+    r->view.emitters = r->emitters.as<float4>();
     r->resetPending = true;
     return PT_OK;
     PT_API_END("pt_renderer_set_material")
@@ -3279,19 +3273,14 @@ int pt_renderer_hit_test(pt_renderer *r, int x, int y, int *material_id, int *is
         ro = make_float4(c.m[0][3], c.m[1][3], c.m[2][3], 0.f);
         rd = make_float4(d[0], d[1], d[2], FLT_MAX);
     }
-    if (!r->picked) r->picked = std::make_unique<HostWord>();
-    DevBuf own;   // where no pinned word was to be had
-    if (!r->picked->p) own.alloc(sizeof(int));
-    int *seen = r->picked->p ? r->picked->p : own.as<int>();
+    int *seen = r->answer.target();
     int cap = 0;
     int *sp = ensureSpill(r, 1, &cap), *ov = r->pp->overflow.as<int>();
     if (r->ldsStack == 32) k_pick<32><<<1, 64, 0, r->stream>>>(r->view, ro, rd, sp, cap, ov, seen);
     else k_pick<16><<<1, 64, 0, r->stream>>>(r->view, ro, rd, sp, cap, ov, seen);
     PT_HIP_TRY(hipGetLastError());
     PT_HIP_TRY(hipStreamSynchronize(r->stream));
-    int mat = -1;
-    if (r->picked->p) mat = *(volatile int *)r->picked->p;
-    else PT_HIP_TRY(hipMemcpy(&mat, own.p, sizeof mat, hipMemcpyDeviceToHost));
+    const int mat = r->answer.read();
     if (material_id) *material_id = mat;
     if (is_hit) *is_hit = mat >= 0 ? 1 : 0;
     return PT_OK;

@@ -130,14 +130,40 @@ __device__ __forceinline__ bool emits(const HostMaterial &m) {
     return m.type == PT_LAMBERTIAN && (m.emit[0] != 0.f || m.emit[1] != 0.f || m.emit[2] != 0.f);
 }
 
-__global__ __launch_bounds__(kThreads) void k_materials(const HostMaterial *mats, int first, int n, PtMaterial *out) {
-    const int i = first + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= first + n) return;
-    const HostMaterial h = mats[i];
+__device__ __forceinline__ void writeMaterial(const HostMaterial &h, PtMaterial *out) {
     const bool lamb = h.type == PT_LAMBERTIAN;
     const float param = h.type == PT_GLASS ? h.ior : (h.type == PT_MICROFACET ? h.alpha : 0.f);
-    out[i].a = make_float4(h.albedo[0], h.albedo[1], h.albedo[2], (float)h.type);
-    out[i].b = make_float4(lamb ? h.emit[0] : 0.f, lamb ? h.emit[1] : 0.f, lamb ? h.emit[2] : 0.f, param);
+    out->a = make_float4(h.albedo[0], h.albedo[1], h.albedo[2], (float)h.type);
+    out->b = make_float4(lamb ? h.emit[0] : 0.f, lamb ? h.emit[1] : 0.f, lamb ? h.emit[2] : 0.f, param);
+}
+
+__global__ __launch_bounds__(kThreads) void k_materials(const HostMaterial *mats, int n, PtMaterial *out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) writeMaterial(mats[i], &out[i]);
+}
+
+// An edit of one material: the kept one and its record, or of id -1 none.  True where it was or is
+// emissive.
+struct MaterialEdit {
+    int id = -1, setAlbedo = 0, setEmit = 0;
+    HostMaterial to{};
+};
+__device__ __forceinline__ bool applyEdit(const MaterialEdit &e, HostMaterial *mats, PtMaterial *records) {
+    const HostMaterial was = mats[e.id];
+    HostMaterial to = e.to;
+    for (int k = 0; k < 3; k++) {
+        if (!e.setAlbedo) to.albedo[k] = was.albedo[k];
+        if (!e.setEmit) to.emit[k] = was.emit[k];
+    }
+    mats[e.id] = to;
+    writeMaterial(to, &records[e.id]);
+    return emits(was) || emits(to);
+}
+
+// The host waits for what it needs to know, which this writes to pinned memory: reading the material back,
+// changing it and copying it up again took 37 us a call, this 15.
+__global__ void k_edit_material(MaterialEdit e, HostMaterial *mats, PtMaterial *records, int *emissive) {
+    if (threadIdx.x == 0) *emissive = applyEdit(e, mats, records) ? 1 : 0;
 }
 
 __global__ __launch_bounds__(kThreads) void k_emitter_flags(const HostMaterial *mats, const int *triMat, int nt, const int *sphMat, int ns,
@@ -149,26 +175,61 @@ __global__ __launch_bounds__(kThreads) void k_emitter_flags(const HostMaterial *
 
 // Emitter records in the reference light order (scene_data.cu:92-115): emissive triangles by
 // index, then emissive spheres.  Their normals are the flat ones.
+__device__ __forceinline__ void writeEmitter(const float *pos, const int *triMat, int nt, const float *sph, const int *sphMat, int i, float4 *o) {
+    if (i < nt) {
+        const float *p = pos + 9 * (size_t)i;
+        o[0] = make_float4(p[0], p[1], p[2], asFloat(triMat[i]));
+        o[1] = make_float4(p[3], p[4], p[5], asFloat(PT_TAG_FLAT));
+        o[2] = make_float4(p[6], p[7], p[8], asFloat(i));
+    } else {
+        const int k = i - nt;
+        const float *s = sph + 4 * (size_t)k;
+        o[0] = make_float4(s[0], s[1], s[2], asFloat(sphMat[k]));
+        o[1] = make_float4(s[3], 0.f, 0.f, asFloat(PT_TAG_SPHERE));
+        o[2] = make_float4(0.f, 0.f, 0.f, asFloat(~k));
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void k_emitters(const HostMaterial *mats, const float *pos, const int *triMat, int nt, const float *sph,
                                                        const int *sphMat, int ns, const uint32_t *rank, float4 *out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nt + ns) return;
-    float4 *o = out + 3 * (size_t)rank[i];
-    if (i < nt) {
-        const int mat = triMat[i];
-        if (!emits(mats[mat])) return;
-        const float *p = pos + 9 * (size_t)i;
-        o[0] = make_float4(p[0], p[1], p[2], asFloat(mat));
-        o[1] = make_float4(p[3], p[4], p[5], asFloat(PT_TAG_FLAT));
-        o[2] = make_float4(p[6], p[7], p[8], asFloat(i));
-    } else {
-        const int k = i - nt, mat = sphMat[k];
-        if (!emits(mats[mat])) return;
-        const float *s = sph + 4 * (size_t)k;
-        o[0] = make_float4(s[0], s[1], s[2], asFloat(mat));
-        o[1] = make_float4(s[3], 0.f, 0.f, asFloat(PT_TAG_SPHERE));
-        o[2] = make_float4(0.f, 0.f, 0.f, asFloat(~k));
+    if (emits(mats[i < nt ? triMat[i] : sphMat[i - nt]])) writeEmitter(pos, triMat, nt, sph, sphMat, i, out + 3 * (size_t)rank[i]);
+}
+
+// The list by one block, and its length, for scenes of up to kEmittersSmall primitives, after an edit or
+// without one; an edit that has nothing to do with emission leaves the list of `now` emitters.  Flags,
+// prefix sums, the length's way to the host and the records' allocation took half of an emission edit's
+// 74 us; with the edit in the same launch it takes 16.
+constexpr int kEmittersSmall = 2048;
+constexpr int kEmittersThreads = 1024;
+__global__ __launch_bounds__(kEmittersThreads) void k_emitters_small(MaterialEdit e, HostMaterial *mats, PtMaterial *records, const float *pos,
+                                                                     const int *triMat, int nt, const float *sph, const int *sphMat, int ns, int now,
+                                                                     float4 *out, int *count) {
+    __shared__ int sWave[kEmittersThreads / 64], sList;
+    if (threadIdx.x == 0) sList = e.id < 0 || applyEdit(e, mats, records) ? 1 : 0;
+    __syncthreads();
+    if (sList == 0) {
+        if (threadIdx.x == 0) *count = now;
+        return;
     }
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int base = 0;
+    for (int i0 = 0; i0 < nt + ns; i0 += kEmittersThreads) {
+        const int i = i0 + threadIdx.x;
+        const bool mine = i < nt + ns && emits(mats[i < nt ? triMat[i] : sphMat[i - nt]]);
+        const uint64_t m = __ballot(mine);
+        if (lane == 0) sWave[wave] = __popcll(m);
+        __syncthreads();
+        int at = base + __popcll(m & ((1ull << lane) - 1));
+        for (int w = 0; w < kEmittersThreads / 64; w++) {
+            if (w < wave) at += sWave[w];
+            base += sWave[w];
+        }
+        if (mine) writeEmitter(pos, triMat, nt, sph, sphMat, i, out + 3 * (size_t)at);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *count = base;
 }
 
 template <class T> void upload(T *d, const std::vector<T> &v, hipStream_t stream) {
@@ -232,39 +293,31 @@ void SceneArrays::load(const pt_scene &s, DevBuf &records, DevBuf &normals, floa
     }
 }
 
-HostMaterial SceneArrays::material(int id, hipStream_t stream) const {
-    HostMaterial m;
-    PT_HIP_TRY(hipMemcpyAsync(&m, mats + id, sizeof m, hipMemcpyDeviceToHost, stream));
-    PT_HIP_TRY(hipStreamSynchronize(stream));
-    return m;
-}
-
-void SceneArrays::setMaterial(int id, const HostMaterial &m, DevBuf &records, hipStream_t stream) {
-    PT_HIP_TRY(hipMemcpyAsync(mats + id, &m, sizeof m, hipMemcpyHostToDevice, stream));
-    k_materials<<<1, kThreads, 0, stream>>>(mats, id, 1, records.as<PtMaterial>());
-    PT_HIP_TRY(hipGetLastError());
-    PT_HIP_TRY(hipStreamSynchronize(stream));
-}
-
 void SceneArrays::buildMaterials(DevBuf &records, hipStream_t stream) const {
     records.alloc(sizeof(PtMaterial) * (size_t)std::max(nMat, 1));
-    if (nMat > 0) k_materials<<<blocksOf(nMat), kThreads, 0, stream>>>(mats, 0, nMat, records.as<PtMaterial>());
+    if (nMat > 0) k_materials<<<blocksOf(nMat), kThreads, 0, stream>>>(mats, nMat, records.as<PtMaterial>());
     PT_HIP_TRY(hipGetLastError());
 }
 
-int SceneArrays::buildEmitters(DevBuf &records, hipStream_t stream) const {
+int SceneArrays::buildEmitters(DevBuf &records, HostInt &answer, hipStream_t stream) const {
     const int n = nTri + nSph;
+    if (n <= kEmittersSmall) {
+        records.alloc(sizeof(float4) * 3 * (size_t)std::max(n, 1));
+        k_emitters_small<<<1, kEmittersThreads, 0, stream>>>(MaterialEdit{}, mats, nullptr, pos, triMat, nTri, sph, sphMat, nSph, 0, records.as<float4>(),
+                                                             answer.target());
+        PT_HIP_TRY(hipGetLastError());
+        PT_HIP_TRY(hipStreamSynchronize(stream));
+        return answer.read();
+    }
     uint32_t count = 0, *rank, *scanTmp;
     WorkArrays work;
-    if (n > 0) {
-        work.want(rank, (size_t)n + 1);
-        work.want(scanTmp, scanEntries(n));
-        work.alloc();
-        k_emitter_flags<<<blocksOf(n), kThreads, 0, stream>>>(mats, triMat, nTri, sphMat, nSph, rank);
-        scanCounts(rank, n, scanTmp, stream);
-        PT_HIP_TRY(hipMemcpyAsync(&count, rank + n, sizeof count, hipMemcpyDeviceToHost, stream));
-        PT_HIP_TRY(hipStreamSynchronize(stream));
-    }
+    work.want(rank, (size_t)n + 1);
+    work.want(scanTmp, scanEntries(n));
+    work.alloc();
+    k_emitter_flags<<<blocksOf(n), kThreads, 0, stream>>>(mats, triMat, nTri, sphMat, nSph, rank);
+    scanCounts(rank, n, scanTmp, stream);
+    PT_HIP_TRY(hipMemcpyAsync(&count, rank + n, sizeof count, hipMemcpyDeviceToHost, stream));
+    PT_HIP_TRY(hipStreamSynchronize(stream));
     records.alloc(sizeof(float4) * std::max<size_t>(3 * (size_t)count, 1));
     if (count > 0) {
         k_emitters<<<blocksOf(n), kThreads, 0, stream>>>(mats, pos, triMat, nTri, sph, sphMat, nSph, rank, records.as<float4>());
@@ -273,6 +326,28 @@ int SceneArrays::buildEmitters(DevBuf &records, hipStream_t stream) const {
         PT_HIP_TRY(hipStreamSynchronize(stream));
     }
     return (int)count;
+}
+
+int SceneArrays::editMaterial(int id, int type, const float *albedo, const float *emit, float ior, float alpha, DevBuf &materials, DevBuf &emitters,
+                              int emittersNow, HostInt &answer, hipStream_t stream) {
+    MaterialEdit e;
+    e.id = id;
+    e.setAlbedo = albedo ? 1 : 0;
+    e.setEmit = emit ? 1 : 0;
+    e.to.type = type;
+    if (albedo) memcpy(e.to.albedo, albedo, sizeof e.to.albedo);
+    if (emit) memcpy(e.to.emit, emit, sizeof e.to.emit);
+    e.to.ior = ior;
+    e.to.alpha = alpha;
+    const bool small = nTri + nSph <= kEmittersSmall;
+    if (small)
+        k_emitters_small<<<1, kEmittersThreads, 0, stream>>>(e, mats, materials.as<PtMaterial>(), pos, triMat, nTri, sph, sphMat, nSph, emittersNow,
+                                                             emitters.as<float4>(), answer.target());
+    else k_edit_material<<<1, 64, 0, stream>>>(e, mats, materials.as<PtMaterial>(), answer.target());
+    PT_HIP_TRY(hipGetLastError());
+    PT_HIP_TRY(hipStreamSynchronize(stream));
+    if (small) return answer.read();
+    return answer.read() != 0 ? buildEmitters(emitters, answer, stream) : emittersNow;
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -164,9 +164,8 @@ def test_a_scene_that_could_not_be_loaded_leaves_no_freed_memory_in_use(run):
         except P.PtError:
             pass
         double.double_fail_at(0)
-        for kernel, index, call in (("k_paths", 0, lambda: r.render(1)), ("k_materials", 0, lambda: r.set_material(1, P.LAMBERTIAN, emit=(2, 2, 2))),
-                                    ("k_emitter_flags", 0, lambda: r.set_material(1, P.LAMBERTIAN, emit=(1, 1, 1))),
-                                    ("k_emitter_flags", 1, lambda: r.set_material(1, P.LAMBERTIAN, emit=(2, 2, 2)))):
+        edit = lambda: r.set_material(1, P.LAMBERTIAN, emit=(2, 2, 2))
+        for kernel, index, call in [("k_paths", 0, lambda: r.render(1))] + [("k_emitters_small", k, edit) for k in (1, 2, 3, 4, 10)]:
             size = 40 if kernel == "k_paths" else 8
             watch("%d%s" % (len(kernel), kernel), index, size)
             try:
