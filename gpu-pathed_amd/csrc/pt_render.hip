@@ -72,9 +72,8 @@ static constexpr int kTraceThreads = 128;
 // Default path-pool capacity: 2^26 paths (about 13 GB of SoA path state), a whole 1024^2 x
 // 64 spp pass in one chunk, so that every bounce's queues stay long.
 static constexpr int64_t kDefaultPool = 1ll << 26;
-// Trace blocks of 128 threads per CU: 14 would fill the 7 waves per SIMD that the trace
-// kernels' 72 VGPRs and 8 KiB of LDS stack per block allow; 11 measured best on C1 (10: 4156,
-// 11: 4185, 12: 4123, 14: 4095 Mrays/s), fewer waves sharing each CU's caches.
+// Trace blocks of 128 threads per CU: as many as a CU's 160 KB of LDS hold of k_trace's 14.5 KB (stack
+// columns and top nodes), 5.5 waves per SIMD; its 80 VGPRs would admit 6.
 static constexpr int kDefaultTraceBlocks = 11;
 // Binary tree under the 4-wide BVH.
 // LBVH measured faster than PLOC on the displaced icosphere at 1024^2, 64 spp (4467 vs 4348
@@ -1381,7 +1380,7 @@ __device__ __forceinline__ bool continuePath(const BsdfSample &bs, f3 thr, f3 *n
 // direction comes from the one-sample mixture c q + (1 - c) p_bsdf of the learned vMF lobes and
 // the BSDF, the continuation is weighted by f cos / (c q + (1 - c) p_bsdf), and the same mixture
 // density is the directional technique's pdf in both MIS weights.
-// Plain shading fits 96 VGPRs without spilling: 5 waves per SIMD.
+// Plain shading takes 119 VGPRs, 4 waves per SIMD; at 5 it spills.
 template <bool GUIDED, bool BATCH = false>
 __global__ __launch_bounds__(256, GUIDED ? 3 : 4) void k_shade(PtSceneView sc, ChunkParams cp, int bounce, int *counters, const float4 *rayO, const float4 *rayD,
                                                const uint4 *state, const float4 *beta, const float4 *hits, float4 *nRayO, float4 *nRayD,
@@ -3529,7 +3528,8 @@ template <class Probe>
 TuneCfg coordinateDescent(TuneCfg cur, const std::vector<int64_t> &pools, Probe probe, int *probes, double *bestRate) {
     double best = probe(cur);
     int n = 1;
-    const std::vector<int> traces = {8, 11, 12, 14}, shades = {4, 8, 16}, ldss = {16, 32};
+    // (no more trace blocks than a CU holds)
+    const std::vector<int> traces = {8, 11}, shades = {4, 8, 16}, ldss = {16, 32};
     for (int dim = 0; dim < 4; dim++) {
         const size_t count = dim == 0 ? pools.size() : dim == 1 ? traces.size() : dim == 2 ? ldss.size() : shades.size();
         for (size_t k = 0; k < count; k++) {

@@ -295,3 +295,17 @@ def test_whole_paths_up_to_the_limit(run):
         r.render(1)
         assert len(launches()) == whole
     """)
+
+
+def test_the_autotuner_tries_no_more_trace_blocks_than_a_cu_holds(run):
+    """160 KB of LDS a CU, 14.5 KB a block of the queue traversal: eleven."""
+    run("""
+    r = P.Renderer(64, 64)
+    r.set_scene(P.Scene.preset(0))
+    r.set_type(P.RENDERER_GUIDED)   # always through the queues
+    r.set_option(P.OPT_GUIDE_TRAIN_STEPS, 0)
+    watch("7k_trace", 0, 8)
+    r.autotune(2)
+    grids = {g for _, g, _, _ in launches()}
+    assert grids and max(grids) <= 11 * 256, grids
+    """)
