@@ -218,11 +218,6 @@ __device__ __forceinline__ int waveAppend(bool want, int *counter) {
     base = __shfl(base, leader);
     return want ? base + (int)lanesBelow(m) : -1;
 }
-// Appends to segment `seg` of a segmented queue: the record's slot, or -1 for lanes without one.
-__device__ __forceinline__ int segAppend(bool want, int *counters, int seg, int bounce, int field, int segLen) {
-    const int k = waveAppend(want, counters + ptQueueField(seg, bounce, field));
-    return k < 0 ? -1 : seg * segLen + k;
-}
 // Appends to each lane's own segment `seg` (the lanes of a wave may hold records of different
 // segments): one atomic per distinct segment among the appending lanes; the slot
 // seg * segLen + index, or -1 for lanes without one.
@@ -580,7 +575,7 @@ template <int STACK, int UNROLL> __device__ __forceinline__ LdsInt *stackEvict(L
     }
     const size_t lanes = gridDim.x * blockDim.x, lane = blockIdx.x * blockDim.x + threadIdx.x;
     int *spilled = ts.spill + (n * lanes + lane);
-#pragma unroll(UNROLL)
+#pragma unroll UNROLL
     for (int k = 0; k < kMove; k++, spilled += lanes) *spilled = first[k * kTraceThreads];
     *count = n + kMove;
     LdsInt *to = first;
@@ -598,7 +593,7 @@ template <int STACK, int UNROLL> __device__ __forceinline__ LdsInt *stackRefill(
     if (n == 0) return first;
     const size_t lanes = gridDim.x * blockDim.x, lane = blockIdx.x * blockDim.x + threadIdx.x;
     const int *from = ts.spill + ((n - kMove) * lanes + lane);
-#pragma unroll(UNROLL)
+#pragma unroll UNROLL
     for (int k = 0; k < kMove; k++, from += lanes) first[k * kTraceThreads] = *from;
     *count = n - kMove;
     return first + kMove * kTraceThreads;
@@ -2246,7 +2241,7 @@ struct pt_renderer {
     BvhInfo bvh;
     int bvhBuilder = kDefaultBvhBuilder;
     int stackNeed = 1;    // deepest traversal stack the tree can need (3 per 4-wide level)
-    int ldsStack = 16;    // stack entries per lane kept in LDS; the rest spill to the pool's `spill`
+    int ldsStack = 16;    // stack rows per lane in LDS (stackEntries of them hold entries; the rest spill to the pool's `spill`)
     int refillLanes = 0;  // idle lanes of a trace wave that trigger taking new rays (0: per launch)
     bool packetCamera = true;  // camera runs of one pixel's samples traced as one packet
     bool traceStats = false;   // PT_OPT_TRACE_STATS: instrumented trace kernels
