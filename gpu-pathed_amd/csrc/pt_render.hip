@@ -2848,6 +2848,10 @@ int pt_renderer_create(int width, int height, pt_renderer **out) {
         delete r;
         return fail(PT_ERR_DEVICE, "pt_renderer_create: " + e.msg);
     }
+    catch (const std::bad_alloc &) {
+        delete r;
+        return fail(PT_ERR_MEMORY, "pt_renderer_create: out of host memory");
+    }
 }
 
 int pt_renderer_destroy(pt_renderer *r) {
@@ -4098,6 +4102,10 @@ int pt_batch_create(pt_batch **out) {
     catch (const HipFailure &e) {
         delete b;
         return fail(PT_ERR_DEVICE, "pt_batch_create: " + e.msg);
+    }
+    catch (const std::bad_alloc &) {
+        delete b;
+        return fail(PT_ERR_MEMORY, "pt_batch_create: out of host memory");
     }
 }
 
