@@ -1776,19 +1776,25 @@ __device__ __forceinline__ TraceHit traceBoth(const PtSceneView &sc, bool alive,
 }
 
 template <int STACK, bool NEE>
-__global__ __launch_bounds__(kTraceThreads, pathBlocksPerCU(STACK, NEE) / 2) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, int runPaths, float4 *Lpath, int *pathCounters,
-                                                           int *spill, int spillCap, int *overflow) {
+__global__ __launch_bounds__(kTraceThreads, pathBlocksPerCU(STACK, NEE) / 2) void k_paths(PtSceneView sc, ChunkParams cp, PtCamera cam, int runPaths, int turn,
+                                                                                                float4 *Lpath, int *pathCounters, int *spill, int spillCap,
+                                                                                                int *overflow) {
     __shared__ int sstack[stackRows(STACK) * kTraceThreads];
     __shared__ ShadowList lists[NEE ? kTraceThreads / 64 : 1];
     const TraceStack ts = traceStack<STACK>(sstack, spill, spillCap);
     ShadowList &sh = lists[NEE ? threadIdx.x >> 6 : 0];
+    // the wave's runs: one in each round of `waves`, `turn` places further on from round to round
     const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), waves = (int)((gridDim.x * blockDim.x) >> 6);
     int *count = pathCounters + (wave % kPathSegs) * kPathCounters;
     auto tally = [&](int field, int bounce, bool mine) {
         const int n = __popcll(__ballot(mine));
         if (n > 0 && laneId() == 0) atomicAdd(&count[field * kMaxBounces + bounce], n);
     };
-    for (int run = wave; run < (cp.nPaths + runPaths - 1) / runPaths; run += waves) {
+    const int runs = (cp.nPaths + runPaths - 1) / runPaths;
+    for (int first = 0, at = wave; first < runs; first += waves) {
+        const int run = first + at;
+        at = at + turn < waves ? at + turn : at + turn - waves;
+        if (run >= runs) continue;
         const int path = run * runPaths + laneId();
         const bool mine = laneId() < runPaths && path < cp.nPaths;
         int s, col;
@@ -2555,18 +2561,21 @@ GuideSceneNorm guideNorm(pt_renderer *r) {
     return nm;
 }
 
-// Whether a chunk's paths are traced whole (k_paths) or through the queues.  Above these sizes it depends
-// on the scene, not on its size, which is faster: queues / whole time at 2^20, 2^21 and 2^22 paths of
-// triangle or sphere soups (rays of a wave part early) 0.98 to 1.7, 0.72 to 1.1 and 0.45 to 0.87, of
-// displaced spheres of 1k to 100k triangles 1.5 to 2.0, 1.2 to 1.5 and 0.84 to 1.2, of rooms 1.1 to 1.7,
-// 0.82 to 1.1 and 0.64 to 0.96.  Trees of 5 to 16 nodes 1.2 to 3.8, 0.89 to 2.8 and 0.61 to 1.9; of up to
-// 4 1.9 to 5.0, 1.4 to 3.9 and 0.90 to 2.6, Cornell box (3 nodes) 2.0, 1.6 and 1.4, at 2^23 0.79.  The
-// timed and the counting kernels are the queues', and so are a batch's: its chunks are filled with paths
-// of several renders.
+// Whether a chunk's paths are traced whole (k_paths) or through the queues.  Which is faster depends on the
+// scene as much as on the size.  Time through the queues to time whole at 2^20, 2^21 and 2^22 paths:
+// trees of up to 4 nodes 1.9 to 5.0, 1.4 to 3.9 and 0.89 to 2.6; of 5 to 16 nodes 1.2 to 3.8, 0.89 to 2.8 and
+// 0.61 to 1.9; displaced spheres of 1k to 100k triangles 1.5 to 2.0, 1.1 to 1.5 and 0.84 to 1.2; rooms of 2k
+// to 100k 1.4 to 1.7, 1.05 to 1.1 and 0.84 to 0.96; soups of triangles, whose rays part early, 0.98 to 1.7,
+// 0.56 to 1.1 and 0.45 to 0.87; soups of spheres 0.82 to 1.2, 0.48 to 0.8 and 0.6.  The larger trees' limit
+// is such that none of these was faster through the queues as they were without k_trace either, which
+// holds for triangles up to 2^21 paths with next-event estimation and 1.5 * 2^20 without.  The timed and the
+// counting kernels are the queues', and so are a batch's: its chunks are filled with paths of several
+// renders.
 bool wholePaths(const pt_renderer *r, const ChunkParams &cp) {
     if (r->type == PT_RENDERER_GUIDED || r->profile || r->traceStats || !r->ownsStream) return false;
     const int nodes = r->view.numNodes;
-    return cp.nPaths <= (nodes <= 4 ? 1 << 22 : nodes <= 16 ? 1 << 21 : 1 << 20);
+    const bool triangles = nodes <= 32768 && r->scene.nTri >= r->scene.nSph;
+    return cp.nPaths <= (nodes <= 4 ? 1 << 22 : nodes <= 16 || (triangles && cp.nee) ? 1 << 21 : triangles ? 3 << 19 : 1 << 20);
 }
 
 // Paths per wave of k_paths.  A pass too small to fill the chip lasts as long as its slowest wave: with
@@ -2585,6 +2594,20 @@ int pathsPerWave(const ChunkParams &cp, int nodes, int resident) {
     return 64;
 }
 
+// Places a wave of k_paths moves on between its runs.  Without, its runs are `waves` apart, and where a row
+// of the image is a divisor of that many runs, always the same column: in a wide view, whose sides are
+// often empty, some waves have all the work (1024 x 512 pixels, 2 samples, without / with turns: sphere of
+// 11.5k triangles 430 / 312 us, 900 triangles as a soup 718 / 503; 1024 x 683, 1 sample 1.03 to 1.25 times
+// as long).  Square views (0.85 to 1.0) and rows that don't divide the waves (0.87 to 1.0) are faster
+// without: the XCDs' L2s keep their part of the tree then.  A tree of up to four nodes has no parts
+// (Cornell box 0.96 to 1.02 at any size, at 1024 x 512 pixels, 8 samples, depth 15 1.72).
+int pathTurn(const pt_renderer *r, const ChunkParams &cp, int runPaths, int waves) {
+    const int row = cp.W * (cp.pixelMajor ? cp.samples : 1);   // paths
+    const bool columns = row % runPaths == 0 && waves % (row / runPaths) == 0;
+    if (r->view.numNodes > 4 && !(columns && 2 * (int64_t)cp.W >= 3 * (int64_t)cp.H)) return 0;
+    return std::min((int)((int64_t)waves * 5 / 13) | 1, waves - 1);
+}
+
 void accumulateChunk(pt_renderer *r, const ChunkParams &cp, bool whole, const PassEnd &end) {
     KTimer t(r, K_ACCUM);
     k_accumulate<<<(cp.npix + 255) / 256, 256, 0, r->stream>>>(cp, r->pp->Lpath.as<float4>(), r->accum.as<double>(), r->pp->counters.as<int>(),
@@ -2599,11 +2622,12 @@ void runChunk(pt_renderer *r, const ChunkParams &cp, const PassEnd &end = PassEn
         const int resident = r->cus * pathBlocksPerCU(r->ldsStack, cp.nee != 0);
         const int runPaths = pathsPerWave(cp, r->view.numNodes, resident), perBlock = runPaths * (kTraceThreads / 64);
         const int grid = std::min((cp.nPaths + perBlock - 1) / perBlock, resident);
+        const int turn = pathTurn(r, cp, runPaths, grid * (kTraceThreads / 64));
         int cap = 0;
         int *sp = ensureSpill(r, grid, &cap);
         float4 *L = r->pp->Lpath.as<float4>();
         int *pc = r->pp->pathCounters.as<int>(), *ov = r->pp->overflow.as<int>();
-        auto run = [&](auto kernel) { kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, runPaths, L, pc, sp, cap, ov); };
+        auto run = [&](auto kernel) { kernel<<<grid, kTraceThreads, 0, r->stream>>>(r->view, cp, r->cam, runPaths, turn, L, pc, sp, cap, ov); };
         if (cp.nee) r->ldsStack == 32 ? run(k_paths<32, true>) : run(k_paths<16, true>);
         else r->ldsStack == 32 ? run(k_paths<32, false>) : run(k_paths<16, false>);
         PT_HIP_TRY(hipGetLastError());

@@ -162,8 +162,8 @@ typedef enum {
     PT_OPT_PROFILE_KERNELS = 3,  /* 1: time each kernel launch with HIP events.  Such a pass runs every
                                     queue kernel by itself; an ordinary one traces a bounce's shadow
                                     rays and the next bounce's extension rays in one launch, or, up to
-                                    2^20 paths (2^22 in the smallest scenes), whole paths in one, and
-                                    takes less time.  The images are the same. */
+                                    2^20 to 2^22 paths by scene, whole paths in one, and takes less
+                                    time.  The images are the same. */
     PT_OPT_CONSISTENT_MIS = 4,   /* 1: the light-sample MIS weight uses the BSDF sampling density
                                     (the reference uses Microfacet::pdf, microfacet.h:124-134,
                                     whose widened alpha differs from sample()'s) */
