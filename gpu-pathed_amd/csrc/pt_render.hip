@@ -2563,8 +2563,8 @@ GuideSceneNorm guideNorm(pt_renderer *r) {
 
 // Whether a chunk's paths are traced whole (k_paths) or through the queues.  Which is faster depends on the
 // scene as much as on the size.  Time through the queues to time whole at 2^20, 2^21 and 2^22 paths:
-// trees of up to 4 nodes 1.9 to 5.0, 1.4 to 3.9 and 0.89 to 2.6; of 5 to 16 nodes 1.2 to 3.8, 0.89 to 2.8 and
-// 0.61 to 1.9; displaced spheres of 1k to 100k triangles 1.5 to 2.0, 1.1 to 1.5 and 0.84 to 1.2; rooms of 2k
+// trees of up to 4 nodes 1.9 to 5.0, 1.4 to 3.9 and 1.0 to 3.0 (at 2^23 1.1 to 2.5, Cornell box of depth 15
+// 0.84 to 1.5); of 5 to 16 nodes 1.2 to 3.8, 0.89 to 2.8 and 0.61 to 1.9; displaced spheres of 1k to 100k triangles 1.5 to 2.0, 1.1 to 1.5 and 0.84 to 1.2; rooms of 2k
 // to 100k 1.4 to 1.7, 1.05 to 1.1 and 0.84 to 0.96; soups of triangles, whose rays part early, 0.98 to 1.7,
 // 0.56 to 1.1 and 0.45 to 0.87; soups of spheres 0.82 to 1.2, 0.48 to 0.8 and 0.6.  The larger trees' limit
 // is such that none of these was faster through the queues as they were without k_trace either, which
@@ -2575,7 +2575,7 @@ bool wholePaths(const pt_renderer *r, const ChunkParams &cp) {
     if (r->type == PT_RENDERER_GUIDED || r->profile || r->traceStats || !r->ownsStream) return false;
     const int nodes = r->view.numNodes;
     const bool triangles = nodes <= 32768 && r->scene.nTri >= r->scene.nSph;
-    return cp.nPaths <= (nodes <= 4 ? 1 << 22 : nodes <= 16 || (triangles && cp.nee) ? 1 << 21 : triangles ? 3 << 19 : 1 << 20);
+    return cp.nPaths <= (nodes <= 4 ? 1 << 23 : nodes <= 16 || (triangles && cp.nee) ? 1 << 21 : triangles ? 3 << 19 : 1 << 20);
 }
 
 // Paths per wave of k_paths.  A pass too small to fill the chip lasts as long as its slowest wave: with
@@ -2599,12 +2599,12 @@ int pathsPerWave(const ChunkParams &cp, int nodes, int resident) {
 // often empty, some waves have all the work (1024 x 512 pixels, 2 samples, without / with turns: sphere of
 // 11.5k triangles 430 / 312 us, 900 triangles as a soup 718 / 503; 1024 x 683, 1 sample 1.03 to 1.25 times
 // as long).  Square views (0.85 to 1.0) and rows that don't divide the waves (0.87 to 1.0) are faster
-// without: the XCDs' L2s keep their part of the tree then.  A tree of up to four nodes has no parts
-// (Cornell box 0.96 to 1.02 at any size, at 1024 x 512 pixels, 8 samples, depth 15 1.72).
+// without: the XCDs' L2s keep their part of the tree then.  A tree of up to four nodes has no parts, and
+// turns where there are columns (1.0 to 2.5 times as long without, at 2^22 and 2^23 paths).
 int pathTurn(const pt_renderer *r, const ChunkParams &cp, int runPaths, int waves) {
     const int row = cp.W * (cp.pixelMajor ? cp.samples : 1);   // paths
     const bool columns = row % runPaths == 0 && waves % (row / runPaths) == 0;
-    if (r->view.numNodes > 4 && !(columns && 2 * (int64_t)cp.W >= 3 * (int64_t)cp.H)) return 0;
+    if (!columns || (r->view.numNodes > 4 && 2 * (int64_t)cp.W < 3 * (int64_t)cp.H)) return 0;
     return std::min((int)((int64_t)waves * 5 / 13) | 1, waves - 1);
 }
 

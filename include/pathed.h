@@ -162,7 +162,7 @@ typedef enum {
     PT_OPT_PROFILE_KERNELS = 3,  /* 1: time each kernel launch with HIP events.  Such a pass runs every
                                     queue kernel by itself; an ordinary one traces a bounce's shadow
                                     rays and the next bounce's extension rays in one launch, or, up to
-                                    2^20 to 2^22 paths by scene, whole paths in one, and takes less
+                                    2^20 to 2^23 paths by scene, whole paths in one, and takes less
                                     time.  The images are the same. */
     PT_OPT_CONSISTENT_MIS = 4,   /* 1: the light-sample MIS weight uses the BSDF sampling density
                                     (the reference uses Microfacet::pdf, microfacet.h:124-134,

@@ -45,7 +45,7 @@ def _queues_and_whole(scene, W, H, spp, nee, lds, nodes=(1, 1 << 30)):
     return out[0][0]
 
 
-@pytest.mark.parametrize("prims,spheres,nee,nodes,limit", [(4, False, 1, (1, 4), 22), (0, False, 1, (1, 4), 22), (40, False, 1, (5, 16), 21),
+@pytest.mark.parametrize("prims,spheres,nee,nodes,limit", [(4, False, 1, (1, 4), 23), (0, False, 1, (1, 4), 23), (40, False, 1, (5, 16), 21),
                                                            (300, False, 1, (17, 1000), 21), (300, False, 0, (17, 1000), 20.585), (300, True, 1, (17, 1000), 20)])
 @pytest.mark.parametrize("above", [0, 1])
 @pytest.mark.parametrize("lds", [16, 32])

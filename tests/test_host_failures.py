@@ -289,7 +289,7 @@ def test_whole_paths_up_to_the_limit(run):
     s = P.Scene()
     s.add_triangles([[0, 0, 0, 1, 0, 0, 0, 1, 0]], [s.add_material(P.LAMBERTIAN, (0.5, 0.5, 0.5))])   # one node
     for height, whole in ((2048, 1), (2049, 0)):
-        r = P.Renderer(2048, height)
+        r = P.Renderer(4096, height)
         r.set_scene(s)
         watch("7k_paths", 3, 4)
         r.render(1)
