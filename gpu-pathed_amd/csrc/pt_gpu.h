@@ -5,7 +5,6 @@
 #include <stdint.h>
 
 #include <string>
-#include <utility>
 #include <vector>
 
 #include "pt_internal.h"
@@ -46,10 +45,6 @@ struct DevBuf {
         PT_HIP_TRY(hipMalloc(&p, n));
         bytes = n;
     }
-    void swap(DevBuf &o) {
-        std::swap(p, o.p);
-        std::swap(bytes, o.bytes);
-    }
     template <class T> T *as() const { return (T *)p; }
 };
 
@@ -64,15 +59,16 @@ struct WorkArrays {
     DevBuf buf;
     template <class T> void want(T *&p, size_t n) { wants.push_back({(void **)&p, (n * sizeof(T) + 255) / 256 * 256}); }
     void alloc() {
+        std::vector<Want> now;
+        now.swap(wants);   // also where there is no memory for them
         size_t total = 256;
-        for (const Want &w : wants) total += w.bytes;
+        for (const Want &w : now) total += w.bytes;
         buf.alloc(total);
         size_t at = 0;
-        for (const Want &w : wants) {
+        for (const Want &w : now) {
             *w.p = buf.as<char>() + at;
             at += w.bytes;
         }
-        wants.clear();
     }
 };
 
@@ -161,17 +157,6 @@ struct SceneArrays {
     // where the material is emissive now or was.
     int editMaterial(int id, int type, const float *albedo, const float *emit, float ior, float alpha, DevBuf &materials, DevBuf &emitters,
                      int emittersNow, HostInt &answer, hipStream_t stream);
-    void swap(SceneArrays &o) {
-        arrays.buf.swap(o.arrays.buf);
-        std::swap(nTri, o.nTri);
-        std::swap(nSph, o.nSph);
-        std::swap(nMat, o.nMat);
-        std::swap(pos, o.pos);
-        std::swap(sph, o.sph);
-        std::swap(triMat, o.triMat);
-        std::swap(sphMat, o.sphMat);
-        std::swap(mats, o.mats);
-    }
 };
 
 }  // namespace pt

@@ -2904,17 +2904,9 @@ int pt_renderer_set_scene(pt_renderer *r, const pt_scene *s) {
     // primitive records in input order (triangles, then spheres)
     const int64_t n = nt + ns;
     float lo[3], hi[3];
-    {
-        // beside the old scene, which stays where there is no memory for the new one's description
-        SceneArrays next;
-        DevBuf records, normals;
-        next.load(*s, records, normals, lo, hi, r->stream);
-        r->scene.swap(next);
-        r->primsIn.swap(records);
-        r->normals.swap(normals);
-    }
-    // from here on the old scene goes: a load that fails leaves none
+    // the new scene takes the old one's memory where it fits: a load that fails leaves none
     r->hasScene = false;
+    r->scene.load(*s, r->primsIn, r->normals, lo, hi, r->stream);
     r->camHost = s->cam;
     computeCamera(r);
     r->prims.alloc(sizeof(float4) * 3 * (size_t)std::max<int64_t>(n, 1));
