@@ -140,7 +140,8 @@ int pt_renderer_create(int width, int height, pt_renderer **out);
 int pt_renderer_destroy(pt_renderer *r);
 
 /* CUDAGlobals::initMaterials/mallocWorld/copySceneData (cuda_globals.cu:51-139): uploads the
- * scene, builds the BVH and the environment alias tables on the GPU, resets accumulation. */
+ * scene, builds the BVH and the environment alias tables on the GPU, resets accumulation.  A
+ * load that fails leaves the renderer without a scene. */
 int pt_renderer_set_scene(pt_renderer *r, const pt_scene *scene);
 
 /* Scene edits (render_session.cu:82-116 callback).  Each resets accumulation. */
