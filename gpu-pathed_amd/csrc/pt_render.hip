@@ -3466,6 +3466,16 @@ int pt_pool_layout(int width, int height, int spp, int64_t pool_option, int64_t 
     PT_API_END("pt_pool_layout")
 }
 
+// Whether a ray (o.xyz tmin d.xyz tmax) can hit anything: its origin is finite, nothing of it is NaN and
+// not all of its direction infinite.  The slab test of any other leaves out every axis, or sees [0, 0]
+// there, and accepts what boxes it is given, an unused child's with no node behind it among them.
+static bool definedRay(const float q[8]) {
+    if (q[0] * 0.f + q[1] * 0.f + q[2] * 0.f + q[4] * 0.f + q[5] * 0.f + q[6] * 0.f == 0.f && q[3] == q[3] && q[7] == q[7]) return true;
+    for (int k = 0; k < 8; k++)
+        if (std::isnan(q[k]) || (k < 3 && std::isinf(q[k]))) return false;
+    return !(std::isinf(q[4]) && std::isinf(q[5]) && std::isinf(q[6]));
+}
+
 int pt_renderer_intersect(pt_renderer *r, const float *rays, int64_t n, int any_hit, float *out) {
     if (guard("pt_renderer_intersect", r) || (n > 0 && (!rays || !out)) || n < 0) return fail(PT_ERR_INVALID, "pt_renderer_intersect: bad arguments");
     if (!r->hasScene) return fail(PT_ERR_STATE, "pt_renderer_intersect: no scene");
@@ -3478,8 +3488,13 @@ int pt_renderer_intersect(pt_renderer *r, const float *rays, int64_t n, int any_
         std::vector<float4> o(cnt), d(cnt);
         for (int i = 0; i < cnt; i++) {
             const float *q = rays + (done + i) * 8;
-            o[i] = make_float4(q[0], q[1], q[2], q[3]);
-            d[i] = make_float4(q[4], q[5], q[6], q[7]);
+            // infinite bounds as the farthest finite ones, below and above every entry distance
+            o[i] = make_float4(q[0], q[1], q[2], std::max(q[3], -FLT_MAX));
+            d[i] = make_float4(q[4], q[5], q[6], std::min(q[7], FLT_MAX));
+            if (!definedRay(q)) {
+                o[i] = make_float4(0.f, 0.f, 0.f, FLT_MAX);
+                d[i] = make_float4(0.f, 0.f, 1.f, -FLT_MAX);
+            }
         }
         if (!any_hit) {
             PT_HIP_TRY(hipMemcpyAsync(r->pp->rayO[0].p, o.data(), cnt * 16, hipMemcpyHostToDevice, r->stream));

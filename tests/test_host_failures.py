@@ -310,3 +310,35 @@ def test_the_autotuner_tries_no_more_trace_blocks_than_a_cu_holds(run):
     grids = {g for _, g, _, _ in launches()}
     assert grids and max(grids) <= 11 * 256, grids
     """)
+
+
+def test_rays_that_can_hit_nothing_are_sent_as_empty_intervals(run):
+    """Ray queries with undefined components, an origin that is not finite or a direction infinite on all
+    axes: the slab test would accept every box for them, those of a node's unused children too.  What is
+    sent to k_extend and k_shadow (arguments 4 and 5, where a ray's origin and direction are) has none."""
+    run("""
+    r = P.Renderer(8, 8)
+    r.set_scene(P.Scene.preset(0))
+    inf, nan = np.inf, np.nan
+    plain = [1, 2, 3, 0.5, 0, -1, 0.25, 7]
+    empty = [[nan] * 3 + plain[3:], [nan] * 3 + [-inf, 0, 0, 1, inf], [inf] + plain[1:], [0, -inf] + plain[2:], [nan] + plain[1:], plain[:3] + [nan] + plain[4:],
+             plain[:7] + [nan], plain[:4] + [nan, 0, 1, 7], plain[:4] + [inf, -inf, inf, 7], [nan, nan, 1e30, nan, 0, 0, 0, inf], [nan] * 8, [inf] * 8]
+    kept = [plain, plain[:4] + [0, 0, 0, 7], plain[:4] + [inf, 0, 1, 7], [1e30, 1e30, 1e30] + plain[3:], [3e38] * 3 + plain[3:], [0.] * 8, plain[:4] + [3e38] * 4]
+    bounds = [plain[:3] + [-inf] + plain[4:7] + [inf], plain[:3] + [inf] + plain[4:7] + [-inf]]
+    big = np.finfo(np.float32).max
+    rays = np.array(empty + kept + bounds, np.float32)
+    want = np.array([[0, 0, 0, big, 0, 0, 1, -big]] * len(empty) + kept + [plain[:3] + [-big] + plain[4:7] + [big], plain[:3] + [inf] + plain[4:7] + [-inf]], np.float32)
+    for any_hit, kernel in ((0, "8k_extend"), (1, "8k_shadow")):
+        sent = []
+        for arg in (4, 5):
+            watch(kernel, arg, 8)
+            r.intersect(rays, any_hit=bool(any_hit))
+            (_, _, _, p), = launches()
+            sent.append(np.frombuffer(C.string_at(struct.unpack("P", p)[0], 16 * len(rays)), np.float32).reshape(-1, 4))
+        o, d = sent
+        assert np.array_equal(o[:, :3], want[:, :3]) and np.array_equal(d[:, :3], want[:, 4:7]), (o, d)
+        if any_hit:
+            assert np.array_equal(o[:, 3], want[:, 7])
+        else:
+            assert np.array_equal(o[:, 3], want[:, 3]) and np.array_equal(d[:, 3], want[:, 7]), (o, d)
+    """)
