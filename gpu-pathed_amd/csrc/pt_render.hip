@@ -809,6 +809,7 @@ __device__ __forceinline__ void traceQueue(const PtSceneView &sc, int refill, co
                                            Finish finish, unsigned long long *tstat = nullptr) {
     bool any = MODE == ANY;
     if (sc.numNodes == 0) {
+        // extension rays; no vertex, so no shadow ray, whose end would be written where its load says
         TraceHit th;
         th.t = FLT_MAX; th.u = 0.f; th.v = 0.f; th.prim = INT32_MIN;
         int slot = 0, got;
@@ -3481,6 +3482,16 @@ int pt_renderer_intersect(pt_renderer *r, const float *rays, int64_t n, int any_
     if (!r->hasScene) return fail(PT_ERR_STATE, "pt_renderer_intersect: no scene");
     if (r->inFlight) return fail(PT_ERR_STATE, "pt_renderer_intersect: a pass is still running");
     PT_API_BEGIN
+    if (r->view.numNodes == 0) {
+        // nothing to hit, and shadow rays are not for the kernels without nodes
+        const float miss[3] = {-1.f, 0.f, 0.f};
+        const int prim = INT32_MIN;
+        for (int64_t i = 0; i < n; i++) {
+            memcpy(out + 4 * i, miss, sizeof miss);
+            memcpy(out + 4 * i + 3, &prim, sizeof prim);
+        }
+        return PT_OK;
+    }
     ensurePool(r);
     r->overflowStale = true;
     for (int64_t done = 0; done < n;) {

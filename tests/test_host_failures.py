@@ -342,3 +342,20 @@ def test_rays_that_can_hit_nothing_are_sent_as_empty_intervals(run):
         else:
             assert np.array_equal(o[:, 3], want[:, 3]) and np.array_equal(d[:, 3], want[:, 7]), (o, d)
     """)
+
+
+def test_ray_queries_of_a_scene_without_primitives_launch_nothing(run):
+    """Every ray misses.  (The kernels' way without nodes takes extension rays only: a shadow ray's end is
+    written to the path that its load has noted, and nothing is loaded there.)"""
+    run("""
+    s = P.Scene()
+    s.add_material(P.LAMBERTIAN, (0.5, 0.5, 0.5))
+    r = P.Renderer(8, 8)
+    r.set_scene(s)
+    for kernel in ("8k_shadow", "8k_extend"):
+        watch(kernel, 0, 8)
+        for any_hit in (False, True):
+            t, u, v, prim = r.intersect(np.ones((70, 8), np.float32), any_hit=any_hit)
+            assert np.all(t == -1) and not u.any() and not v.any() and np.all(prim == P.MISS)
+        assert not launches()
+    """)
