@@ -317,8 +317,10 @@ def test_rays_that_can_hit_nothing_are_sent_as_empty_intervals(run):
     axes: the slab test would accept every box for them, those of a node's unused children too.  What is
     sent to k_extend and k_shadow (arguments 4 and 5, where a ray's origin and direction are) has none."""
     run("""
+    s = P.Scene()
+    s.add_triangles([[0, 0, 0, 1, 0, 0, 0, 1, 0]], [s.add_material(P.LAMBERTIAN, (0.5, 0.5, 0.5))])
     r = P.Renderer(8, 8)
-    r.set_scene(P.Scene.preset(0))
+    r.set_scene(s)
     inf, nan = np.inf, np.nan
     plain = [1, 2, 3, 0.5, 0, -1, 0.25, 7]
     empty = [[nan] * 3 + plain[3:], [nan] * 3 + [-inf, 0, 0, 1, inf], [inf] + plain[1:], [0, -inf] + plain[2:], [nan] + plain[1:], plain[:3] + [nan] + plain[4:],
