@@ -276,7 +276,8 @@ int pt_renderer_get_path_radiance(pt_renderer *r, float *out, int64_t capacity, 
  * the renderer's own extend and shadow kernels.
  * any_hit = 0: over [tmin, tmax]; out[4n]: t, u, v, primitive (int bits: >= 0 triangle index,
  * < 0 ~sphere index, INT32_MIN miss) -- the indexing of World::hit's PrimitiveIndex
- * (world.cu:5-41); t = -1 on a miss.
+ * (world.cu:5-41); t = -1 on a miss.  A ray with an undefined component, an origin that is not finite
+ * or a direction infinite on all axes misses; infinite bounds stand for the farthest finite ones.
  * any_hit = 1: the shadow-ray query of directSampleLights (path_tracer.cu:104-110), over
  * [1e-4, tmax] whatever tmin says; out[4n]: occluded rays 0, 0, 0, primitive 0; unoccluded
  * rays -1, 0, 0, INT32_MIN (which occluder stopped the ray is not reported). */
