@@ -3726,11 +3726,14 @@ void buildWave(pt_batch *b) {
     w->ownsStream = false;
     w->pp = b->pp;
     w->cus = b->jobs[0]->cus;
+    // normals go in threes, as the triangles' tags count them (a scene without smooth triangles
+    // keeps one unused float4)
+    const auto triples = [](const pt_renderer *r) { return (int64_t)((r->normals.bytes / sizeof(float4) + 2) / 3); };
     int64_t nN = 0, nP = 0, nNrm = 0, nM = 0, nE = 0;
     for (pt_renderer *r : b->jobs) {
         nN += std::max(r->bvh.numNodes, 1);
         nP += r->view.numPrims;
-        nNrm += (int64_t)(r->normals.bytes / sizeof(float4));
+        nNrm += triples(r);
         nM += r->scene.nMat;
         nE += r->view.numEmitters;
         w->stackNeed = std::max(w->stackNeed, r->stackNeed);
@@ -3739,7 +3742,7 @@ void buildWave(pt_batch *b) {
         throw HipFailure("batch: too many primitives for one wavefront");
     w->nodes.alloc(sizeof(float4) * PT_NODE_F4 * (size_t)std::max<int64_t>(nN, 1));
     w->prims.alloc(sizeof(float4) * 3 * (size_t)std::max<int64_t>(nP, 1));
-    w->normals.alloc(sizeof(float4) * (size_t)std::max<int64_t>(nNrm, 1));
+    w->normals.alloc(sizeof(float4) * 3 * (size_t)std::max<int64_t>(nNrm, 1));
     w->materials.alloc(sizeof(PtMaterial) * (size_t)std::max<int64_t>(nM, 1));
     w->emitters.alloc(sizeof(float4) * 3 * (size_t)std::max<int64_t>(nE, 1));
     // A render without primitives has a node without children (boxes that nothing hits): its rays
@@ -3752,14 +3755,14 @@ void buildWave(pt_batch *b) {
     for (size_t j = 0; j < b->jobs.size(); j++) {
         pt_renderer *r = b->jobs[j];
         const int nn = r->bvh.numNodes, np = r->view.numPrims, ne = r->view.numEmitters;
-        const int64_t nrm = (int64_t)(r->normals.bytes / sizeof(float4)), nm = r->scene.nMat;
+        const int64_t nm = r->scene.nMat;
         float4 *dn = w->nodes.as<float4>() + (size_t)PT_NODE_F4 * oN, *dp = w->prims.as<float4>() + 3 * (size_t)oP;
         float4 *de = w->emitters.as<float4>() + 3 * (size_t)oE;
         if (nn > 0) PT_HIP_TRY(hipMemcpyAsync(dn, r->nodes.p, sizeof(float4) * PT_NODE_F4 * (size_t)nn, hipMemcpyDeviceToDevice, b->stream));
         else PT_HIP_TRY(hipMemcpyAsync(dn, empty, sizeof empty, hipMemcpyHostToDevice, b->stream));
         PT_HIP_TRY(hipMemcpyAsync(dp, r->prims.p, sizeof(float4) * 3 * (size_t)np, hipMemcpyDeviceToDevice, b->stream));
-        if (nrm > 0)
-            PT_HIP_TRY(hipMemcpyAsync(w->normals.as<float4>() + oNrm, r->normals.p, sizeof(float4) * (size_t)nrm, hipMemcpyDeviceToDevice, b->stream));
+        if (r->normals.bytes > 0)
+            PT_HIP_TRY(hipMemcpyAsync(w->normals.as<float4>() + 3 * (size_t)oNrm, r->normals.p, r->normals.bytes, hipMemcpyDeviceToDevice, b->stream));
         PT_HIP_TRY(hipMemcpyAsync(w->materials.as<PtMaterial>() + oM, r->materials.p, sizeof(PtMaterial) * (size_t)nm, hipMemcpyDeviceToDevice,
                                   b->stream));
         if (ne > 0) PT_HIP_TRY(hipMemcpyAsync(de, r->emitters.p, sizeof(float4) * 3 * (size_t)ne, hipMemcpyDeviceToDevice, b->stream));
@@ -3781,7 +3784,7 @@ void buildWave(pt_batch *b) {
         R.accum = r->accum.as<double>();
         oN += std::max(nn, 1);
         oP += np;
-        oNrm += nrm;
+        oNrm += triples(r);
         oM += nm;
         oE += ne;
     }

@@ -214,6 +214,30 @@ def test_a_batch_render_without_primitives_has_a_node_of_its_own(run, empty):
     """, *empty)
 
 
+@pytest.mark.parametrize("count", [2, 5])
+def test_a_batch_keeps_its_renders_vertex_normals_in_threes(run, count):
+    """A smooth triangle's tag counts triples of normals: what a batch adds to it (k_rebase_prims's offset)
+    counts triples too, and each render's first triple lies inside the merged array (k_extend's scene view)."""
+    run("""
+    count = int(sys.argv[1])
+    b = P.Batch()
+    for k in range(count):
+        s = P.Scene()
+        s.add_triangles([[0, 0, 0, 1, 0, 0, 0, 1, 0]], [s.add_material(P.LAMBERTIAN, (0.5, 0.5, 0.5))])
+        s.set_environment(np.ones((2, 4, 4), np.float32))
+        b.add(s, 8, 8, 1, 2)
+    b.set_option(P.OPT_BATCH_GRAPH, 0)
+    watch("14k_rebase_prims", 3, 4)
+    b.run()
+    offsets = [struct.unpack("i", l[3])[0] for l in launches()]
+    assert len(offsets) == count and offsets == sorted(set(offsets)) and offsets[0] == 0, offsets
+    watch("8k_extend", 0, 56)
+    b.run()
+    normals = struct.unpack("5P", launches()[0][3][:40])[2]
+    assert double.double_room(normals) >= 16 * 3 * (offsets[-1] + 1), (offsets, double.double_room(normals))
+    """, count)
+
+
 @pytest.mark.parametrize("width,height", [(1, 1), (1 << 28, 1), (1, 1 << 28), (1 << 14, 1 << 14)])
 def test_the_normals_view_of_the_largest_images_has_a_grid(run, width, height):
     run("""
