@@ -2601,7 +2601,9 @@ int pathsPerWave(const ChunkParams &cp, int nodes, int resident) {
 // 11.5k triangles 430 / 312 us, 900 triangles as a soup 718 / 503; 1024 x 683, 1 sample 1.03 to 1.25 times
 // as long).  Square views (0.85 to 1.0) and rows that don't divide the waves (0.87 to 1.0) are faster
 // without: the XCDs' L2s keep their part of the tree then.  A tree of up to four nodes has no parts, and
-// turns where there are columns (1.0 to 2.5 times as long without, at 2^22 and 2^23 paths).
+// turns where there are columns (as long without as with, at 2^18 to 2^23 paths: wide views 1.0 to 2.5
+// times, square ones of scenes that leave some columns empty 0.91 to 1.7, of the Cornell box, which
+// fills them all, 0.98 to 1.02).
 int pathTurn(const pt_renderer *r, const ChunkParams &cp, int runPaths, int waves) {
     const int row = cp.W * (cp.pixelMajor ? cp.samples : 1);   // paths
     const bool columns = row % runPaths == 0 && waves % (row / runPaths) == 0;
